@@ -9,9 +9,8 @@ sweep (diagonal update + vertex list + worm update) of every walker followed
 by the measurement (energy, uniform and staggered magnetization family),
 accumulated on the device.  After thermalization the library's autotuner
 measures its launch forms (stream groups at several counts, the persistent
-work-queue launch at two LDS sizes, the record-lookahead chase) on real
-sweeps (untimed setup) and keeps the fastest; then the warm-up steps and
-the timed steps, in one call.  The process asks for --hw-queues (8) hardware
+work-queue launch at two LDS sizes) on real sweeps (untimed setup) and keeps
+the fastest; then the warm-up steps and the timed steps, in one call.  The process asks for --hw-queues (8) hardware
 queues (GPU_MAX_HW_QUEUES) so up to 8 stream groups get a queue each.
 
 Reported beside it, in the same run:
@@ -242,18 +241,15 @@ def tune(batch, what, max_calls=12):
 def parallelism(choice, walkers, generic=False):
     if not choice:
         return "one wavefront per walker (untuned defaults)"
-    chase = "record-lookahead chase" if choice["chase"] else "scalar chase"
     lds = ("worm LDS sized from the largest walker" if not choice["k2_lds"]
            else f"worm LDS {choice['k2_lds']} B")
     if generic:
-        chase = "chase codes in LDS"
         lds = "worm LDS sized from the largest walker"
     if choice["persistent"]:
         return (f"autotuned: persistent work-queue launch (one workgroup per walker task, "
-                f"{walkers} tasks per call, HIP-graph replay), {lds}, {chase}")
+                f"{walkers} tasks per call, HIP-graph replay), {lds}")
     return (f"autotuned: {choice['groups']} stream groups of per-sweep kernels (one stream and "
-            f"hardware queue per group, direct launches), one wavefront per walker, {lds}, "
-            f"{chase}")
+            f"hardware queue per group, direct launches), one wavefront per walker, {lds}")
 
 
 def kernel_region(sse, batch, flats, wds, steps, budgets=None):
@@ -400,8 +396,9 @@ def sweep_budgets(cost, factor=4, cap=400):
 def operator_count_costs(batch, n_walkers, k2_lds, slow=3.0):
     """Work per sweep of each walker from its chain: the operator count n,
     times `slow` when the worm update cannot hold the walker's records in
-    LDS (8-byte records need n <= 4096 and 8n <= the worm LDS per walker;
-    beyond, links are read from L2 at about three times the time per step)."""
+    LDS (8 bytes per operator cover its 6-byte record, the exit table and
+    the site entries; larger walkers are taken to read records from L2 at
+    about three times the time per step)."""
     ns = np.array([batch.get_walker(k, with_ops=False, with_spins=False)[0]["num_operators"]
                    for k in range(n_walkers)], dtype=np.float64)
     in_lds = ns <= min(4096, k2_lds // 8)

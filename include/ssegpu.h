@@ -65,8 +65,8 @@ enum sse_status {
  * 0..n_sites-1 are the lower legs of bond sites 0..n_sites-1 (state before
  * the operator), n_sites..2*n_sites-1 the upper legs (state after).  Both
  * kernel families take any n_sites.  In wave mode a batch whose models all
- * have two-site bonds runs the two-site kernels (LDS records, the chase
- * table, the work-queue launch); a batch with any other model runs every
+ * have two-site bonds runs the two-site kernels (and the work-queue
+ * launch); a batch with any other model runs every
  * walker through the generic wave kernels, which have no work-queue launch
  * (SSE_OPT_PERSISTENT and sse_run_budgets_noalloc are refused;
  * sse_run_budgets issues one launch per sweep index).                      */
@@ -255,8 +255,8 @@ int sse_call_time(const sse_batch *b, double *ms, int64_t *sweeps);
  * No reference counterpart (tuning introspection).                         */
 int sse_lds_bytes(const sse_batch *b, int64_t *k1, int64_t *k2, int32_t *k2_per_cu);
 /* The autotuner's choice for sse_run (which 0) or sse_run_budgets (which 1):
- * persistent launch (0/1), stream groups, chase variant, worm-kernel LDS
- * setting (0 = sized from the operator counts) and the measured vertex
+ * persistent launch (0/1), stream groups, chase (always 0: the traversal has
+ * one form), worm-kernel LDS setting (0 = sized from the operator counts) and the measured vertex
  * updates per second; candidates receives the number of forms measured.
  * SSE_ERR_STATE while still measuring.  No reference counterpart (tuning
  * introspection).                                                          */
@@ -339,14 +339,15 @@ int sse_pt_get_ladders(sse_batch *b, int32_t *slot_walkers, int64_t *accepted,
  *                list, worm and measurement kernels, or the persistent
  *                launch), with direct launches instead of graph replays
  *                (sse_kernel_times).
- * SSE_OPT_WORM_RECORDS (default 0): record layout of the worm kernel.  0 picks
- *                the smallest that fits (8-byte LDS records for n <= 4096 and
- *                <= 256 chase codes, 10-byte LDS records for n <= 16384, chase
- *                codes in LDS with links read from global memory, else global
- *                memory); the kernel's LDS per walker is capped at 64 KiB so
- *                large walkers take the later layouts; 1 skips the 8-byte
- *                layout; 2 forces global memory; 3 forces the hybrid.  Results
- *                are identical; this is a tuning/testing knob.
+ * SSE_OPT_WORM_RECORDS (default 0): record layout of the worm kernel.  0 keeps
+ *                a walker's records in LDS where they fit (two entries per
+ *                operator of a two-site bond, 3 bytes each with <= 256 worm
+ *                codes, else 4), with the model's exit table beside them, else
+ *                both in global memory; the kernel's LDS per walker is capped
+ *                at 64 KiB, so larger walkers take the global layout.  1 =
+ *                4-byte entries and the exit table in global memory; 2 forces
+ *                global records; 3 = the exit table in global memory.
+ *                Results are identical; this is a tuning/testing knob.
  * SSE_OPT_PERSISTENT (default 0): 1 = sse_run/sse_sweep issue one persistent,
  *                work-queue-driven launch per call (wave mode): each
  *                workgroup takes a walker from an atomic task counter and runs
@@ -370,23 +371,16 @@ int sse_pt_get_ladders(sse_batch *b, int32_t *slot_walkers, int64_t *accepted,
  *                stream groups from each group's own largest count.  Walkers
  *                that do not fit take a slower record layout; results are
  *                identical.
- * SSE_OPT_CHASE (default 0): worm traversal over the LDS record layouts.
- *                0 = the scalar chase (one record read per step); 1 = record
- *                lookahead: at each step four lanes read the records linked
- *                to the current operator's four legs while the exit is
- *                selected, so the next record is already in registers (more
- *                instructions per step; slower where the step is bound by
- *                instruction issue, as on the batched Heisenberg workload).
- *                Results are identical.
+ * SSE_OPT_CHASE (default 0): 0 or 1, accepted without effect: the worm
+ *                traversal has one form.
  * SSE_OPT_TUNE (default 1): autotuner.  The first measuring sse_run calls of
  *                a wave-mode batch run their sweeps in turn (segments of four
  *                sweeps, twice round-robin) with the candidate launch forms: stream
  *                groups at 2, 4, 8 (with more hardware queues than 8) and
  *                hardware-queue-count groups; the
  *                persistent work-queue launch with the worm-kernel LDS sized
- *                from the largest walker or capped at 32 KiB; then the
- *                winner with the record-lookahead chase.  Each is scored by
- *                vertex updates (the chains' own counters) per second; the
+ *                from the largest walker or capped at 32 KiB.  Each is
+ *                scored by vertex updates (the chains' own counters) per second; the
  *                fastest is kept.  sse_run_budgets tunes the same way over
  *                its first calls (work-queue forms only).  Setting
  *                SSE_OPT_STREAMS, SSE_OPT_PERSISTENT, SSE_OPT_K2_LDS or
@@ -414,9 +408,9 @@ int sse_pt_get_ladders(sse_batch *b, int32_t *slot_walkers, int64_t *accepted,
  *                0 = walker index order.  Results are identical.
  * SSE_OPT_GENERIC (wave mode): 1 = run every model, two-site bonds included,
  *                through the generic wave kernels (the ones that bonds of one,
- *                three and four sites always take: chase codes of two bytes
- *                per operator in LDS, no work-queue launch); 0 = the two-site
- *                kernels (an error while a model has bonds of other sizes).
+ *                three and four sites always take; no work-queue launch);
+ *                0 = the two-site kernels (an error while a model has bonds
+ *                of other sizes).
  *                Default: 0 unless such a model is present.  Restarts tuning.
  *                Results are identical.                                     */
 enum sse_option {

@@ -7,12 +7,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <mutex>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -52,11 +54,16 @@ struct GraphKey {
     bool same(const GraphKey &o) const { return memcmp(this, &o, sizeof *this) == 0; }
 };
 
-// What sse_set_walker checks a restored state against, per model: the vertex
-// count of each bond's type and each site's local dimension.
+// Host copies of a model: what sse_set_walker checks a restored state against
+// (the vertex count of each bond's type and each site's local dimension), and
+// the bonds' sites, from which sse_get_vertex_list spells out the links.
 struct HostModelCheck {
     std::vector<int16_t> bond_nv;
     std::vector<uint8_t> site_dims;
+    std::vector<int32_t> bond_sites;
+    // sum over bonds of the largest diagonal weight: beta times it bounds the
+    // mean operator count of a diagonal state, and estimates it for sizing
+    double weight_sum = 0;
 };
 
 }  // namespace
@@ -127,7 +134,7 @@ struct sse_batch {
     // autotuner (SSE_OPT_TUNE): launch forms measured on the caller's own
     // sweeps; all of them give the same chains and accumulators
     struct TuneCfg {
-        int persistent, groups, chase;
+        int persistent, groups;
         size_t k2_lds;  // SSE_OPT_K2_LDS value (0 = sized from the operator counts)
     };
     struct Tuner {
@@ -135,7 +142,6 @@ struct sse_batch {
         std::vector<double> rate;  // best vertex updates per second seen per candidate
         std::vector<int> runs;
         int best = -1;             // chosen candidate (-1: still measuring)
-        bool twin = true;          // add the lookahead-chase twin of the fastest
     };
     bool tune = true;         // tuning enabled (an explicit launch option turns it off)
     int lane_width = 64;      // lane mode: walkers per wavefront (threads per workgroup)
@@ -147,7 +153,7 @@ struct sse_batch {
     // one group's sweeps overlap the slow tail of another's (0: automatic,
     // see group_count)
     int n_groups = 0;
-    unsigned long long seen_max_n = 0, seen_max_L = 0;  // operator counts behind the LDS size
+    unsigned long long seen_need = 0;  // worm_lds_need behind the LDS size
     std::vector<hipStream_t> gstreams;
     std::vector<hipEvent_t> gjoin;
     hipEvent_t gfork = nullptr;
@@ -303,6 +309,228 @@ static int validate_model(const sse_model_desc &m, int k)
     return SSE_OK;
 }
 
+// Host image of a model's worm tables (DevModel::w*).
+struct WormTables {
+    std::vector<uint4> bond;
+    std::vector<uint2> code;
+    std::vector<uint64_t> thr;
+    std::vector<uint32_t> row;
+    std::vector<uint4> exit;
+    std::vector<WormEntry> wide;
+    int nthr = 0, lg = 0, mw = 1, dim = 0;
+};
+
+// Exit rows take LDS beside every walker's records, which the step without a
+// compare has to be worth.
+constexpr size_t kWormRowBytes = 16384;
+// 16-byte exit entries beyond this are read from the global wide table.
+constexpr size_t kWormExitBytes = 16384;
+
+static int build_worm_tables(const sse_model_desc &m, WormTables &t)
+{
+    const int ns = m.bond_n_sites, legs = 2 * ns;
+    t.lg = ns == 1 ? 0 : ns == 2 ? 1 : 2;
+    for (int i = 0; i < m.n_types; ++i)
+        t.mw = std::max(t.mw, (int)m.types[i].max_worm_count);
+    t.dim = m.site_dims[0];
+    for (int i = 1; i < m.n_sites; ++i)
+        if (m.site_dims[i] != t.dim)
+            t.dim = 0;
+    // r < c  <=>  (word >> 11) < ceil(c * 2^53)
+    auto thr = [](double c) {
+        return c <= 0.0 ? 0ull : c >= 1.0 ? (1ull << 53) : (uint64_t)std::ceil(std::ldexp(c, 53));
+    };
+    // bond types with equal vertices and transitions share a range of codes
+    std::map<std::string, int> seen;
+    std::vector<int> base(m.n_types), rep;  // code base per type; representative types
+    for (int i = 0; i < m.n_types; ++i) {
+        const sse_vertex_data_desc &vd = m.types[i];
+        std::string key;
+        auto add = [&](const void *p, size_t bytes) { key.append((const char *)p, bytes); };
+        const int nt = vd.n_vertices * vd.max_worm_count * legs;
+        add(&vd.n_vertices, sizeof vd.n_vertices);
+        add(&vd.max_worm_count, sizeof vd.max_worm_count);
+        add(vd.leg_states, (size_t)legs * vd.n_vertices);
+        for (int k = 0; k < nt; ++k) {
+            const int off = vd.transition_offset[k], cnt = off < 0 ? -1 : vd.transition_count[k];
+            if (cnt >= 4096)
+                return fail(SSE_ERR_INVALID, "transition with more than 4095 exits");
+            add(&cnt, sizeof cnt);
+            for (int j = 0; j < cnt; ++j) {
+                add(vd.exit_cumprob + off + j, sizeof(double));
+                add(vd.exit_target + off + j, sizeof(int32_t));
+                add(vd.exit_leg + off + j, 1);
+                add(vd.exit_worm + off + j, 1);
+            }
+        }
+        auto it = seen.find(key);
+        if (it != seen.end()) {
+            base[i] = it->second;
+            continue;
+        }
+        base[i] = (int)t.code.size();
+        seen.emplace(std::move(key), base[i]);
+        rep.push_back(i);
+        for (int v = 0; v < vd.n_vertices; ++v) {
+            const uint8_t *ls = vd.leg_states + (size_t)legs * v;
+            uint32_t lower = 0;
+            bool diag = true;
+            for (int k = 0; k < ns; ++k) {
+                lower |= (uint32_t)ls[k] << (8 * k);
+                diag &= ls[k] == ls[ns + k];
+            }
+            t.code.push_back(make_uint2(lower, (uint32_t)diag | (uint32_t)v << 1 | (uint32_t)i << 10));
+        }
+        // a vertex's diagonal flag is the one its exits' targets carry (equal to
+        // the comparison of its leg states in the reference's tables,
+        // vertex_data.jl:171-187)
+        for (int e = 0; e < vd.n_exits; ++e) {
+            uint32_t &y = t.code[(size_t)base[i] + ((uint32_t)vd.exit_target[e] >> 1)].y;
+            y = (y & ~1u) | ((uint32_t)vd.exit_target[e] & 1u);
+        }
+    }
+    const size_t nc = t.code.size(), ports = 2 * (size_t)t.mw;
+    const size_t nent = ((nc << t.lg) + 1) * ports;
+    if (nent >= ((size_t)1 << 30))
+        return fail(SSE_ERR_INVALID, "too many worm table entries");
+    for (int i : rep) {
+        const sse_vertex_data_desc &vd = m.types[i];
+        for (int e = 0; e < vd.n_exits; ++e) {
+            const uint64_t k = thr(vd.exit_cumprob[e]);
+            if (k < kWormTail)
+                t.thr.push_back(k);
+        }
+    }
+    std::sort(t.thr.begin(), t.thr.end());
+    t.thr.erase(std::unique(t.thr.begin(), t.thr.end()), t.thr.end());
+    t.nthr = (int)t.thr.size();
+    // m < k  <=>  q < rank(k), for words below kWormTail
+    auto rank = [&](uint64_t k) {
+        return k >= kWormTail ? 0xFFFFFFFFu
+                                 : (uint32_t)(std::lower_bound(t.thr.begin(), t.thr.begin() + t.nthr, k) -
+                                              t.thr.begin()) + 1u;
+    };
+    WormEntry none;
+    memset(&none, 0, sizeof none);
+    none.r[0] = none.r[1] = none.r[2] = 0xFFFFFFFFu;
+    for (int j = 0; j < 4; ++j)
+        none.out[j] = kWormSpecial;
+    t.wide.assign(nent, none);
+    bool rows = ns <= 2 && ports <= 128 && (nc << t.lg) <= 255 &&
+                (size_t)(t.nthr + 1) * nent * 4 <= kWormRowBytes;
+    std::map<size_t, std::array<uint64_t, 3>> fifth;  // fourth rank, exits 3 and 4
+    std::vector<uint32_t> row(rows ? (size_t)(t.nthr + 1) * nent : 0, 0u);
+    for (int i : rep) {
+        const sse_vertex_data_desc &vd = m.types[i];
+        for (int v = 0; v < vd.n_vertices; ++v)
+            for (int wv = 0; wv < vd.max_worm_count; ++wv)
+                for (int l = 0; l < legs; ++l) {
+                    const int src = (v * vd.max_worm_count + wv) * legs + l;
+                    const int off = vd.transition_offset[src], cnt = off < 0 ? 0 : vd.transition_count[src];
+                    const uint32_t pos = (uint32_t)(l % ns), side = (uint32_t)(l / ns);
+                    const size_t ix = ((((size_t)base[i] + v) << t.lg) + pos) * ports + 2 * (size_t)wv + side;
+                    WormEntry &x = t.wide[ix];
+                    auto word = [&](int j) {
+                        const uint32_t lo = vd.exit_leg[off + j], up = lo >= (uint32_t)ns;
+                        return worm_word(worm_leg(ns, pos, lo),
+                                         2u * ((uint32_t)vd.exit_worm[off + j] - 1u) + (up ^ 1u),
+                                         ((uint32_t)base[i] + ((uint32_t)vd.exit_target[off + j] >> 1)) << t.lg);
+                    };
+                    // exit 3 stands for every word past the first three
+                    // thresholds: the fourth exit if it ends the list at 1,
+                    // else none (the exact search decides)
+                    for (int j = 0; j < 3 && j < cnt; ++j) {
+                        x.r[j] = rank(thr(vd.exit_cumprob[off + j]));
+                        if (j && x.r[j] < x.r[j - 1])
+                            x.r[j] = x.r[j - 1];
+                        x.out[j] = word(j);
+                    }
+                    if (cnt > 0 && cnt < 3)  // past the last exit: none
+                        for (int j = cnt; j < 3; ++j)
+                            x.r[j] = 0xFFFFFFFFu;
+                    if (cnt >= 4) {
+                        const uint32_t r3 = rank(thr(vd.exit_cumprob[off + 3]));
+                        if (cnt == 4 && r3 == 0xFFFFFFFFu)
+                            x.out[3] = word(3);
+                        if (ns == 4 && cnt == 5 && rank(thr(vd.exit_cumprob[off + 4])) == 0xFFFFFFFFu)
+                            fifth[ix] = {r3, word(3), word(4)};
+                    }
+                    if (cnt > 0)
+                        rows = rows && thr(vd.exit_cumprob[off + cnt - 1]) == (1ull << 53);
+                    if (rows)
+                        for (int q = 0; q <= t.nthr && rows; ++q) {
+                            int j = 0;
+                            while (j < cnt && (uint32_t)q >= rank(thr(vd.exit_cumprob[off + j])))
+                                ++j;
+                            if (j >= cnt) {
+                                rows = false;  // a word without an exit
+                                break;
+                            }
+                            const uint64_t o = word(j);
+                            const uint32_t nc0 = (uint32_t)(o >> 32);
+                            row[(size_t)q * nent + ix] =
+                                ((uint32_t)o & 0x3Fu) | (((uint32_t)o >> 8) & 255u) << 8 | (nc0 | pos) << 16 |
+                                (nc0 | (pos ^ 1u)) << 24;
+                        }
+                }
+    }
+    if (rows) {
+        t.row.swap(row);
+    } else {
+        // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none),
+        // ranks in three 10-bit fields (511: always), for four sites per bond
+        // a fifth exit
+        const int lcb = ns <= 2 ? 2 : 3;
+        if (t.nthr <= 509 && nc <= 128 && ports <= ((size_t)1 << (8 - lcb)) && nent * 16 <= kWormExitBytes) {
+            t.exit.resize(nent);
+            for (size_t e = 0; e < nent; ++e) {
+                const WormEntry &x = t.wide[e];
+                auto narrow = [&](uint64_t w) {
+                    return (w & kWormSpecial) ? 0xFFFFu
+                                              : (uint32_t)((w >> 4) & 7u) | (uint32_t)(w >> 8 & 0xFFFFFFu) << lcb |
+                                                    (uint32_t)(w >> (32 + t.lg)) << 8;
+                };
+                uint32_t r = 0, o[4], last = 511u | 0xFFFFu << 16;
+                for (int j = 0; j < 3; ++j)
+                    r |= std::min(x.r[j], 511u) << (10 * j);
+                for (int j = 0; j < 4; ++j)
+                    o[j] = narrow(x.out[j]);
+                const auto f = fifth.find(e);
+                if (f != fifth.end()) {
+                    o[3] = narrow(f->second[1]);
+                    last = std::min((uint32_t)f->second[0], 511u) | narrow(f->second[2]) << 16;
+                }
+                t.exit[e] = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, r, last);
+            }
+        }
+    }
+    std::vector<uint16_t> bkt;
+    if (t.nthr > 8) {
+        bkt.resize(256);  // saturated where it must be: the search goes on from there
+        for (uint64_t b = 0; b < 256; ++b)
+            bkt[b] = (uint16_t)std::min<ptrdiff_t>(
+                65535, std::upper_bound(t.thr.begin(), t.thr.end(), b << 45) - t.thr.begin());
+    }
+    do
+        t.thr.push_back(~0ull);
+    while (t.thr.size() % 8);
+    if (!bkt.empty()) {
+        const size_t at = t.thr.size();
+        t.thr.resize(at + 64);
+        memcpy(t.thr.data() + at, bkt.data(), 512);
+    }
+    // sites two per word: the wave kernels take lattices far below 65536 sites
+    t.bond.resize(m.n_bonds);
+    for (int b = 0; b < m.n_bonds; ++b) {
+        uint32_t s[4] = {0, 0, 0, 0};
+        for (int k = 0; k < ns; ++k)
+            s[k] = (uint32_t)m.bond_sites[(size_t)ns * b + k];
+        t.bond[b] = make_uint4((s[0] & 0xFFFFu) | s[1] << 16, (s[2] & 0xFFFFu) | s[3] << 16,
+                               (uint32_t)base[m.bond_type[b]], 0u);
+    }
+    return SSE_OK;
+}
+
 // Upload one model: every array into one device buffer, pointers fixed up.
 // The model's HostModelCheck goes into hc; the caller commits both hc and dm
 // only once every step of the upload has succeeded.
@@ -312,6 +540,19 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     hc.bond_nv.resize(m.n_bonds);
     for (int k = 0; k < m.n_bonds; ++k)
         hc.bond_nv[k] = (int16_t)m.types[m.bond_type[k]].n_vertices;
+    hc.bond_sites.assign(m.bond_sites, m.bond_sites + (size_t)m.n_bonds * m.bond_n_sites);
+    hc.weight_sum = 0;
+    for (int k = 0; k < m.n_bonds; ++k) {
+        const sse_vertex_data_desc &vd = m.types[m.bond_type[k]];
+        double w = 0;
+        size_t states = 1;
+        for (int i = 0; i < m.bond_n_sites; ++i)
+            states *= (size_t)vd.dims[i];
+        for (size_t i = 0; i < states; ++i)
+            if (vd.diagonal_vertices[i] >= 0)
+                w = std::max(w, vd.weights[vd.diagonal_vertices[i] >> 1]);
+        hc.weight_sum += w;
+    }
     std::vector<char> blob;
     auto put = [&](const void *src, size_t bytes) {
         size_t off = (blob.size() + 15) & ~(size_t)15;
@@ -361,170 +602,19 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     size_t o_ec = put(m.est_coef, sizeof(double) * ne * m.n_sites);
     size_t o_em = put(m.est_mval, sizeof(double) * ne * m.n_sites * (m.n_estimators ? m.est_max_dim : 0));
     size_t o_types = put(nullptr, sizeof(DevVD) * m.n_types);
-    // packed worm tables: hdr | trans | eout | cum
-    std::vector<uint32_t> hdr, trans, eout;
-    std::vector<double> cum;
-    int total_exits = 0;
-    for (int t = 0; t < m.n_types; ++t) {
-        const sse_vertex_data_desc &vd = m.types[t];
-        hdr.push_back((uint32_t)trans.size());
-        hdr.push_back((uint32_t)vd.n_vertices);
-        hdr.push_back((uint32_t)vd.max_worm_count);
-        int nt = vd.n_vertices * vd.max_worm_count * legs;
-        for (int i = 0; i < nt; ++i) {
-            int off = vd.transition_offset[i], cnt = vd.transition_count[i];
-            if (off < 0 || cnt <= 0)
-                trans.push_back(0xFFFFFFFFu);
-            else
-                trans.push_back((uint32_t)(total_exits + off) | ((uint32_t)cnt << 20));
-            if (cnt >= 4096)
-                return fail(SSE_ERR_INVALID, "transition with more than 4095 exits");
-        }
-        for (int e = 0; e < vd.n_exits; ++e) {
-            eout.push_back((uint32_t)vd.exit_target[e] | ((uint32_t)vd.exit_leg[e] << 10) |
-                           ((uint32_t)vd.exit_worm[e] << 12));
-            cum.push_back(vd.exit_cumprob[e]);
-        }
-        total_exits += vd.n_exits;
-    }
-    if (total_exits >= (1 << 20))
-        return fail(SSE_ERR_INVALID, "too many transition exits");
-    std::vector<char> wt;
-    size_t w_trans = hdr.size() * 4;
-    size_t w_eout = w_trans + trans.size() * 4;
-    size_t w_cum = (w_eout + eout.size() * 4 + 7) & ~(size_t)7;
-    size_t w_bytes = (w_cum + cum.size() * 8 + 15) & ~(size_t)15;
-    wt.assign(w_bytes, 0);
-    memcpy(wt.data(), hdr.data(), hdr.size() * 4);
-    if (!trans.empty())
-        memcpy(wt.data() + w_trans, trans.data(), trans.size() * 4);
-    if (!eout.empty())
-        memcpy(wt.data() + w_eout, eout.data(), eout.size() * 4);
-    if (!cum.empty())
-        memcpy(wt.data() + w_cum, cum.data(), cum.size() * 8);
-    size_t o_wtab = put(wt.data(), wt.size());
-    // chase table: one entry per (ecode, worm-1, leg_in), ecode = type << lgp | vcode
-    // with P = 2^lgp >= 2 * max vertex count, so both diagonal-flag variants of a
-    // vertex index address the same transitions (the flag rides in the vcode)
-    int dnv = 1, dmw = 1;
-    for (int t = 0; t < m.n_types; ++t) {
+    WormTables wt;
+    int wrc = build_worm_tables(m, wt);
+    if (wrc)
+        return wrc;
+    size_t o_wbond = put(wt.bond.data(), sizeof(uint4) * wt.bond.size());
+    size_t o_wcode = put(wt.code.data(), sizeof(uint2) * wt.code.size());
+    size_t o_wthr = put(wt.thr.data(), sizeof(uint64_t) * wt.thr.size());
+    size_t o_wrow = put(wt.row.data(), sizeof(uint32_t) * wt.row.size());
+    size_t o_wexit = put(wt.exit.data(), sizeof(uint4) * wt.exit.size());
+    size_t o_wwide = put(wt.wide.data(), sizeof(WormEntry) * wt.wide.size());
+    int dnv = 1;
+    for (int t = 0; t < m.n_types; ++t)
         dnv = std::max(dnv, (int)m.types[t].n_vertices);
-        dmw = std::max(dmw, (int)m.types[t].max_worm_count);
-    }
-    int lgp = 1;
-    while ((1 << lgp) < 2 * dnv)
-        ++lgp;
-    const size_t P = (size_t)1 << lgp;
-    // (the wave kernels' tables; built for two-site bonds only, the bonds
-    // the wave kernels take)
-    std::vector<DirectEntry> dt(ns == 2 ? (size_t)m.n_types * P * dmw * 4 : 1);
-    for (auto &x : dt) {  // invalid transition: every word takes the exact path, which fails
-        for (int j = 0; j < 4; ++j) {
-            x.K[j] = 0;
-            x.out[j] = kChaseSlow;
-        }
-        x.count = 0;
-        x.trans = 0xFFFFFFFFu;
-        x.pad[0] = x.pad[1] = 0;
-    }
-    if (ns == 2) {
-        int ebase = 0;
-        for (int t = 0; t < m.n_types; ++t) {
-            const sse_vertex_data_desc &vd = m.types[t];
-            for (int v = 0; v < vd.n_vertices; ++v)
-                for (int wv = 0; wv < vd.max_worm_count; ++wv)
-                    for (int l = 0; l < 4; ++l) {
-                        int src = (v * vd.max_worm_count + wv) * 4 + l;
-                        int off = vd.transition_offset[src], cnt = vd.transition_count[src];
-                        if (off < 0 || cnt <= 0)
-                            continue;
-                        DirectEntry x;
-                        x.count = (uint32_t)cnt;
-                        x.trans = (uint32_t)(ebase + off) | ((uint32_t)cnt << 20);
-                        x.pad[0] = x.pad[1] = 0;
-                        // r < c  <=>  (word >> 11) < ceil(c * 2^53)
-                        auto thr = [](double c) {
-                            return c <= 0.0 ? 0ull
-                                   : c >= 1.0 ? (1ull << 53)
-                                              : (uint64_t)std::ceil(std::ldexp(c, 53));
-                        };
-                        auto word = [&](int j) {
-                            const uint32_t ec = (uint32_t)t << lgp | (uint32_t)vd.exit_target[off + j];
-                            return dmw == 1 ? chase_out1(ec, vd.exit_leg[off + j])
-                                            : chase_out(ec, vd.exit_leg[off + j], vd.exit_worm[off + j]);
-                        };
-                        // slots past the last exit: K = 2^53 (always taken), slow marker
-                        for (int j = 0; j < 4; ++j) {
-                            x.K[j] = j < cnt ? thr(vd.exit_cumprob[off + j]) : (1ull << 53);
-                            x.out[j] = j < cnt ? word(j) : kChaseSlow;
-                        }
-                        if (cnt > 4) {  // first three inline, the rest from the exit list
-                            x.K[3] = 1ull << 53;
-                            x.out[3] = kChaseSlow;
-                        } else if (cnt == 4) {
-                            x.pad[0] = x.out[3];
-                            if (x.K[3] < (1ull << 53))  // the fourth exit needs its compare
-                                x.out[3] = kChaseSlow;
-                        }
-                        for (int dg = 0; dg < 2; ++dg)
-                            dt[((((size_t)t << lgp) + (2 * v + dg)) * dmw + wv) * 4 + l] = x;
-                    }
-            ebase += vd.n_exits;
-        }
-    }
-    size_t o_dtab = put(dt.data(), sizeof(DirectEntry) * dt.size());
-    // the generic wave kernels' chase table (every bond size): the same
-    // entries with PL = 2^glg legs per (ecode, worm) and gen_out exit words
-    const int glg = legs <= 2 ? 1 : legs <= 4 ? 2 : 3;
-    std::vector<DirectEntry> gt((size_t)m.n_types * P * dmw << glg);
-    for (auto &x : gt) {
-        for (int j = 0; j < 4; ++j) {
-            x.K[j] = 0;
-            x.out[j] = kChaseSlow;
-        }
-        x.count = 0;
-        x.trans = 0xFFFFFFFFu;
-        x.pad[0] = x.pad[1] = 0;
-    }
-    {
-        auto thr = [](double c) {
-            return c <= 0.0 ? 0ull : c >= 1.0 ? (1ull << 53) : (uint64_t)std::ceil(std::ldexp(c, 53));
-        };
-        for (int t = 0; t < m.n_types; ++t) {
-            const sse_vertex_data_desc &vd = m.types[t];
-            for (int v = 0; v < vd.n_vertices; ++v)
-                for (int wv = 0; wv < vd.max_worm_count; ++wv)
-                    for (int l = 0; l < legs; ++l) {
-                        int src = (v * vd.max_worm_count + wv) * legs + l;
-                        int off = vd.transition_offset[src], cnt = vd.transition_count[src];
-                        if (off < 0 || cnt <= 0)
-                            continue;
-                        DirectEntry x;
-                        x.count = (uint32_t)cnt;
-                        x.trans = (uint32_t)off;  // first exit in the type's own exit list
-                        x.pad[0] = x.pad[1] = 0;
-                        auto word = [&](int j) {
-                            const uint32_t ec = (uint32_t)t << lgp | (uint32_t)vd.exit_target[off + j];
-                            return gen_out(ec, vd.exit_leg[off + j], vd.exit_worm[off + j]);
-                        };
-                        for (int j = 0; j < 4; ++j) {
-                            x.K[j] = j < cnt ? thr(vd.exit_cumprob[off + j]) : (1ull << 53);
-                            x.out[j] = j < cnt ? word(j) : kChaseSlow;
-                        }
-                        if (cnt > 4) {
-                            x.K[3] = 1ull << 53;
-                            x.out[3] = kChaseSlow;
-                        } else if (cnt == 4) {
-                            x.pad[0] = x.out[3];
-                            if (x.K[3] < (1ull << 53))
-                                x.out[3] = kChaseSlow;
-                        }
-                        for (int dg = 0; dg < 2; ++dg)
-                            gt[(((((size_t)t << lgp) + (2 * v + dg)) * dmw + wv) << glg) + l] = x;
-                    }
-        }
-    }
-    size_t o_gtab = put(gt.data(), sizeof(DirectEntry) * gt.size());
     // measurement tables: per (bond, vertex) the change of each estimator
     // across the vertex, the same expression in the same order as the
     // measurement kernels' own (two sites: cf[a] (mv[a][u0] - mv[a][l0]) +
@@ -681,25 +771,26 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     dm.est_coef = (const double *)(d + o_ec);
     dm.est_mval = (const double *)(d + o_em);
     dm.types = (const DevVD *)(d + o_types);
-    dm.wtab = (const uint32_t *)(d + o_wtab);
-    dm.wtab_bytes = (int32_t)w_bytes;
-    dm.wtab_trans_off = (int32_t)w_trans;
-    dm.wtab_eout_off = (int32_t)w_eout;
-    dm.wtab_cum_off = (int32_t)w_cum;
-    dm.dtab = (const DirectEntry *)(d + o_dtab);
-    dm.dt_nv = dnv;
-    dm.dt_mw = dmw;
-    dm.dt_lgp = lgp;
-    dm.dtab_bytes = (int32_t)(sizeof(DirectEntry) * dt.size());
+    dm.wbond = (const uint4 *)(d + o_wbond);
+    dm.wcode = (const uint2 *)(d + o_wcode);
+    dm.wthr = (const uint64_t *)(d + o_wthr);
+    dm.wrow = wt.row.empty() ? nullptr : (const uint32_t *)(d + o_wrow);
+    dm.w_rank = wt.nthr > 8 ? (int32_t)(8 * wt.thr.size()) : 0;
+    dm.pad_w = 0;
+    dm.wexit = wt.exit.empty() ? nullptr : (const uint4 *)(d + o_wexit);
+    dm.wwide = (const WormEntry *)(d + o_wwide);
+    dm.w_ncode = (int32_t)wt.code.size();
+    dm.w_lg = wt.lg;
+    dm.w_nthr = wt.nthr;
+    dm.w_mw = wt.mw;
+    dm.w_nent = (int32_t)wt.wide.size();
+    dm.w_dim = wt.dim;
     dm.k1tab = (const uint8_t *)(d + o_k1);
     dm.k1tab_bytes = (int32_t)k1.size();
     dm.pad_k1 = 0;
     dm.k1ntab = (const uint8_t *)(d + o_kn);
     dm.k1ntab_bytes = (int32_t)kn.size();
     dm.k1n_bond_off = (int32_t)kn_bond_off;
-    dm.gtab = (const DirectEntry *)(d + o_gtab);
-    dm.gtab_bytes = (int32_t)(sizeof(DirectEntry) * gt.size());
-    dm.g_lg = glg;
     dm.est_dtab = edt ? (const double *)(d + o_edt) : nullptr;
     dm.est_dsgn = edt ? (const int8_t *)(d + o_esg) : nullptr;
     dm.est_dnv = dnv;
@@ -716,14 +807,23 @@ static size_t env_size(const char *name, size_t dflt)
 }
 
 // host-side bump allocation of a slab (only while no kernel runs)
-static char *host_slab(sse_batch *b, int64_t cap, int legs)
+static char *host_slab(sse_batch *b, int64_t cap, const DevModel &m)
 {
-    size_t bytes = slab_bytes(cap, legs);
+    size_t bytes = slab_bytes(cap, m, b->max_sites, b->mode == SSE_MODE_WAVE);
     if (b->pool_host_next + bytes > b->pool_size)
         return nullptr;
     char *p = b->pool_base + b->pool_host_next;
     b->pool_host_next += bytes;
     return p;
+}
+
+// LDS with which a walker takes its fastest worm-update layout, for the operator
+// count to expect of it: n is beta times the mean bond weight, 1.16 times the
+// largest diagonal weights' sum for the 16x16 beta = 8 Heisenberg walkers.
+static unsigned long long expected_need(const sse_batch *b, const sse_walker_desc &wd)
+{
+    const double n = std::min(1e9, 1.3 * b->h_check[wd.model].weight_sum / wd.T + 64.0);
+    return worm_lds_need(b->h_models[wd.model], (int64_t)n);
 }
 
 static int sync_pool_to_device(sse_batch *b)
@@ -734,8 +834,9 @@ static int sync_pool_to_device(sse_batch *b)
     p.base = b->pool_base;
     p.overflow = 0;
     p.status = 0;
-    p.max_n = 0;
-    p.max_L = 0;
+    p.max_sites = b->max_sites;
+    p.pad = 0;
+    memset(p.max_need, 0, sizeof p.max_need);
     HIPCHECK(bmemcpy(b, b->d_pool, &p, sizeof p, hipMemcpyHostToDevice));
     return SSE_OK;
 }
@@ -757,20 +858,21 @@ static int check_walker_errors(sse_batch *b)
     HIPCHECK(bmemcpy(b, &p, b->d_pool, sizeof p, hipMemcpyDeviceToHost));
     if (p.overflow)
         return fail(SSE_ERR_OOM, "slab pool exhausted; raise SSE_POOL_MB");
-    if (b->mode == SSE_MODE_WAVE && (p.max_n || p.max_L)) {
+    unsigned long long need = 0;
+    for (int g = 0; g < 8; ++g)
+        need = std::max(need, p.max_need[g]);
+    if (b->mode == SSE_MODE_WAVE && need) {
         // size the worm kernel's LDS from the operator counts of this call's
         // sweeps (the device maxima restart at zero for the next call): one
         // size for single-stream launches, one per stream group
-        b->seen_max_n = p.max_n;
-        b->seen_max_L = p.max_L;
-        const unsigned long long zero[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        static_assert(sizeof zero == sizeof p.max_n + sizeof p.max_L + sizeof p.group_max_n,
-                      "pool maxima layout");
-        HIPCHECK(bmemcpy(b, &b->d_pool->max_n, zero, sizeof zero, hipMemcpyHostToDevice));
-        wave_resize_lds(b->wave, b->seen_max_n, b->seen_max_L);
+        b->seen_need = need;
+        const unsigned long long zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        static_assert(sizeof zero == sizeof p.max_need, "pool maxima layout");
+        HIPCHECK(bmemcpy(b, b->d_pool->max_need, zero, sizeof zero, hipMemcpyHostToDevice));
+        wave_resize_lds(b->wave, b->seen_need);
         for (int g = 0; g < 7; ++g)
-            if (p.group_max_n[g])
-                b->wave.lds_k2_group[g] = wave_k2_lds_for(b->wave, p.group_max_n[g], p.max_L);
+            if (p.max_need[g])
+                b->wave.lds_k2_group[g] = wave_k2_lds_for(b->wave, p.max_need[g]);
     }
     if (p.status) {
         if (p.status & (1 << SSE_ERR_SCATTER))
@@ -925,7 +1027,7 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
         L0[w] = wd.init_opstring_cutoff >= 0 ? wd.init_opstring_cutoff
                                              : (int64_t)std::nearbyint((double)m.n_sites * wd.T);
         cap0[w] = slab_capacity(L0[w]);
-        need += slab_bytes(cap0[w], 2 * m.bond_n_sites);
+        need += slab_bytes(cap0[w], b->h_models[wd.model], b->max_sites, mode == SSE_MODE_WAVE);
         b->widths[w] = 5 + 5 * m.n_estimators;
         b->offsets[w] = off;
         b->nsites[w] = m.n_sites;
@@ -999,7 +1101,7 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
             x.ctr = 0;
             x.n_sites = b->nsites[w];
             x.last_wlf = NAN;
-            char *s = host_slab(b, cap0[w], 2 * b->h_models[wd.model].nsb);
+            char *s = host_slab(b, cap0[w], b->h_models[wd.model]);
             if (!s) {
                 rc = fail(SSE_ERR_OOM, "slab pool too small");
                 break;
@@ -1034,11 +1136,10 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
         }
         std::stable_sort(order.begin(), order.end(),
                          [&](int32_t a, int32_t c) { return key[a] > key[c]; });
-        // n ~ 0.7 beta * bonds for the magnets here; beyond ~3600 operators a
-        // walker outgrows the 8-byte records, and with stream groups these
-        // walkers get a group (and a worm-kernel LDS size) of their own
+        // walkers expected to need more than 32 KB of LDS: with stream groups
+        // they get a group (and a worm-kernel LDS size) of their own
         b->n_big = 0;
-        while (b->n_big < n_walkers && 0.7 * key[order[b->n_big]] > 3600.0)
+        while (b->n_big < n_walkers && expected_need(b, walkers[order[b->n_big]]) > 32768)
             ++b->n_big;
         rc = dev_alloc(b, &b->d_order, (size_t)n_walkers);
         if (!rc && bmemcpy(b, b->d_order, order.data(), sizeof(int32_t) * n_walkers,
@@ -1051,7 +1152,12 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
         (void)bmemset(b, b->d_count, 0, sizeof(int64_t) * n_walkers);
         (void)bmemset(b, b->d_wlf, 0, sizeof(double) * 3 * n_walkers);
         (void)bmemset(b, b->d_done, 0, sizeof(int32_t) * n_walkers);
+        (void)bmemset(b, b->d_last, 0, sizeof(int32_t) * nsp);
         rc = wave_configure(b->wave, b->h_models, b->max_sites);
+        // worm-kernel LDS of the first call: from the expected operator counts
+        for (int w = 0; w < n_walkers; ++w)
+            b->seen_need = std::max(b->seen_need, expected_need(b, walkers[w]));
+        wave_resize_lds(b->wave, b->seen_need);
         if (!rc && b->wave.lds_limit > 65536)
             (void)hipFuncSetAttribute((const void *)wave_persist_kernel,
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1602,9 +1708,8 @@ static void tune_apply(sse_batch *b, const sse_batch::TuneCfg &c)
 {
     b->persistent = c.persistent != 0 && !b->wave.generic;
     b->n_groups = c.groups;
-    b->wave.chase = c.chase;
     b->wave.lds_k2_fixed = c.k2_lds;
-    wave_resize_lds(b->wave, b->seen_max_n, b->seen_max_L);
+    wave_resize_lds(b->wave, b->seen_need);
     for (size_t &g : b->wave.lds_k2_group)
         g = 0;
 }
@@ -1613,8 +1718,7 @@ static void tune_apply(sse_batch *b, const sse_batch::TuneCfg &c)
 // (not for budgeted calls, which always use the work-queue launch), and the
 // persistent work-queue launch with the worm-kernel LDS sized from the
 // largest walker or capped at 32 KiB (more workgroups per CU; larger walkers
-// then take the global record layouts).  The record-lookahead chase is tried
-// on the winner afterwards.
+// then keep their records in global memory).
 static void tune_init(sse_batch *b, sse_batch::Tuner &t, bool budgets)
 {
     t.cands.clear();
@@ -1627,17 +1731,16 @@ static void tune_init(sse_batch *b, sse_batch::Tuner &t, bool budgets)
         gs.erase(std::unique(gs.begin(), gs.end()), gs.end());
         for (int g : gs)
             if (g <= std::max(1, n / 32))
-                t.cands.push_back({0, g, 0, 0});
+                t.cands.push_back({0, g, 0});
         if (t.cands.empty())
-            t.cands.push_back({0, 1, 0, 0});
+            t.cands.push_back({0, 1, 0});
     }
     if (!b->wave.generic) {  // the generic kernels have no work-queue launch
-        t.cands.push_back({1, 0, 0, 0});
-        t.cands.push_back({1, 0, 0, 32768});
+        t.cands.push_back({1, 0, 0});
+        t.cands.push_back({1, 0, 32768});
     }
     if (t.cands.empty())
-        t.cands.push_back({0, 1, 0, 0});
-    t.twin = !b->wave.generic;  // the generic worm kernel has one chase form
+        t.cands.push_back({0, 1, 0});
     t.rate.assign(t.cands.size(), 0.0);
     t.runs.assign(t.cands.size(), 0);
     t.best = -1;
@@ -1653,8 +1756,7 @@ static int tune_next(const sse_batch::Tuner &t)
     return -1;
 }
 
-// Record one measurement; when every candidate ran twice, keep the fastest
-// (after adding its lookahead-chase twin once).
+// Record one measurement; when every candidate ran twice, keep the fastest.
 static void tune_record(sse_batch::Tuner &t, int i, double updates, double seconds)
 {
     const double rate = seconds > 0 ? updates / seconds : 0.0;
@@ -1666,20 +1768,6 @@ static void tune_record(sse_batch::Tuner &t, int i, double updates, double secon
     for (size_t k = 1; k < t.cands.size(); ++k)
         if (t.rate[k] > t.rate[best])
             best = (int)k;
-    sse_batch::TuneCfg tw = t.cands[best];
-    if (tw.chase == 0 && t.twin) {
-        tw.chase = 1;
-        bool have = false;
-        for (auto &c : t.cands)
-            have |= c.persistent == tw.persistent && c.groups == tw.groups && c.chase == 1 &&
-                    c.k2_lds == tw.k2_lds;
-        if (!have) {
-            t.cands.push_back(tw);
-            t.rate.push_back(0.0);
-            t.runs.push_back(1);  // one measurement suffices for the twin
-            return;
-        }
-    }
     t.best = best;
 }
 
@@ -1964,9 +2052,9 @@ static int lane_run_budgets(sse_batch *b, const int64_t *sweeps, int32_t measure
             hipLaunchKernelGGL(waven_diag_vlist_kernel, dim3(n), dim3(64), b->wave.lds_k1n, b->stream,
                                b->d_walkers, b->d_models, b->d_pool, 0, n, 3, -1, ord, 7, bp, (int)i,
                                (int)b->wave.lds_k1n);
-            hipLaunchKernelGGL(waven_worm_kernel, dim3(n), dim3(64), b->wave.lds_k2n, b->stream,
+            hipLaunchKernelGGL(waven_worm_kernel, dim3(n), dim3(64), b->wave.lds_k2, b->stream,
                                b->d_walkers, b->d_models, b->d_pool, 0, n, 1, ord, bp, (int)i,
-                               (int)b->wave.lds_k2n);
+                               (int)b->wave.lds_k2, b->wave.rec_mode);
             if (measure)
                 hipLaunchKernelGGL(waven_measure_kernel, dim3(n), dim3(64), 0, b->stream,
                                    b->d_walkers, b->d_models, b->d_out, b->d_sum, b->d_sumsq,
@@ -2305,7 +2393,7 @@ int sse_set_walker(sse_batch *b, int32_t walker, const sse_walker_scalars *s, co
         return rc;
     if (s->cutoff > w.cap) {
         int64_t cap = slab_capacity(s->cutoff);
-        char *slab = host_slab(b, cap, 2 * m.nsb);
+        char *slab = host_slab(b, cap, m);
         if (!slab)
             return fail(SSE_ERR_OOM, "slab pool exhausted");
         w.ops = (uint32_t *)slab;
@@ -2346,47 +2434,56 @@ int sse_get_vertex_list(sse_batch *b, int32_t walker, int32_t *links, int64_t li
         if (links && links_capacity >= legs * w.L && w.L > 0)
             HIPCHECK(bmemcpy(b, links, w.links, sizeof(int32_t) * legs * w.L, hipMemcpyDeviceToHost));
     }
-    std::vector<int64_t> pos;  // wave path: operator rank -> slot
     if (b->mode != SSE_MODE_LANE) {
-        // compact records (rank-indexed, leg ids PL*rank + leg with PL the leg
-        // count rounded up to a power of two) -> the reference's dense layout
-        const int legs = 2 * b->h_models[w.model].nsb;
-        const int lg = legs <= 2 ? 1 : legs <= 4 ? 2 : 3, pl = 1 << lg;
-        int64_t nch = (w.L + 63) / 64;
-        const uint32_t *vt = (const uint32_t *)w.links;
-        std::vector<uint64_t> mask(nch > 0 ? nch : 1);
-        std::vector<uint32_t> lk((size_t)pl * (w.n > 0 ? w.n : 1));
-        if (nch > 0)
-            HIPCHECK(bmemcpy(b, mask.data(), (const uint64_t *)(vt + (1 + pl) * w.cap), 8 * nch,
-                               hipMemcpyDeviceToHost));
-        if (w.n > 0)
-            HIPCHECK(bmemcpy(b, lk.data(), vt + w.cap, 4 * (size_t)pl * w.n, hipMemcpyDeviceToHost));
-        for (int64_t c = 0; c < nch; ++c)
-            for (int i = 0; i < 64; ++i)
-                if ((mask[c] >> i) & 1ull)
-                    pos.push_back(64 * c + i);
-        if ((int64_t)pos.size() != w.n)
+        // the operators' places along their sites -> the reference's dense links
+        const int ns = b->h_models[w.model].nsb, legs = 2 * ns;
+        const std::vector<int32_t> &sites = b->h_check[w.model].bond_sites;
+        std::vector<uint32_t> ops(w.L > 0 ? w.L : 1), idx((size_t)ns * (w.L > 0 ? w.L : 1));
+        std::vector<int32_t> count(w.n_sites), start(w.n_sites + 1, 0);
+        if (w.L > 0) {
+            HIPCHECK(bmemcpy(b, ops.data(), w.ops, 4 * (size_t)w.L, hipMemcpyDeviceToHost));
+            HIPCHECK(bmemcpy(b, idx.data(), w.links, 4 * (size_t)ns * w.L, hipMemcpyDeviceToHost));
+        }
+        HIPCHECK(bmemcpy(b, count.data(), w.last, 4 * w.n_sites, hipMemcpyDeviceToHost));
+        bool built = true;
+        for (int i = 0; i < w.n_sites && built; ++i) {
+            built = count[i] >= 0 && count[i] <= w.n;
+            start[i + 1] = start[i] + (built ? count[i] : 0);
+        }
+        built = built && (int64_t)start[w.n_sites] == ns * w.n;
+        // leg ids (lower legs) of the operators of each site, in order
+        std::vector<int32_t> along(built ? start[w.n_sites] : 0, -1);
+        for (int64_t p = 0; p < w.L && built; ++p)
+            if (ops[p])
+                for (int k = 0; k < ns; ++k) {
+                    const int s = sites[(size_t)ns * (ops[p] >> SSE_OP_BOND_SHIFT) + k];
+                    const uint32_t j = idx[(size_t)ns * p + k];
+                    if (j >= (uint32_t)count[s] || along[start[s] + j] >= 0) {
+                        built = false;
+                        break;
+                    }
+                    along[start[s] + j] = (int32_t)(legs * p + k);
+                }
+        for (int32_t a : along)
+            built = built && a >= 0;
+        if (!built)
             return fail(SSE_ERR_STATE, "vertex list not built for the current operator string");
-        auto dense = [&](int32_t leg) -> int32_t {
-            return leg < 0 ? leg : (int32_t)(legs * pos[leg >> lg] + (leg & (pl - 1)));
-        };
-        if (links && links_capacity >= legs * w.L) {
+        const bool want = links && links_capacity >= legs * w.L;
+        if (want)
             for (int64_t k = 0; k < legs * w.L; ++k)
                 links[k] = -1;
-            for (int64_t r = 0; r < w.n; ++r)
-                for (int k = 0; k < legs; ++k)
-                    links[legs * pos[r] + k] = dense((int32_t)lk[(size_t)pl * r + k]);
-        }
-        if (first || last) {
-            std::vector<int32_t> f(w.n_sites), l(w.n_sites);
-            HIPCHECK(bmemcpy(b, f.data(), w.first, 4 * w.n_sites, hipMemcpyDeviceToHost));
-            HIPCHECK(bmemcpy(b, l.data(), w.last, 4 * w.n_sites, hipMemcpyDeviceToHost));
-            for (int i = 0; i < w.n_sites; ++i) {
-                if (first)
-                    first[i] = dense(f[i] < 0 ? -1 : f[i]);
-                if (last)
-                    last[i] = dense(l[i] < 0 ? -1 : l[i]);
+        for (int i = 0; i < w.n_sites; ++i) {
+            const int n = count[i];
+            const int32_t *a = along.data() + start[i];
+            for (int j = 0; j < n && want; ++j) {
+                const int32_t up = a[j] + ns, next = a[j + 1 < n ? j + 1 : 0];
+                links[up] = next;
+                links[next] = up;
             }
+            if (first)
+                first[i] = n ? a[0] : -1;
+            if (last)
+                last[i] = n ? a[n - 1] + ns : -1;
         }
         return SSE_OK;
     }
@@ -2415,7 +2512,7 @@ static int compact_pool(sse_batch *b)
     for (auto &w : h) {
         bool live = w.active || w.pending || w.remaining != 0;
         int64_t cap = live ? w.cap : 64;
-        size_t bytes = slab_bytes(cap, 2 * b->h_models[w.model].nsb);
+        size_t bytes = slab_bytes(cap, b->h_models[w.model], b->max_sites, b->mode == SSE_MODE_WAVE);
         if (next + bytes > b->pool_size) {
             (void)hipFree(np);
             return fail(SSE_ERR_OOM, "pool compaction: live slabs exceed the pool");
@@ -2474,10 +2571,6 @@ int sse_add_model(sse_batch *b, const sse_model_desc *model, int32_t *index)
     b->h_models.swap(hm);
     b->h_check.push_back(std::move(hc));
     b->d_models = nd;
-    if (((int64_t)dm.n_types << dm.dt_lgp) > 256 && b->wave.small_codes) {
-        b->wave.small_codes = false;  // 10-byte worm records from now on: size LDS for them
-        wave_resize_lds(b->wave, b->seen_max_n, b->seen_max_L);
-    }
     if (dm.nsb != 2 || b->wave.generic) {
         // bonds of other than two sites: the generic wave kernels from now on
         // (they take two-site models too), never the work-queue launch
@@ -2520,8 +2613,12 @@ int sse_slot_start(sse_batch *b, int32_t slot, const sse_walker_desc *wd, int64_
     int64_t L0 = wd->init_opstring_cutoff >= 0 ? wd->init_opstring_cutoff
                                                : (int64_t)std::nearbyint((double)m.n_sites * wd->T);
     int64_t cap = slab_capacity(L0);
-    if (cap > x.cap || !x.ops) {
-        char *s = host_slab(b, cap, 2 * m.nsb);
+    const bool wave = b->mode == SSE_MODE_WAVE;
+    // a slab carved for a model of fewer bytes per slot does not hold this one
+    const bool small = slab_bytes(x.cap, m, b->max_sites, wave) >
+                       slab_bytes(x.cap, b->h_models[x.model], b->max_sites, wave);
+    if (cap > x.cap || small || !x.ops) {
+        char *s = host_slab(b, cap, m);
         if (!s) {
             x.active = 0;
             x.pending = 0;
@@ -2530,7 +2627,7 @@ int sse_slot_start(sse_batch *b, int32_t slot, const sse_walker_desc *wd, int64_
             rc = compact_pool(b);
             if (rc)
                 return rc;
-            s = host_slab(b, cap, 2 * m.nsb);
+            s = host_slab(b, cap, m);
             if (!s)
                 return fail(SSE_ERR_OOM, "slab pool full; raise SSE_POOL_MB");
         }
@@ -2673,12 +2770,12 @@ int sse_set_option(sse_batch *b, int32_t option, int64_t value)
         b->tune_bud = sse_batch::Tuner();
         return SSE_OK;
     case SSE_OPT_K2_LDS: {
-        if (value != 0 && (value < 8 * (int64_t)K2Stream::kNW + 256 || value > (int64_t)b->wave.lds_limit))
+        if (value != 0 && (value < 768 || value > (int64_t)b->wave.lds_limit))
             return fail(SSE_ERR_INVALID, "SSE_OPT_K2_LDS: 0 or a size the device allows");
         HIPCHECK(hipStreamSynchronize(b->stream));
         b->tune = false;
         b->wave.lds_k2_fixed = (size_t)value & ~(size_t)15;
-        wave_resize_lds(b->wave, b->seen_max_n, b->seen_max_L);
+        wave_resize_lds(b->wave, b->seen_need);
         for (size_t &g : b->wave.lds_k2_group)
             g = 0;
         return SSE_OK;
@@ -2749,7 +2846,7 @@ int sse_set_option(sse_batch *b, int32_t option, int64_t value)
             return fail(SSE_ERR_INVALID, "SSE_OPT_WORM_RECORDS takes 0, 1, 2 or 3");
         b->wave.rec_mode = (int)value;
         HIPCHECK(hipStreamSynchronize(b->stream));
-        wave_resize_lds(b->wave, b->seen_max_n, b->seen_max_L);  // layouts differ in size
+        wave_resize_lds(b->wave, b->seen_need);  // layouts differ in size
         return SSE_OK;
     default:
         return fail(SSE_ERR_INVALID, "unknown option");
@@ -2775,7 +2872,7 @@ int sse_tuning(const sse_batch *b, int32_t which, int32_t *persistent, int32_t *
     if (groups)
         *groups = c.groups;
     if (chase)
-        *chase = c.chase;
+        *chase = 0;  // the traversal has one form
     if (k2_lds)
         *k2_lds = (int64_t)c.k2_lds;
     if (rate)

@@ -5,17 +5,16 @@
 //   DevWalker[n_walkers]    per-walker scalars and slab pointers
 //   slab pool               per walker one slab: ops[cap] (u32), then a record
 //                           region used as dense links[legs*cap] (i32, legs =
-//                           2 * sites per bond) by the lane kernels, or by the
-//                           wave kernels (two-site bonds) as compact records
-//                           indexed by operator rank r (r-th non-identity slot):
-//                             vt[cap]      vcode | bond type << 10
-//                             link[4*cap]  linked leg id 4r'+leg'
-//                             mask[cap/64+1], base[cap/64+1]  per 64-slot chunk:
-//                                          non-identity bit mask, rank of its
-//                                          first operator
-//                           carved from a device bump allocator, so the cutoff
-//                           L grows inside the kernels
-//   spins/first/last        [n_walkers][n_sites] u8 / i32 / i32
+//                           2 * sites per bond) by the lane kernels; the wave
+//                           kernels keep there, per slot p and bond site k,
+//                             idx[sites*cap]  how many earlier operators act on
+//                                             the operator's k-th site (u32)
+//                           and behind it the worm update's entry words of the
+//                           slots, or its records when they do not fit LDS
+//                           (sse_worm.h); carved from a device bump allocator,
+//                           so the cutoff L grows inside the kernels
+//   spins/first/last        [n_walkers][n_sites] u8 / i32 / i32 (wave kernels: last
+//                           holds the site's operator count, first its first entry)
 //
 // Operator code (u32): 0 = identity, else 1 | vcode<<1 | bond<<11,
 // vcode = diag | vidx<<1 (vidx 0-based).
@@ -53,18 +52,21 @@ struct DevModel {
     const double *est_mval;    // [n_est][n_sites][est_max_dim]
     // packed per-bond record for the kernels: sites and type in one int2
     const int2 *bond_rec;      // [n_bonds] (site0 | type<<20, site1)
-    // packed worm tables (staged in LDS by the worm kernel):
-    //   u32 hdr[3*n_types]   (trans offset, nv, max_worm) per type
-    //   u32 trans[...]       exit index | count << 20, or 0xFFFFFFFF
-    //   u32 eout[n_exits]    target vcode | leg << 10 | worm << 12
-    //   f64 cum[n_exits]     at byte offset wtab_cum_off
-    const uint32_t *wtab;
-    int32_t wtab_bytes, wtab_cum_off, wtab_eout_off, wtab_trans_off;
-    // chase table: one 64-byte entry (DirectEntry) per (ecode, worm-1, leg_in)
-    // at index (ecode*dt_mw + worm-1)*4 + leg_in, ecode = type << dt_lgp | vcode
-    // (2^dt_lgp >= 2*dt_nv); up to 4 exits inline, more are looked up in wtab
-    const struct DirectEntry *dtab;
-    int32_t dt_nv, dt_mw, dtab_bytes, dt_lgp;
+    // worm tables (sse_worm.h).  Bond types with equal vertices and transitions
+    // share one range of vertex codes, code = range base + vertex index; an
+    // operator's entry on its k-th site carries c = code << w_lg | k.
+    const uint4 *wbond;        // [n_bonds] sites two per word (u16), code base, 0
+    const uint2 *wcode;        // [w_ncode] lower leg states, one byte per site; vcode | type << 10
+    // distinct exit thresholds, ascending, ended by ~0 and padded to a multiple of
+    // 8; then (above 8 thresholds) u16[256], the thresholds <= bucket << 45
+    const uint64_t *wthr;
+    const uint32_t *wrow;      // exit rows (null: too large, or some word has no exit)
+    const uint4 *wexit;        // 16-byte exit entries (null: too many codes or thresholds)
+    const struct WormEntry *wwide;  // exit entries of any table
+    int32_t w_ncode, w_lg, w_nthr, w_mw;
+    int32_t w_nent;            // exit entries: ((w_ncode << w_lg) + 1) * 2 * w_mw
+    int32_t w_dim;             // local dimension of every site, 0 when they differ
+    int32_t w_rank, pad_w;     // bytes of the threshold search image, 0 for up to 8 thresholds
     // diagonal-update table, copied to LDS by K1 next to the bond records:
     //   per type a 16-byte header {weights off, diag-vertex off, leg-state off,
     //   nv | dims0 << 16}, then f64 weights[nv], i16 diagonal vertex codes
@@ -79,11 +81,6 @@ struct DevModel {
     // leg states [nv] (one byte per bond position); offsets from the start
     const uint8_t *k1ntab;
     int32_t k1ntab_bytes, k1n_bond_off;
-    // chase table of the generic wave kernels (any bond size): one entry per
-    // (ecode, worm-1, leg_in) at ((ecode*dt_mw + worm-1) << g_lg) + leg_in,
-    // 2^g_lg = leg count rounded up to a power of two; exit words gen_out()
-    const struct DirectEntry *gtab;
-    int32_t gtab_bytes, g_lg;
     // measurement tables (null when too large): per
     // (bond, vertex) at bond * est_dnv + vertex, the change of each estimator
     // across the vertex, f64 [n_est] (the measurement adds it for off-diagonal
@@ -93,61 +90,38 @@ struct DevModel {
     int32_t est_dnv, any_neg;  // vertex stride; some vertex has a negative sign
 };
 
-// Exit j is taken by the first j with r < cum[j], r = (word >> 11) * 2^-53.
+// Exit j of a scatter is the first j with r < cum[j], r = (word >> 11) * 2^-53.
 // With m = word >> 11 (an integer < 2^53) and K = ceil(cum * 2^53) this is
-// exactly m < K, so the worm kernel compares integers.  Layout for the chase:
-// out[0] is taken for m < K[0], out[j] for K[j-1] <= m < K[j]; m >= K[3] falls
-// through.  With count < 4 exits the last threshold is repeated and the unused
-// outs are 0xFFFFFFFF, so m >= K[count-1] reaches the fall-through test.  An
-// invalid transition (count 0) or one with more than 4 exits has all K = 0:
-// every word falls through and the count decides.
-// The chase compares m with K[0..2] only and takes out[3] otherwise, so
-// out[j] holds kChaseSlow (send the step to the exact path) wherever that
-// would be wrong: slots past the last exit (K = 2^53 there), the fourth exit
-// when its threshold is below 2^53 (its word is then kept in pad[0]), and
-// out[3] of an entry with more than four exits (the first three are inline).
-struct __align__(16) DirectEntry {
-    uint64_t K[4];     // integer thresholds ceil(cum[j] * 2^53)
-    uint32_t out[4];   // chase_out(target ecode, exit leg, exit worm) or kChaseSlow
-    uint32_t count;    // number of exits
-    uint32_t trans;    // wtab trans word (exit index | count << 20)
-    uint32_t pad[2];   // pad[0]: the fourth exit's word when count == 4
+// exactly m < K.  A model has few distinct K (the Heisenberg magnet 2, the
+// tables of this repository's tests at most 157), so a word is reduced once to
+// q = the number of K of the model that are <= m, and m < K becomes q < r with
+// r = 1 + the index of K: exact, and independent of where the worm is.
+//
+// Exit entry (c, worm-1, side the worm enters by: 0 lower, 1 upper) has index
+// c * 2 * w_mw + 2 * (worm - 1) + side.  Its exit word names the leg relative
+// to the entering site, the port 2 * (worm - 1) + side with which the worm
+// enters the next operator, and the new vertex code.
+struct __align__(16) WormEntry {
+    uint32_t r[3];     // exit j < 3: the first with q < r[j] (r ascending); else exit 3
+    uint32_t pad;
+    uint64_t out[4];   // worm_word(), or kWormSpecial: no exit here (see worm_exact)
+    uint32_t tail[4];
 };
+#define kWormSpecial (1ull << 63)
 
-// Marker exit word: worm-1 has bit 13 set, which no real exit word has (the
-// model check keeps every worm count below 8192).
-#define kChaseSlow 0xFFFFFFFFu
-#define kChaseSlowBit 0x2000u
-
-// Exit word of the generic chase table: worm-1 in bits 0..11, exit leg in
-// bits 12..14, target ecode in bits 16..31; bit 15 is set only in the slow
-// marker kChaseSlow (worm counts stay below 4096, legs below 8).
-__host__ __device__ inline uint32_t gen_out(uint32_t ecode, uint32_t leg, uint32_t worm)
+// Leg selector of an exit: for one and two sites per bond other | upper << 1
+// (other: not the entering site), else (position - entering position) mod sites
+// | upper << 2.  16 * selector is the shift that picks the next entry.
+__host__ __device__ inline uint32_t worm_leg(int ns, uint32_t pos_in, uint32_t leg_out)
 {
-    return (worm - 1u) | (leg << 12) | (ecode << 16);
+    const uint32_t n = (uint32_t)ns, up = leg_out >= n, pos = up ? leg_out - n : leg_out;
+    const uint32_t rel = (pos + n - pos_in) % n;
+    return n <= 2 ? rel | up << 1 : rel | up << 2;
 }
-#define kGenSlowBit 0x8000u
-
-// exit word of the chase: worm-1 in bits 0..13, exit leg in 14..15, target
-// ecode (type << dt_lgp | vcode) in 16..31
-__host__ __device__ inline uint32_t chase_out(uint32_t ecode, uint32_t leg, uint32_t worm)
+// Wide exit word: selector << 4 in bits 0..6, port in 8..31, code << lg in 32..62.
+__host__ __device__ inline uint64_t worm_word(uint32_t leg, uint32_t port, uint32_t code_lg)
 {
-    return (worm - 1u) | (leg << 14) | (ecode << 16);
-}
-// exit word of a model with one worm type: worm-1 is always 0, so bits 0..5
-// carry 14 * exit leg instead, the shift that takes the exit leg's link out of
-// an 8-byte record
-__host__ __device__ inline uint32_t chase_out1(uint32_t ecode, uint32_t leg)
-{
-    return (14u * leg) | (leg << 14) | (ecode << 16);
-}
-__host__ __device__ inline uint32_t ecode_of_vt(uint32_t vt, uint32_t lgp)
-{
-    return ((vt >> 10) << lgp) | (vt & 1023u);
-}
-__host__ __device__ inline uint32_t vt_of_ecode(uint32_t e, uint32_t lgp)
-{
-    return (e & ((1u << lgp) - 1u)) | ((e >> lgp) << 10);
+    return (uint64_t)(leg << 4 | port << 8) | (uint64_t)code_lg << 32;
 }
 
 // Pointers known to address global memory.  Loads and stores through them are
@@ -183,10 +157,10 @@ struct DevWalker {
     int32_t error, n_sites;
     // buffers
     uint32_t *ops;    // [cap]
-    int32_t *links;   // record region (dense links [legs*cap] or compact records)
+    int32_t *links;   // record region (lane: dense links [legs*cap]; wave: idx, records)
     uint8_t *spins;   // [n_sites]
-    int32_t *first;   // [n_sites]
-    int32_t *last;    // [n_sites]
+    int32_t *first;   // [n_sites] lane: first leg; wave: first entry (global records)
+    int32_t *last;    // [n_sites] lane: last leg; wave: operators on the site
     // work counters (sum over sweeps since reset)
     int64_t acc_L, acc_n, acc_W, acc_sweeps;
     int32_t meas_offset, meas_width;
@@ -204,9 +178,10 @@ struct DevPool {
     char *base;
     int32_t overflow;
     int32_t status;           // bit (1 << code) per walker error code seen
-    unsigned long long max_n; // largest operator count after a diagonal update
-    unsigned long long max_L; // largest cutoff
-    unsigned long long group_max_n[8];  // the same per walker group (stream group)
+    int32_t max_sites, pad;   // sites of the batch's largest lattice (slab_bytes)
+    // largest LDS size the worm update could use for a walker (worm_lds_need),
+    // per walker group (stream group; slot 7: every other launch)
+    unsigned long long max_need[8];
 };
 
 __device__ __forceinline__ void flag_error(DevPool *pool, int code)
@@ -427,32 +402,23 @@ __device__ __host__ __forceinline__ int64_t slab_capacity(int64_t L)
     return (c + 63) & ~(int64_t)63;
 }
 
-// Slab of a walker with leg_count legs per operator: ops[cap], then a record
-// region that holds either the compact records of the wave kernels (4 bytes
-// of vertex code and 4 * PL bytes of links per slot, plus the chunk masks and
-// bases; 20 bytes per slot for two-site bonds) or the dense links of the lane
-// kernels (4 * legs bytes per slot), whichever is larger.
-__device__ __host__ __forceinline__ uint64_t slab_bytes(int64_t cap, int legs = 4)
+// Bytes of a chase code in global records: 2, or 4 when the codes need them.
+__device__ __host__ __forceinline__ int worm_code_bytes(const DevModel &m)
 {
-    // wave layout: vt[cap] and links[PL*cap] (PL = legs rounded up to a power
-    // of two), then the chunk masks and bases
-    const uint64_t pl = legs <= 2 ? 2u : legs <= 4 ? 4u : 8u;
-    const uint64_t wave = (uint64_t)cap * 4u * (1u + pl) + ((uint64_t)cap / 64u + 1u) * 16u;
-    const uint64_t lane = (uint64_t)cap * 4u * (uint64_t)legs;
-    uint64_t b = (uint64_t)cap * 4u + (wave > lane ? wave : lane);
-    return (b + 255u) & ~(uint64_t)255u;
+    return ((int64_t)m.w_ncode << m.w_lg) <= 65535 ? 2 : 4;
 }
 
-// compact-record views of a walker's record region (wave kernels)
-__device__ __forceinline__ uint32_t *rec_vt(const DevWalker &w) { return (uint32_t *)w.links; }
-__device__ __forceinline__ uint32_t *rec_link(const DevWalker &w) { return (uint32_t *)w.links + w.cap; }
-__device__ __forceinline__ uint64_t *rec_mask(const DevWalker &w)
+// Slab of a walker: ops[cap], then the record region.  Lane kernels: dense
+// links.  Wave kernels: idx (4 bytes per slot and bond site), then the global
+// worm records (a 4-byte partner and a chase code per entry, one entry per slot
+// and bond site and two more per lattice site of the batch's largest lattice, so
+// that a slot's slab serves every model of its shape); the entry words of the
+// LDS layouts, 4 or 8 bytes per slot, take the same place.
+__device__ __host__ __forceinline__ uint64_t slab_bytes(int64_t cap, const DevModel &m, int sites, bool wave)
 {
-    return (uint64_t *)((uint32_t *)w.links + 5 * w.cap);
-}
-__device__ __forceinline__ uint32_t *rec_base(const DevWalker &w)
-{
-    return (uint32_t *)(rec_mask(w) + (w.cap / 64 + 1));
+    const uint64_t ns = (uint64_t)m.nsb, c = (uint64_t)cap, cb = (uint64_t)worm_code_bytes(m);
+    const uint64_t rec = wave ? 4u * ns * c + (4u + cb) * (ns * c + 2u * (uint64_t)sites) : 8u * ns * c;
+    return (c * 4u + rec + 255u) & ~(uint64_t)255u;
 }
 
 // Bump allocation from the batch's slab pool; returns nullptr on exhaustion.

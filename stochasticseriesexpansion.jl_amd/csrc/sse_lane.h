@@ -13,13 +13,13 @@
 
 // Grow the cutoff if n >= L/2, reallocating the slab from the pool when the
 // capacity is exceeded.  Returns false (walker untouched) on pool exhaustion.
-__device__ bool lane_grow(DevWalker &w, DevPool *pool, int legs)
+__device__ bool lane_grow(DevWalker &w, DevPool *pool, const DevModel &m)
 {
     if ((double)w.n >= (double)w.L * 0.5) {
         int64_t nl = grown_cutoff(w.L);
         if (nl > w.cap) {
             int64_t cap = slab_capacity(nl);
-            char *s = pool_alloc(pool, slab_bytes(cap, legs));
+            char *s = pool_alloc(pool, slab_bytes(cap, m, pool->max_sites, false));
             if (!s) {
                 w.error = SSE_ERR_OOM;
                 return false;
@@ -240,7 +240,7 @@ __global__ void lane_sweep_kernel(DevWalker *W, const DevModel *models, DevPool 
     LaneRng rng;
     rng.init(w.key, w.ctr);
     if (phases & 1) {
-        if (!lane_grow(w, pool, 2 * m.nsb)) {
+        if (!lane_grow(w, pool, m)) {
             W[wi].error = w.error;
             flag_error(pool, w.error);
             return;
@@ -285,7 +285,7 @@ __global__ void lane_init_kernel(DevWalker *W, const DevModel *models, DevPool *
         w.ops[p] = 0u;
     w.n = 0;
     for (int k = 0; k < w.warmup; ++k) {
-        if (!lane_grow(w, pool, 2 * m.nsb)) {
+        if (!lane_grow(w, pool, m)) {
             flag_error(pool, w.error);
             break;
         }

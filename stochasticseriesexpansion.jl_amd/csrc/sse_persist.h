@@ -19,9 +19,8 @@
 // (both atomics) and the pool's error/maximum words (atomicOr / atomicMax).
 // Between the phases of one walker the workgroup passes a barrier (which
 // orders its own global and LDS accesses), and every global record a phase
-// reads was written by vector stores of the same workgroup: the worm phase
-// reads global links with vector loads (RecHV, RecGV), never through the
-// scalar cache.  Tasks run largest expected work first (the schedule order),
+// reads was written by vector stores of the same workgroup and is read with
+// vector loads, never through the scalar cache.  Tasks run largest expected work first (the schedule order),
 // so the launch ends with the small tasks.
 #pragma once
 #include "sse_wave.h"
@@ -30,14 +29,14 @@
 // call's sweep count when budgets is null).  The counter *queue must be 0 at
 // launch (persist_reset_kernel).  measure 1 runs the measurement after every
 // thermalized sweep (sse_run), 0 leaves it out (sse_sweep).
-__global__ __launch_bounds__(64) void wave_persist_kernel(DevWalker *W, const DevModel *models,
+__global__ __launch_bounds__(64, 2) void wave_persist_kernel(DevWalker *W, const DevModel *models,
                                                           DevPool *pool, double *out, double *sum,
                                                           double *sumsq, int64_t *count,
                                                           double *wlf, int32_t *done,
                                                           const int32_t *order, int n_tasks,
                                                           const int32_t *budgets, int n_sweeps,
                                                           int measure, int lds_bytes, int rec_mode,
-                                                          int chase, int32_t *queue)
+                                                          int32_t *queue)
 {
     extern __shared__ __align__(16) char lds[];
     const int lane = threadIdx.x;
@@ -58,7 +57,7 @@ __global__ __launch_bounds__(64) void wave_persist_kernel(DevWalker *W, const De
                 break;
             k1_walker(W, models, pool, wi, 3, -1, lds, lds_bytes, 7);
             __syncthreads();
-            k2_walker<true>(W, models, pool, wi, 1, lds_bytes, rec_mode, lds, chase);
+            worm_walker<2>(W, models, pool, wi, 1, lds_bytes, rec_mode, lds);
             __syncthreads();
             if (measure) {
                 k3_walker(W, models, out, sum, sumsq, count, wlf, wi, 1, done);
@@ -106,6 +105,6 @@ static inline int wave_launch_persist(WaveConfig &c, hipStream_t s, DevWalker *W
     hipLaunchKernelGGL(persist_reset_kernel, dim3(1), dim3(1), 0, s, queue);
     hipLaunchKernelGGL(wave_persist_kernel, dim3(grid), dim3(64), lds, s, W, M, pool, out, sum, sumsq,
                        count, wlf, done, order, n_tasks, budgets, n_sweeps, measure, (int)lds,
-                       c.rec_mode, c.chase, queue);
+                       c.rec_mode, queue);
     return hipGetLastError() == hipSuccess ? SSE_OK : SSE_ERR_HIP;
 }

@@ -7,7 +7,7 @@
 //     are fixed before the update, so every lane's Philox words follow from a
 //     ballot prefix count; the words come from a 256-word LDS buffer that all
 //     lanes refill cooperatively.
-//   * spins at identity slots and vertex-list predecessors: every lane ORs its
+//   * spins at identity slots and places along the sites: every lane ORs its
 //     bit into per-site LDS lane masks (one for bond position 0, one for 1);
 //     "latest earlier operator on site s" is the highest lower bit of the mask
 //     filtered by the off-diagonal (spins) or final non-identity (links) set.
@@ -17,9 +17,7 @@
 //     the rare ambiguous lanes are resolved in slot order with the exact n.
 //   * a Lemire rejection of the bond draw (probability Nb/2^64) would shift
 //     later draw offsets; that chunk is then processed slot by slot.
-// K2 wave_worm_kernel: worm_update (sse.jl:193-303) -- the traversal is a
-//   sequential pointer chase executed uniformly by the wave; the lanes refill
-//   the Philox buffer together (64 blocks per refill).
+// K2 wave_worm_kernel: worm_update (sse.jl:193-303), sse_worm.h.
 // K3 wave_measure_kernel: measure (sse.jl:70-87,305-376) with the estimator
 //   running sums as wave prefix sums.
 #pragma once
@@ -32,18 +30,15 @@
 struct WaveConfig {
     int max_sites = 0;
     int max_warmup = 0;
-    int max_wtab = 0;
     size_t lds_k1 = 0, lds_k2 = 0, lds_k3 = 0;
     size_t lds_limit = 65536;  // device limit on dynamic LDS per workgroup
-    bool small_codes = true;   // every model has <= 256 chase codes (Rec8 records)
-    int rec_mode = 0;          // worm-kernel record layout: 0 auto, 1 no Rec8, 2 global
-    int chase = 0;             // LDS-record chase: 0 plain, 1 with record lookahead
+    int rec_mode = 0;          // worm-kernel layout (worm_walker): 0 auto, 1 wide codes, 2 global
+    int chase = 0;             // SSE_OPT_CHASE as set (the traversal has one form)
     size_t lds_k2_fixed = 0;   // worm-kernel LDS per walker set by the caller (0 = sized here)
     size_t lds_k2_group[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // per stream group (0 = lds_k2)
     int fuse_measure = 0;      // measuring sweeps: worm update + measurement in one kernel
     int generic = 0;           // some model has bonds of other than two sites: sse_wave_n.h kernels
     size_t lds_k1n = 0;        // LDS of the generic diagonal-update kernel
-    size_t lds_k2n = 0;        // LDS of the generic worm kernel (chase codes, 2 bytes per operator)
 };
 
 __device__ __forceinline__ uint64_t below_mask(int lane) { return lane ? (~0ull >> (64 - lane)) : 0ull; }
@@ -224,24 +219,24 @@ struct K2RegStream {
         return hi;
     }
 };
-typedef K2RegStream K2Stream;
-
 __device__ __forceinline__ uint32_t uni(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ __forceinline__ uint64_t uni64(uint64_t x)
 {
     return (uint64_t)uni((uint32_t)x) | ((uint64_t)uni((uint32_t)(x >> 32)) << 32);
 }
 
+#include "sse_worm.h"
+
 // LDS layout of K1 (per workgroup = one walker):
 //   rbuf  u64[256]        Philox words
 //   tm0   u64[N]          per-site lane mask, bond position 0
 //   tm1   u64[N]          per-site lane mask, bond position 1
-//   vfirst, vlast i32[N]  vertex-list first/last leg per site
+//   cnt   u32[N]          operators on the site so far
 //   cups  u16[64]         upper-leg states of this chunk's operators
 //   sp    u8[N]           spins at the current slot
 __host__ __device__ inline size_t k1_lds_bytes(int N)
 {
-    size_t b = 2048 + 16 * (size_t)N + 8 * (size_t)N + 128 + (size_t)N;
+    size_t b = 2048 + 16 * (size_t)N + 4 * (size_t)N + 128 + (size_t)N;
     return (b + 15) & ~(size_t)15;
 }
 
@@ -311,18 +306,14 @@ __host__ __device__ inline size_t k1_lds_staged(int N, int n_bonds, int k1tab_by
 
 // Slot-by-slot processing of one chunk (reference order).  Used when a bond
 // draw of the chunk hits a Lemire rejection, and when forced for validation.
-// Emits the same compact records as the parallel path.
+// Emits the same idx words as the parallel path.
 __device__ void k1_serial_chunk(DevWalker &w, const DevModel &m, WaveStream &rs, int64_t base,
-                                int64_t &n, int64_t &nr, double pm_raw, double pr_raw,
-                                bool do_diag, bool do_vl, uint8_t *sp, int32_t *vfirst,
-                                int32_t *vlast)
+                                int64_t &n, double pm_raw, double pr_raw, bool do_diag, bool do_vl,
+                                uint8_t *sp, uint32_t *cnt)
 {
     const int lane = threadIdx.x;
     const int64_t L = w.L;
-    uint32_t *gvt = rec_vt(w);
-    uint32_t *glk = rec_link(w);
-    const int64_t nr0 = nr;
-    uint64_t cmask = 0ull;
+    uint32_t *gidx = (uint32_t *)w.links;
     for (int i = 0; i < 64 && base + i < L; ++i) {
         const int64_t p = base + i;
         uint32_t op = w.ops[p];
@@ -365,35 +356,17 @@ __device__ void k1_serial_chunk(DevWalker &w, const DevModel &m, WaveStream &rs,
         }
         if (do_vl && nop != 0u) {
             int2 br = m.bond_rec[op_bond(nop)];
-            int sites[2] = {br.x & 0xFFFFF, br.y};
-            const int32_t rk = (int32_t)nr;
-            for (int k = 0; k < 2; ++k) {
-                int s = sites[k];
-                int32_t me = 4 * rk + k;
-                int32_t lst = vlast[s];
-                __syncthreads();
-                if (lane == 0) {
-                    if (lst >= 0) {
-                        glk[lst] = (uint32_t)me;
-                        glk[me] = (uint32_t)lst;
-                    } else {
-                        vfirst[s] = me;
-                    }
-                    vlast[s] = 4 * rk + 2 + k;
-                }
-                __syncthreads();
-            }
+            const int sites[2] = {br.x & 0xFFFFF, br.y};
+            __syncthreads();
             if (lane == 0)
-                gvt[rk] = op_vcode(nop) | ((uint32_t)(br.x >> 20) << 10);
-            cmask |= 1ull << i;
-            nr += 1;
+                for (int k = 0; k < 2; ++k) {
+                    gidx[2 * p + k] = cnt[sites[k]];
+                    cnt[sites[k]] += 1u;
+                }
+            __syncthreads();
         }
         if (lane == 0 && nop != op)
             w.ops[p] = nop;
-    }
-    if (do_vl && lane == 0) {
-        rec_mask(w)[base >> 6] = cmask;
-        rec_base(w)[base >> 6] = (uint32_t)nr0;
     }
     __syncthreads();
 }
@@ -402,17 +375,17 @@ __device__ void k1_serial_chunk(DevWalker &w, const DevModel &m, WaveStream &rs,
 // and stream stay in registers; the rare path gets a call instead of inlined
 // code in the chunk loop).  Returns the counts and the stream position.
 struct K1SerialOut {
-    int64_t n, nr;
+    int64_t n;
     uint64_t bbase;
     uint32_t off;
 };
 __device__ __noinline__ K1SerialOut k1_serial_chunk_ool(DevWalker w, const DevModel *m, WaveStream rs,
-                                                        int64_t base, int64_t n, int64_t nr, double pm_raw,
-                                                        double pr_raw, bool do_diag, bool do_vl, uint8_t *sp,
-                                                        int32_t *vfirst, int32_t *vlast)
+                                                        int64_t base, int64_t n, double pm_raw,
+                                                        double pr_raw, bool do_diag, bool do_vl,
+                                                        uint8_t *sp, uint32_t *cnt)
 {
-    k1_serial_chunk(w, *m, rs, base, n, nr, pm_raw, pr_raw, do_diag, do_vl, sp, vfirst, vlast);
-    return K1SerialOut{n, nr, rs.bbase, rs.off};
+    k1_serial_chunk(w, *m, rs, base, n, pm_raw, pr_raw, do_diag, do_vl, sp, cnt);
+    return K1SerialOut{n, rs.bbase, rs.off};
 }
 
 // phases: 1 diagonal update, 2 vertex list, 8 force the slot-by-slot path.
@@ -436,9 +409,8 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
     uint64_t *rbuf = (uint64_t *)lds;
     uint64_t *tm0 = (uint64_t *)(lds + 2048);
     uint64_t *tm1 = tm0 + N;
-    int32_t *vfirst = (int32_t *)(tm1 + N);
-    int32_t *vlast = vfirst + N;
-    uint16_t *cups = (uint16_t *)(vlast + N);
+    uint32_t *cnt = (uint32_t *)(tm1 + N);
+    uint16_t *cups = (uint16_t *)(cnt + N);
     uint8_t *sp = (uint8_t *)(cups + 64);
     uint32_t *tm0w = (uint32_t *)tm0;
     uint32_t *tm1w = (uint32_t *)tm1;
@@ -450,8 +422,7 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
     for (int i = lane; i < N; i += 64) {
         tm0[i] = 0ull;
         tm1[i] = 0ull;
-        vfirst[i] = -1;
-        vlast[i] = -1;
+        cnt[i] = 0u;
         sp[i] = w.spins[i];
     }
     // growth check, no draws (sse.jl:138-145)
@@ -461,7 +432,7 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
             int64_t cap = slab_capacity(nl);
             unsigned long long sp_addr = 0;
             if (lane == 0)
-                sp_addr = (unsigned long long)pool_alloc(pool, slab_bytes(cap));
+                sp_addr = (unsigned long long)pool_alloc(pool, slab_bytes(cap, m, pool->max_sites, true));
             uint32_t lo = __shfl((uint32_t)sp_addr, 0), hi = __shfl((uint32_t)(sp_addr >> 32), 0);
             char *s = (char *)(((unsigned long long)hi << 32) | lo);
             if (!s) {
@@ -491,12 +462,8 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
     const uint64_t Nb = (uint64_t)m.n_bonds;
     const int64_t L = w.L;
     int64_t n0 = w.n;
-    int64_t nr = 0;  // operators (ranks) emitted so far
     const uint64_t below = below_mask(lane), above = above_mask(lane);
-    gmem<uint32_t> *gvt = as_global(rec_vt(w));
-    gmem<uint32_t> *glk = as_global(rec_link(w));
-    gmem<uint64_t> *gmask = as_global(rec_mask(w));
-    gmem<uint32_t> *gbase = as_global(rec_base(w));
+    gmem<uint64_t> *gidx = as_global((uint64_t *)w.links);  // both sites' idx words of a slot
     gmem<uint32_t> *ops = as_global(w.ops);
 
     // The operator string reaches the chunks in blocks of K1_BLOCK chunks held
@@ -579,20 +546,18 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
                 }
             }
             if (__ballot(reject)) {
-                const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, nr, pm_raw, pr_raw, do_diag,
-                                                           do_vl, sp, vfirst, vlast);
+                const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, pm_raw, pr_raw, do_diag,
+                                                           do_vl, sp, cnt);
                 n0 = so.n;
-                nr = so.nr;
                 rs.bbase = so.bbase;
                 rs.off = so.off;
                 continue;
             }
             rs.advance((uint32_t)D);
         } else if (force_serial) {
-            const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, nr, pm_raw, pr_raw, do_diag,
-                                                       do_vl, sp, vfirst, vlast);
+            const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, pm_raw, pr_raw, do_diag,
+                                                       do_vl, sp, cnt);
             n0 = so.n;
-            nr = so.nr;
             rs.bbase = so.bbase;
             rs.off = so.off;
             continue;
@@ -696,62 +661,27 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
                 ops[p] = fop;
         }
 
-        // vertex list over the final non-identity operators of the chunk, in
-        // compact form: operator rank r = nr + (non-identity lanes below)
+        // vertex list over the chunk's final non-identity operators: how many
+        // earlier operators act on each of the operator's sites
         const uint64_t NI = do_diag ? ((identm & plus) | (diam & ~minus) | offm) : (diam | offm);
-        const bool isni = (NI >> lane) & 1ull;
-        const int32_t rank = (int32_t)(nr + popc(NI & below));
-        int32_t pred0 = -1, pred1 = -1;
+        const bool isni = do_vl && ((NI >> lane) & 1ull);
+        uint32_t i0 = 0, i1 = 0;
         bool last0 = false, last1 = false;
-        if (do_vl && isni) {
-            uint64_t m0 = (a0 | a1) & NI, m1 = (c0 | c1) & NI;
-            uint64_t cand = m0 & below;
-            if (cand) {
-                int q = hi_bit(cand);
-                pred0 = 4 * (int32_t)(nr + popc(NI & below_mask(q))) + 2 + (((a0 >> q) & 1ull) ? 0 : 1);
-            } else {
-                pred0 = vlast[s0];
-                if (pred0 < 0)
-                    pred0 = -2;  // first occurrence of the site
-            }
-            cand = m1 & below;
-            if (cand) {
-                int q = hi_bit(cand);
-                pred1 = 4 * (int32_t)(nr + popc(NI & below_mask(q))) + 2 + (((c0 >> q) & 1ull) ? 0 : 1);
-            } else {
-                pred1 = vlast[s1];
-                if (pred1 < 0)
-                    pred1 = -2;
-            }
+        if (isni) {
+            const uint64_t m0 = (a0 | a1) & NI, m1 = (c0 | c1) & NI;
+            i0 = cnt[s0] + (uint32_t)popc(m0 & below);
+            i1 = cnt[s1] + (uint32_t)popc(m1 & below);
             last0 = (m0 & above) == 0ull;
             last1 = (m1 & above) == 0ull;
         }
         wave_lds_sync();
-        if (do_vl && isni) {
-            const int32_t me0 = 4 * rank, me1 = 4 * rank + 1;
-            if (pred0 >= 0) {
-                glk[me0] = (uint32_t)pred0;
-                glk[pred0] = (uint32_t)me0;
-            } else {
-                vfirst[s0] = me0;
-            }
-            if (pred1 >= 0) {
-                glk[me1] = (uint32_t)pred1;
-                glk[pred1] = (uint32_t)me1;
-            } else {
-                vfirst[s1] = me1;
-            }
+        if (isni) {
+            gidx[p] = (uint64_t)i0 | (uint64_t)i1 << 32;
             if (last0)
-                vlast[s0] = 4 * rank + 2;
+                cnt[s0] = i0 + 1u;
             if (last1)
-                vlast[s1] = 4 * rank + 3;
-            gvt[rank] = op_vcode(fop) | ((uint32_t)type << 10);
+                cnt[s1] = i1 + 1u;
         }
-        if (do_vl && lane == 0) {
-            gmask[base >> 6] = NI;
-            gbase[base >> 6] = (uint32_t)nr;
-        }
-        nr += popc(NI);
         // spins after the chunk: the last off-diagonal operator on a site wins
         if (do_diag && offd) {
             if ((((a0 | a1) & offm) & above) == 0ull)
@@ -766,18 +696,9 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
         wave_lds_sync();
     }
 
-    // periodic closure (vertex_list.jl:46-51) and write-back
     if (do_vl) {
-        for (int s = lane; s < N; s += 64) {
-            int32_t f = vfirst[s];
-            if (f >= 0) {
-                int32_t l = vlast[s];
-                glk[f] = (uint32_t)l;
-                glk[l] = (uint32_t)f;
-            }
-            w.first[s] = f;
-            w.last[s] = vlast[s];
-        }
+        for (int s = lane; s < N; s += 64)
+            w.last[s] = (int32_t)cnt[s];
     }
     if (do_diag) {
         for (int s = lane; s < N; s += 64)
@@ -791,9 +712,8 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
         o.ops = w.ops;
         o.links = w.links;
         o.ctr = rs.ctr();
-        atomicMax(&pool->max_n, (unsigned long long)n0);
-        atomicMax(&pool->group_max_n[grp & 7], (unsigned long long)n0);
-        atomicMax(&pool->max_L, (unsigned long long)L);
+        if (do_vl)
+            atomicMax(&pool->max_need[grp & 7], (unsigned long long)worm_lds_need(m, n0));
     }
 }
 
@@ -836,917 +756,17 @@ __global__ __launch_bounds__(64) void wave_diag_vlist_kernel(DevWalker *W, const
 }
 
 // ------------------------------------------------------------------ K2
-// Exit lists of the packed worm tables (DevModel::wtab) for transitions with
-// more than four exits.
-struct WormTab {
-    const uint32_t *hdr, *trans, *eout;
-    const double *cum;
-};
-
-__device__ __forceinline__ WormTab worm_tab(const char *base, const DevModel &m)
-{
-    WormTab t;
-    t.hdr = (const uint32_t *)base;
-    t.trans = (const uint32_t *)(base + m.wtab_trans_off);
-    t.eout = (const uint32_t *)(base + m.wtab_eout_off);
-    t.cum = (const double *)(base + m.wtab_cum_off);
-    return t;
-}
-
-// Worm records of one walker during K2, indexed by operator rank r: the chase
-// code ecode = type << dt_lgp | vcode and the four links (leg ids 4r'+leg').
-// K1 leaves them in global memory (u32 vt = vcode | type << 10, uint4 links);
-// K2 stages them in LDS when they fit:
-//   Rec8   one u64 per rank: links in 14-bit fields, ecode in bits 56..63
-//          (n <= 4096, at most 256 ecodes)
-//   Rec10  u64 links in 16-bit fields + a u16 ecode array (n <= 16384)
-//   RecG   global memory: ecode rewritten in place over vt, links read through
-//          the scalar cache (K2 never writes them)
-// load() returns wave-uniform words; put_ecode() is called by the whole wave
-// with one value (all lanes store it).
-typedef __attribute__((address_space(3))) uint64_t lds_u64;
-typedef __attribute__((address_space(3))) uint16_t lds_u16;
-typedef __attribute__((address_space(3))) uint8_t lds_u8;
-struct U4 {
-    uint32_t x, y, z, w;
-};
-typedef const __attribute__((address_space(4))) U4 const_u4;
-typedef const __attribute__((address_space(4))) char const_char;
-typedef const __attribute__((address_space(4))) DirectEntry ConstEntry;
-
-struct Rec8 {
-    lds_u64 *rec;
-    static constexpr bool kChecked = false;
-    typedef uint32_t Key;  // leg id < 2^16: (leg id << 14 | worm-1) fits 32 bits
-    struct Word {
-        uint32_t lo, hi;
-    };
-    __device__ __forceinline__ Word load(uint32_t r) const
-    {
-        const uint64_t x = rec[r];
-        return Word{uni((uint32_t)x), uni((uint32_t)(x >> 32))};
-    }
-    __device__ __forceinline__ static uint32_t ecode(const Word &x) { return x.hi >> 24; }
-    __device__ __forceinline__ static uint32_t link(const Word &x, uint32_t leg)
-    {
-        const uint64_t v = (uint64_t)x.lo | ((uint64_t)x.hi << 32);
-        return (uint32_t)(v >> (14u * leg)) & 0x3FFFu;
-    }
-    __device__ __forceinline__ static void set_link0(Word &x, uint32_t v) { x.lo = (x.lo & ~0x3FFFu) | v; }
-    // link of the exit leg when the exit word carries 14 * leg in its low six
-    // bits (one-worm tables): one 64-bit shift by the word itself
-    __device__ __forceinline__ static uint32_t link_sh(const Word &x, uint32_t eo)
-    {
-        const uint64_t v = (uint64_t)x.lo | ((uint64_t)x.hi << 32);
-        return (uint32_t)(v >> (eo & 63u)) & 0x3FFFu;
-    }
-    // every lane writes the same byte (no exec-mask switch in the chase loop)
-    __device__ __forceinline__ void put_ecode(uint32_t r, uint32_t e) const
-    {
-        ((lds_u8 *)rec)[8u * r + 7u] = (uint8_t)e;
-    }
-    __device__ __forceinline__ uint32_t get_ecode(uint32_t r) const { return (uint32_t)(rec[r] >> 56); }
-    // lookahead chase: each lane reads one record (lane-varying rank); the
-    // wave then takes the word of one lane with v_readlane
-    struct Cand {
-        uint32_t lo, hi;
-    };
-    __device__ __forceinline__ Cand load_lane(uint32_t r) const
-    {
-        const uint64_t x = rec[r];
-        return Cand{(uint32_t)x, (uint32_t)(x >> 32)};
-    }
-    __device__ __forceinline__ static Word pick(const Cand &c, uint32_t lane)
-    {
-        return Word{(uint32_t)__builtin_amdgcn_readlane((int)c.lo, (int)lane),
-                    (uint32_t)__builtin_amdgcn_readlane((int)c.hi, (int)lane)};
-    }
-    __device__ __forceinline__ static void set_ecode(Word &x, uint32_t e)
-    {
-        x.hi = (x.hi & 0x00FFFFFFu) | (e << 24);
-    }
-};
-
-struct Rec10 {
-    lds_u64 *lk;
-    lds_u16 *ec;
-    static constexpr bool kChecked = false;
-    typedef uint32_t Key;
-    struct Word {
-        uint32_t lo, hi, e;
-    };
-    __device__ __forceinline__ Word load(uint32_t r) const
-    {
-        const uint64_t x = lk[r];
-        const uint32_t e = ec[r];
-        return Word{uni((uint32_t)x), uni((uint32_t)(x >> 32)), uni(e)};
-    }
-    __device__ __forceinline__ static uint32_t ecode(const Word &x) { return x.e; }
-    __device__ __forceinline__ static uint32_t link(const Word &x, uint32_t leg)
-    {
-        const uint64_t v = (uint64_t)x.lo | ((uint64_t)x.hi << 32);
-        return (uint32_t)(v >> (16u * leg)) & 0xFFFFu;
-    }
-    __device__ __forceinline__ static void set_link0(Word &x, uint32_t v) { x.lo = (x.lo & ~0xFFFFu) | v; }
-    __device__ __forceinline__ void put_ecode(uint32_t r, uint32_t e) const { ec[r] = (uint16_t)e; }
-    __device__ __forceinline__ uint32_t get_ecode(uint32_t r) const { return ec[r]; }
-    struct Cand {
-        uint32_t lo, hi, e;
-    };
-    __device__ __forceinline__ Cand load_lane(uint32_t r) const
-    {
-        const uint64_t x = lk[r];
-        return Cand{(uint32_t)x, (uint32_t)(x >> 32), (uint32_t)ec[r]};
-    }
-    __device__ __forceinline__ static Word pick(const Cand &c, uint32_t lane)
-    {
-        return Word{(uint32_t)__builtin_amdgcn_readlane((int)c.lo, (int)lane),
-                    (uint32_t)__builtin_amdgcn_readlane((int)c.hi, (int)lane),
-                    (uint32_t)__builtin_amdgcn_readlane((int)c.e, (int)lane)};
-    }
-    __device__ __forceinline__ static void set_ecode(Word &x, uint32_t e) { x.e = e; }
-};
-
-struct RecG {
-    uint32_t *ec;
-    const_u4 *lk;
-    static constexpr bool kChecked = true;
-    typedef uint64_t Key;
-    struct Word {
-        U4 l;
-        uint32_t e;
-    };
-    __device__ __forceinline__ Word load(uint32_t r) const
-    {
-        const_u4 &q = lk[r];
-        return Word{U4{q.x, q.y, q.z, q.w}, uni(ec[r])};
-    }
-    __device__ __forceinline__ static uint32_t ecode(const Word &x) { return x.e; }
-    __device__ __forceinline__ static uint32_t link(const Word &x, uint32_t leg)
-    {
-        return leg == 0 ? x.l.x : leg == 1 ? x.l.y : leg == 2 ? x.l.z : x.l.w;
-    }
-    __device__ __forceinline__ static void set_link0(Word &x, uint32_t v) { x.l.x = v; }
-    // every lane stores, so each lane's own later load is ordered after it
-    __device__ __forceinline__ void put_ecode(uint32_t r, uint32_t e) const { ec[r] = e; }
-    __device__ __forceinline__ uint32_t get_ecode(uint32_t r) const { return ec[r]; }
-};
-
-// Hybrid for walkers too large for Rec8/Rec10: chase codes in LDS (u16), links
-// in global memory through the scalar cache (K2 never writes them)
-struct RecH {
-    lds_u16 *ec;
-    const_u4 *lk;
-    static constexpr bool kChecked = true;
-    typedef uint64_t Key;
-    struct Word {
-        U4 l;
-        uint32_t e;
-    };
-    __device__ __forceinline__ Word load(uint32_t r) const
-    {
-        const_u4 &q = lk[r];
-        return Word{U4{q.x, q.y, q.z, q.w}, uni(ec[r])};
-    }
-    __device__ __forceinline__ static uint32_t ecode(const Word &x) { return x.e; }
-    __device__ __forceinline__ static uint32_t link(const Word &x, uint32_t leg)
-    {
-        return leg == 0 ? x.l.x : leg == 1 ? x.l.y : leg == 2 ? x.l.z : x.l.w;
-    }
-    __device__ __forceinline__ static void set_link0(Word &x, uint32_t v) { x.l.x = v; }
-    __device__ __forceinline__ void put_ecode(uint32_t r, uint32_t e) const { ec[r] = (uint16_t)e; }
-    __device__ __forceinline__ uint32_t get_ecode(uint32_t r) const { return ec[r]; }
-};
-
-// The four links of record r read by one vector load (lane j reads link
-// j & 3; lane-varying addresses are never turned into scalar loads) and made
-// wave-uniform with v_readlane.  Used inside the persistent launch, where the
-// diagonal/vertex-list phase rewrites the records between worm phases: the
-// scalar cache is not kept coherent with those vector stores within a launch.
-__device__ __forceinline__ U4 links_vec(const uint32_t *lk4, uint32_t r)
-{
-    const uint32_t v = as_global(lk4)[4u * r + (threadIdx.x & 3u)];
-    return U4{(uint32_t)__builtin_amdgcn_readlane((int)v, 0),
-              (uint32_t)__builtin_amdgcn_readlane((int)v, 1),
-              (uint32_t)__builtin_amdgcn_readlane((int)v, 2),
-              (uint32_t)__builtin_amdgcn_readlane((int)v, 3)};
-}
-
-// RecG with vector link loads (persistent launch)
-struct RecGV {
-    uint32_t *ec;
-    const uint32_t *lk;
-    static constexpr bool kChecked = true;
-    typedef uint64_t Key;
-    typedef RecG::Word Word;
-    __device__ __forceinline__ Word load(uint32_t r) const
-    {
-        const U4 l = links_vec(lk, r);
-        // the code: lane j reads code r + (j & 1) (r + 1 stays inside the
-        // slab: the link region follows the code array), so the load is a
-        // vector load as well
-        const uint32_t e = as_global(ec)[r + (threadIdx.x & 1u)];
-        return Word{l, (uint32_t)__builtin_amdgcn_readlane((int)e, 0)};
-    }
-    __device__ __forceinline__ static uint32_t ecode(const Word &x) { return x.e; }
-    __device__ __forceinline__ static uint32_t link(const Word &x, uint32_t leg) { return RecG::link(x, leg); }
-    __device__ __forceinline__ static void set_link0(Word &x, uint32_t v) { x.l.x = v; }
-    __device__ __forceinline__ void put_ecode(uint32_t r, uint32_t e) const { ec[r] = e; }
-    __device__ __forceinline__ uint32_t get_ecode(uint32_t r) const { return ec[r]; }
-};
-
-// RecH with vector link loads (persistent launch)
-struct RecHV {
-    lds_u16 *ec;
-    const uint32_t *lk;
-    static constexpr bool kChecked = true;
-    typedef uint64_t Key;
-    typedef RecH::Word Word;
-    __device__ __forceinline__ Word load(uint32_t r) const { return Word{links_vec(lk, r), uni(ec[r])}; }
-    __device__ __forceinline__ static uint32_t ecode(const Word &x) { return x.e; }
-    __device__ __forceinline__ static uint32_t link(const Word &x, uint32_t leg) { return RecH::link(x, leg); }
-    __device__ __forceinline__ static void set_link0(Word &x, uint32_t v) { x.l.x = v; }
-    __device__ __forceinline__ void put_ecode(uint32_t r, uint32_t e) const { ec[r] = (uint16_t)e; }
-    __device__ __forceinline__ uint32_t get_ecode(uint32_t r) const { return ec[r]; }
-};
-
-// Record index of the leg id held shifted in lidS (lid << S).  For the 8-byte
-// LDS records it is produced on the vector unit (v_bfe), so the record's LDS
-// address takes no scalar instruction and no scalar-to-vector move: the scalar
-// unit is what the chase runs out of when several walkers share a compute unit.
-template <class R, uint32_t S>
-struct RecIndex {
-    __device__ __forceinline__ static uint32_t of(typename R::Key lidS) { return (uint32_t)(lidS >> (S + 2)); }
-};
-template <uint32_t S>
-struct RecIndex<Rec8, S> {
-    __device__ __forceinline__ static uint32_t of(uint32_t lidS)
-    {
-        uint32_t r;
-        asm("v_bfe_u32 %0, %1, %2, 16" : "=v"(r) : "s"(lidS), "i"(S + 2));
-        return r;
-    }
-};
-
-// Exit selection of one scatter on the scalar unit: m = word >> 11 against the
-// entry's first three thresholds by 64-bit borrow chains (s_sub/s_subb leave
-// the borrow, m < K, in SCC), from the last to the first: out[j] for the first
-// j < 3 with m < K[j], else out[3].  The table puts the chase's slow marker
-// (kChaseSlow) wherever the answer is not simply out[3] (a fourth exit whose
-// threshold is below 2^53, more than four exits, a fall-through), so the
-// caller tests one bit of the result.
-__device__ __forceinline__ uint32_t chase_select(uint32_t mlo, uint32_t mhi, ConstEntry *E)
-{
-    // K[3] is loaded too (unused by the selection) so that the thresholds
-    // arrive in one 32-byte scalar load
-    const uint64_t K0 = E->K[0], K1 = E->K[1], K2 = E->K[2], K3 = E->K[3];
-    const uint32_t o0 = E->out[0], o1 = E->out[1], o2 = E->out[2], o3 = E->out[3];
-    uint32_t eo, t;
-    asm("s_sub_u32 %1, %2, %8\n\t"
-        "s_subb_u32 %1, %3, %9\n\t"
-        "s_cselect_b32 %0, %12, %13\n\t"
-        "s_sub_u32 %1, %2, %6\n\t"
-        "s_subb_u32 %1, %3, %7\n\t"
-        "s_cselect_b32 %0, %11, %0\n\t"
-        "s_sub_u32 %1, %2, %4\n\t"
-        "s_subb_u32 %1, %3, %5\n\t"
-        "s_cselect_b32 %0, %10, %0"
-        : "=&s"(eo), "=&s"(t)
-        : "s"(uni(mlo)), "s"(uni(mhi)), "s"((uint32_t)K0), "s"((uint32_t)(K0 >> 32)), "s"((uint32_t)K1),
-          "s"((uint32_t)(K1 >> 32)), "s"((uint32_t)K2), "s"((uint32_t)(K2 >> 32)), "s"(o0), "s"(o1),
-          "s"(o2), "s"(o3), "s"((uint32_t)K3), "s"((uint32_t)(K3 >> 32))
-        : "scc");
-    return eo;
-}
-
-// Worm start (sse.jl:241-251): draw (slot, leg) pairs until the leg belongs
-// to an operator (an operator's four legs are all linked), then the worm
-// function.  Returns the operator's rank r0, leg l0, the site's dimension and
-// the worm function wf0 (1-based); false when wf0 exceeds the chase table.
-__device__ __forceinline__ bool worm_start(const DevWalker &w, const DevModel &m, K2Stream &rs,
-                                           const gmem<uint64_t> *MASK, const gmem<uint32_t> *BASE,
-                                           uint32_t dmw, uint32_t &r0, uint32_t &l0, uint32_t &dim0,
-                                           uint32_t &wf0)
-{
-    const int64_t L = w.L;
-    int64_t p0;
-    for (;;) {
-        p0 = (int64_t)uni64(rs.range((uint64_t)L));
-        l0 = uni((uint32_t)rs.range(4));
-        const uint64_t mk = uni64(MASK[p0 >> 6]);
-        const int bit = (int)(p0 & 63);
-        if ((mk >> bit) & 1ull) {
-            r0 = uni(BASE[p0 >> 6] + (uint32_t)popc(mk & below_mask(bit)));
-            break;
-        }
-    }
-    const int2 b0 = m.bond_rec[op_bond(w.ops[p0])];
-    const uint32_t site0 = uni((uint32_t)((l0 & 1) ? b0.y : (b0.x & 0xFFFFF)));
-    dim0 = uni(m.site_dims[site0]);
-    wf0 = 1u + uni((uint32_t)rs.range((uint64_t)(dim0 - 1)));
-    return wf0 - 1u < dmw;
-}
-
-// The exact scatter (vertex_data.jl:113-125) of a step whose chase entry
-// carries the slow marker: the entry's own thresholds for up to four exits,
-// the exit list for more.  A fall-through or an invalid transition sets err
-// and returns efail (the code rewritten unchanged, exit leg 0, the worm field
-// of the closing test), which the caller turns into a loop exit.
-template <bool kOneWorm>
-__device__ __forceinline__ uint32_t chase_exact(const DevModel &m, const_char *CT, uint32_t eoff,
-                                                uint32_t mlo, uint32_t mhi, uint32_t e, uint32_t lgp,
-                                                uint32_t efail, uint32_t &err)
-{
-    ConstEntry *ES = (ConstEntry *)(CT + eoff);
-    const uint32_t cnt = uni(ES->count);
-    if (cnt <= 4u) {
-        const uint64_t mm = ((uint64_t)mhi << 32) | mlo;
-        uint32_t j = 0;
-        for (; j < cnt; ++j)
-            if (mm < uni64(ES->K[j]))
-                break;
-        if (j >= cnt) {
-            err = SSE_ERR_SCATTER;
-            return efail;
-        }
-        return uni(j < 3u ? ES->out[j] : ES->pad[0]);
-    }
-    const uint32_t trw = uni(ES->trans);
-    const WormTab tab = worm_tab((const char *)m.wtab, m);
-    const double xr = (double)(((uint64_t)mhi << 32) | mlo) * 0x1.0p-53;
-    uint32_t ex = trw & 0xFFFFFu;
-    const uint32_t eend = ex + (trw >> 20);
-    for (; ex < eend; ++ex) {
-        const uint64_t cb = uni64((uint64_t)__double_as_longlong(tab.cum[ex]));
-        if (xr < __longlong_as_double((long long)cb))
-            break;
-    }
-    if (ex >= eend) {
-        err = SSE_ERR_SCATTER;
-        return efail;
-    }
-    const uint32_t vc = uni(tab.eout[ex]);
-    const uint32_t ecn = (e >> lgp << lgp) | (vc & 1023u), lg = (vc >> 10) & 3u;
-    return kOneWorm ? chase_out1(ecn, lg) : chase_out(ecn, lg, vc >> 12);
-}
-
-// The worm update of one walker (sse.jl:193-303), executed uniformly by the
-// whole wave.  The chase is scalar work: the record and the next Philox word
-// leave LDS together and become wave-uniform at once, the transition entry
-// arrives in one scalar load (constant address space, uniform offset), the exit
-// is selected on the scalar unit, and the closing tests compare packed keys
-// (leg id << 14 | worm-1).  Returns an error code (0 = ok).
-template <class R, bool kOneWorm>
-__device__ __forceinline__ int worm_chase(DevWalker &w, const DevModel &m, K2Stream &rs, const R &rec,
-                          const gmem<uint64_t> *MASK, const gmem<uint32_t> *BASE, double &total,
-                          int64_t &scat)
-{
-    const uint32_t n = (uint32_t)w.n;
-    const int64_t nworms = (int64_t)ceil(w.num_worms);
-    const uint32_t dmw = uni((uint32_t)m.dt_mw);
-    const uint32_t lgp = uni((uint32_t)m.dt_lgp);
-    const uint32_t estride = dmw << 8;  // bytes per ecode
-    const_char *CT = (const_char *)(const void *)uni64((uint64_t)(const void *)m.dtab);
-    total = 1.0;
-    uint32_t sc = 0;
-    for (int64_t k = 0; k < nworms; ++k) {
-        if (n == 0)
-            continue;  // worm_traverse! returns 0 without draws (sse.jl:234-236)
-        uint32_t r0, l0, dim0, wf0;
-        if (!worm_start(w, m, rs, MASK, BASE, dmw, r0, l0, dim0, wf0))
-            return SSE_ERR_STATE;
-        const uint32_t lid0 = 4u * r0 + l0;
-        // closing tests (sse.jl:290-297), both on the key of the next leg: the
-        // worm leaves through (r0, l0) with worm dim0 - wf0 exactly when the hop
-        // lands on the leg linked to (r0, l0) (the links are an involution
-        // without fixed points, so at most one test holds), and it re-enters
-        // (r0, l0) with worm wf0.  Key = lid << S | worm-1; with one worm type
-        // the worm field is always 0 and S = 6 puts the leg at bits 6..7, the
-        // entry's leg offset in the transition table.
-        constexpr uint32_t S = kOneWorm ? 6u : 14u;
-        typedef typename R::Key Key;
-        const uint32_t lnk0 = uni(R::link(rec.load(r0), l0));
-        const Key keyA = ((Key)lnk0 << S) | (kOneWorm ? 0u : dim0 - wf0 - 1u);
-        const Key keyB = ((Key)lid0 << S) | (kOneWorm ? 0u : wf0 - 1u);
-        Key lidS = (Key)lid0 << S;
-        uint32_t wfm = wf0 - 1u;
-        // one Philox word per step: the step count is the stream advance
-        const uint64_t pos0 = rs.bbase + rs.off;
-        uint32_t err = 0;
-        Key kB = 0;
-        do {  // sse.jl:274-300
-            // the rare paths (refill, exact scatter, worm end) are marked
-            // unlikely so the step runs straight through with one taken branch
-            if (__builtin_expect(rs.off >= K2Stream::kNW, 0)) {
-                if (rs.off == K2Stream::kNW)
-                    rs.refill_next();
-                else
-                    rs.ensure(1);
-            }
-            const uint32_t off = uni(rs.off);
-            const uint32_t r = RecIndex<R, S>::of(lidS);
-            typename R::Word x = rec.load(r);
-            // rand() = mm * 2^-53: the mantissa of this step's word
-            const uint32_t mlo = (uint32_t)__builtin_amdgcn_readlane((int)rs.mlo, (int)off);
-            const uint32_t mhi = (uint32_t)__builtin_amdgcn_readlane((int)rs.mhi, (int)off);
-            rs.off = off + 1u;
-            const uint32_t e = R::ecode(x);
-            const uint32_t legbits = kOneWorm ? (uint32_t)lidS & 0xC0u          // leg_in << 6
-                                              : (uint32_t)(lidS >> 8) & 0xC0u;
-            const uint32_t eoff = kOneWorm ? (e << 8) | legbits : e * estride + (wfm << 8) + legbits;
-            ConstEntry *E = (ConstEntry *)(CT + eoff);
-            uint32_t eo = chase_select(mlo, mhi, E);
-            if (__builtin_expect((eo & kChaseSlowBit) != 0, 0)) {
-                // the entry's address is formed here, not hoisted into the fast path
-                uint32_t eoff_s = eoff;
-                asm volatile("" : "+s"(eoff_s));
-                const uint32_t efail = (e << 16) | (kOneWorm ? 0u : dim0 - wf0 - 1u);
-                eo = chase_exact<kOneWorm>(m, CT, eoff_s, mlo, mhi, e, lgp, efail, err);
-                if (err)  // exit leg 0 of the record copy becomes the leg linked to (r0, l0)
-                    R::set_link0(x, lnk0);
-            }
-            rec.put_ecode(r, eo >> 16);
-            uint32_t nx;
-            if constexpr (kOneWorm && std::is_same<R, Rec8>::value)
-                nx = Rec8::link_sh(x, eo);
-            else
-                nx = R::link(x, (eo >> 14) & 3u);
-            if (R::kChecked && (nx >> 2) >= n) {
-                err = SSE_ERR_STATE;
-                break;
-            }
-            const uint32_t wfn = kOneWorm ? 0u : eo & 0x3FFFu;
-            const Key nxS = (Key)nx << S;
-            kB = kOneWorm ? nxS : nxS | wfn;
-            lidS = nxS;
-            wfm = wfn;
-        } while (__builtin_expect(min(kB ^ keyA, kB ^ keyB) != 0, 1));
-        const uint32_t endB = kB != keyA;  // closed on re-entry
-        if (err)
-            return (int)err;
-        const uint32_t steps = (uint32_t)(rs.bbase + rs.off - pos0);
-        sc += steps;
-        // worm length: scatters + 1 when the worm closed on re-entry
-        total += (double)(steps + endB);
-    }
-    scat = sc;
-    return 0;
-}
-
-// The worm update with record lookahead, for the LDS record layouts (Rec8,
-// Rec10).  Same steps, draws and results as worm_chase; what changes is when
-// the next record is read.  At the top of a step the current record x is
-// wave-uniform, so lane j (j = lane % 4) reads, with one LDS instruction, the
-// record of the operator linked to leg j of x.  While those loads are in
-// flight the scalar unit selects the exit; the next record is then the word of
-// lane exit-leg (v_readlane), and the LDS latency leaves the step's
-// dependency chain.  The loads were issued before this step rewrote the
-// current operator's chase code, so a hop onto the same operator (a site
-// with one operator, linked to itself through the periodic closure) patches
-// the code into the picked record.
-template <class R, bool kOneWorm>
-__device__ __forceinline__ int worm_chase_la(DevWalker &w, const DevModel &m, K2Stream &rs, const R &rec,
-                             const gmem<uint64_t> *MASK, const gmem<uint32_t> *BASE, double &total,
-                             int64_t &scat)
-{
-    const uint32_t n = (uint32_t)w.n;
-    const int64_t nworms = (int64_t)ceil(w.num_worms);
-    const uint32_t dmw = uni((uint32_t)m.dt_mw);
-    const uint32_t lgp = uni((uint32_t)m.dt_lgp);
-    const uint32_t estride = dmw << 8;  // bytes per ecode
-    const_char *CT = (const_char *)(const void *)uni64((uint64_t)(const void *)m.dtab);
-    const uint32_t myleg = threadIdx.x & 3u;
-    total = 1.0;
-    uint32_t sc = 0;
-    for (int64_t k = 0; k < nworms; ++k) {
-        if (n == 0)
-            continue;  // worm_traverse! returns 0 without draws (sse.jl:234-236)
-        uint32_t r0, l0, dim0, wf0;
-        if (!worm_start(w, m, rs, MASK, BASE, dmw, r0, l0, dim0, wf0))
-            return SSE_ERR_STATE;
-        const uint32_t lid0 = 4u * r0 + l0;
-        constexpr uint32_t S = kOneWorm ? 6u : 14u;
-        typedef typename R::Key Key;
-        typename R::Word x = rec.load(r0);
-        const uint32_t lnk0 = uni(R::link(x, l0));
-        // closing tests as in worm_chase
-        const Key keyA = ((Key)lnk0 << S) | (kOneWorm ? 0u : dim0 - wf0 - 1u);
-        const Key keyB = ((Key)lid0 << S) | (kOneWorm ? 0u : wf0 - 1u);
-        Key lidS = (Key)lid0 << S;
-        uint32_t wfm = wf0 - 1u;
-        const uint64_t pos0 = rs.bbase + rs.off;
-        uint32_t err = 0;
-        Key kB = 0;
-        do {  // sse.jl:274-300
-            // the records linked to the current operator's four legs
-            const typename R::Cand cand = rec.load_lane(R::link(x, myleg) >> 2);
-            if (__builtin_expect(rs.off >= K2Stream::kNW, 0)) {
-                if (rs.off == K2Stream::kNW)
-                    rs.refill_next();
-                else
-                    rs.ensure(1);
-            }
-            const uint32_t off = uni(rs.off);
-            const uint32_t r = RecIndex<R, S>::of(lidS);
-            const uint32_t mlo = (uint32_t)__builtin_amdgcn_readlane((int)rs.mlo, (int)off);
-            const uint32_t mhi = (uint32_t)__builtin_amdgcn_readlane((int)rs.mhi, (int)off);
-            rs.off = off + 1u;
-            const uint32_t e = R::ecode(x);
-            const uint32_t legbits = kOneWorm ? (uint32_t)lidS & 0xC0u
-                                              : (uint32_t)(lidS >> 8) & 0xC0u;
-            const uint32_t eoff = kOneWorm ? (e << 8) | legbits : e * estride + (wfm << 8) + legbits;
-            ConstEntry *E = (ConstEntry *)(CT + eoff);
-            uint32_t eo = chase_select(mlo, mhi, E);
-            if (__builtin_expect((eo & kChaseSlowBit) != 0, 0)) {
-                uint32_t eoff_s = eoff;
-                asm volatile("" : "+s"(eoff_s));
-                const uint32_t efail = (e << 16) | (kOneWorm ? 0u : dim0 - wf0 - 1u);
-                eo = chase_exact<kOneWorm>(m, CT, eoff_s, mlo, mhi, e, lgp, efail, err);
-                if (err)
-                    R::set_link0(x, lnk0);
-            }
-            const uint32_t enew = eo >> 16;
-            rec.put_ecode(r, enew);
-            const uint32_t leg = (eo >> 14) & 3u;
-            uint32_t nx;
-            if constexpr (kOneWorm && std::is_same<R, Rec8>::value)
-                nx = Rec8::link_sh(x, eo);
-            else
-                nx = R::link(x, leg);
-            typename R::Word xn = R::pick(cand, leg);
-            // (the record index on the scalar unit: r itself is a vector
-            // register, the LDS address of the code store)
-            if ((nx >> 2) == (uint32_t)(lidS >> (S + 2)))
-                R::set_ecode(xn, enew);
-            const uint32_t wfn = kOneWorm ? 0u : eo & 0x3FFFu;
-            const Key nxS = (Key)nx << S;
-            kB = kOneWorm ? nxS : nxS | wfn;
-            lidS = nxS;
-            wfm = wfn;
-            x = xn;
-        } while (__builtin_expect(min(kB ^ keyA, kB ^ keyB) != 0, 1));
-        const uint32_t endB = kB != keyA;
-        if (err)
-            return (int)err;
-        const uint32_t steps = (uint32_t)(rs.bbase + rs.off - pos0);
-        sc += steps;
-        total += (double)(steps + endB);
-    }
-    scat = sc;
-    return 0;
-}
-
-// state refresh (sse.jl:219-228) and operator write-back after the worms
-template <class R>
-__device__ __noinline__ void worm_writeback(R rec, uint32_t lgp, uint32_t *ops_p, int64_t L,
-                                            const gmem<uint64_t> *MASK, const gmem<uint32_t> *BASE);
-
-template <class R, class RS>
-__device__ __forceinline__ void worm_finish(DevWalker &w, const DevModel &m, RS &rs, const R &rec,
-                            const gmem<uint64_t> *MASK, const gmem<uint32_t> *BASE)
-{
-    const int lane = threadIdx.x;
-    const int N = m.n_sites;
-    const uint32_t lgp = (uint32_t)m.dt_lgp;
-    // sites in blocks of 32 so that one block draws at most 32 words (the
-    // stream holds 64)
-    for (int sb = 0; sb < N; sb += 32) {
-        const int s = sb + lane;
-        const bool vs = lane < 32 && s < N;
-        const int32_t f = vs ? w.first[s] : 0;
-        const bool fr = vs && f < 0;
-        const uint64_t frm = __ballot(fr);
-        const int D = popc(frm);
-        const uint64_t dim = vs ? (uint64_t)m.site_dims[s] : 1;
-        bool reject = false;
-        uint8_t val = 0;
-        if (D > 0) {
-            rs.ensure((uint32_t)D);
-            // every lane takes part in the cross-lane read; lane s of the
-            // refreshed sites uses word off + (its rank among them)
-            const uint64_t x = rs.peek(fr ? (uint32_t)popc(frm & below_mask(lane)) : 0u);
-            if (fr) {
-                uint64_t lo = x * dim;
-                if (lo < dim && lo < (0ull - dim) % dim)
-                    reject = true;
-                val = (uint8_t)(1 + __umul64hi(x, dim));
-            }
-        }
-        if (vs && !fr && (int64_t)(f >> 2) < w.n) {
-            const uint32_t vt = vt_of_ecode(rec.get_ecode((uint32_t)f >> 2), lgp);
-            const DevVD &vd = m.types[vt >> 10];
-            val = vd.leg_states[4 * ((vt & 1023u) >> 1) + (f & 3)];
-        }
-        if (__ballot(reject)) {
-            for (int i = 0; i < 32 && sb + i < N; ++i) {
-                const bool fi = (frm >> i) & 1ull;
-                uint8_t vi = 0;
-                if (fi)
-                    vi = (uint8_t)(1 + rs.range((uint64_t)m.site_dims[sb + i]));
-                if (lane == i && fi)
-                    val = vi;
-            }
-        } else {
-            rs.advance((uint32_t)D);
-        }
-        if (vs)
-            w.spins[s] = val;
-    }
-    worm_writeback<R>(rec, lgp, w.ops, w.L, MASK, BASE);
-}
-
-// Write the worm-updated vertex codes back into the operator string (the
-// last step of the worm update), K 64-slot chunks per pass so their loads are
-// in flight together: lane u loads chunk u's mask and base (vector loads, read
-// back by v_readlane), every lane its slot of each chunk.  A function of its
-// own: inlined, its registers would crowd the chase loop's scalar operands.
-template <class R>
-__device__ __noinline__ void worm_writeback(R rec, uint32_t lgp, uint32_t *ops_p, int64_t L,
-                                            const gmem<uint64_t> *MASK, const gmem<uint32_t> *BASE)
-{
-    const int lane = threadIdx.x;
-    constexpr int K = 16;
-    gmem<uint32_t> *ops = as_global(ops_p);
-    for (int64_t base = 0; base < L; base += 64 * K) {
-        const int64_t cl = (base >> 6) + lane;
-        const bool lin = lane < K && base + 64 * lane < L;
-        const uint64_t mkl = lin ? MASK[cl] : 0ull;
-        const uint32_t bsl = lin ? BASE[cl] : 0u;
-        uint32_t op[K];
-#pragma unroll
-        for (int u = 0; u < K; ++u) {
-            const int64_t p = base + 64 * u + lane;
-            op[u] = p < L ? ops[p] : 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < K; ++u) {
-            const uint64_t mk = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mkl >> 32), u) << 32) |
-                                (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mkl, u);
-            if ((mk >> lane) & 1ull) {
-                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)bsl, u) +
-                                   (uint32_t)popc(mk & below_mask(lane));
-                const uint32_t vc = vt_of_ecode(rec.get_ecode(r), lgp) & 1023u;
-                const uint32_t nop = (op[u] & ~(1023u << 1)) | (vc << 1);
-                if (nop != op[u])
-                    ops[base + 64 * u + lane] = nop;
-            }
-        }
-    }
-}
-
-// LDS bytes the worm kernel needs for a walker with n operators, cutoff L, in
-// the Rec8 (fmt 8) or Rec10 (fmt 10) layout
-__host__ __device__ inline size_t k2_lds_need(int64_t n, int64_t, int fmt)
-{
-    const size_t b = 0;  // the Philox words live in registers
-    if (fmt == 2)                        // RecH: chase codes only
-        return b + (((size_t)n * 2 + 15) & ~(size_t)15);
-    return b + (size_t)n * 8 + (fmt == 10 ? (((size_t)n * 2 + 15) & ~(size_t)15) : 0);
-}
-
-// LDS per walker the worm kernel is sized for at most: beyond it a walker uses
-// the hybrid or global records instead of lowering every walker's residency
-constexpr size_t K2_LDS_CAP = 65536;
-
-// Stage the compact records of K1 (global) into the LDS layout R, converting
-// vt to ecodes and checking every ecode and link; returns false on a bad record.
-// K 64-record chunks per pass, their loads in flight together; a function of
-// its own (arguments by value) so that its registers stay out of the chase's.
-template <int FMT>
-__device__ __noinline__ bool k2_stage_records(uint32_t n, uint32_t lgp, uint32_t nt, const uint32_t *vt_p,
-                                              const U4 *lk_p, lds_u64 *lk, lds_u16 *ec)
-{
-    constexpr int K = 16;
-    const int lane = threadIdx.x;
-    const gmem<uint32_t> *gvt = as_global(vt_p);
-    const gmem<U4> *glk = as_global(lk_p);
-    const uint32_t lmax = 4u * n;
-    bool bad = false;
-    for (uint32_t i0 = 0; i0 < n; i0 += 64 * K) {
-        uint32_t vt[K];
-        uint4 l4[K];
-#pragma unroll
-        for (int u = 0; u < K; ++u) {
-            const uint32_t i = i0 + 64u * u + lane;
-            if (i < n) {
-                vt[u] = gvt[i];
-                const gmem<U4> &q = glk[i];
-                l4[u] = make_uint4(q.x, q.y, q.z, q.w);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < K; ++u) {
-            const uint32_t i = i0 + 64u * u + lane;
-            if (i < n) {
-                const uint32_t e = ecode_of_vt(vt[u], lgp);
-                bad |= (vt[u] & 1023u) >= (1u << lgp) || (vt[u] >> 10) >= nt || l4[u].x >= lmax ||
-                       l4[u].y >= lmax || l4[u].z >= lmax || l4[u].w >= lmax;
-                if (FMT == 8) {
-                    lk[i] = (uint64_t)l4[u].x | ((uint64_t)l4[u].y << 14) | ((uint64_t)l4[u].z << 28) |
-                            ((uint64_t)l4[u].w << 42) | ((uint64_t)e << 56);
-                } else {
-                    lk[i] = (uint64_t)l4[u].x | ((uint64_t)l4[u].y << 16) | ((uint64_t)l4[u].z << 32) |
-                            ((uint64_t)l4[u].w << 48);
-                    ec[i] = (uint16_t)e;
-                }
-            }
-        }
-    }
-    return __ballot(bad) == 0;
-}
-
-template <int FMT>
-__device__ __forceinline__ bool k2_stage(const DevWalker &w, const DevModel &m, lds_u64 *lk, lds_u16 *ec)
-{
-    return k2_stage_records<FMT>((uint32_t)w.n, (uint32_t)m.dt_lgp, (uint32_t)m.n_types,
-                                 (const uint32_t *)rec_vt(w), (const U4 *)rec_link(w), lk, ec);
-}
-
-// vt -> ecode into an LDS u16 array (RecH path), checking every code.
-__device__ bool k2_stage_codes(const DevWalker &w, const DevModel &m, lds_u16 *ec)
-{
-    const int lane = threadIdx.x;
-    const uint32_t n = (uint32_t)w.n, lgp = (uint32_t)m.dt_lgp, nt = (uint32_t)m.n_types;
-    const gmem<uint32_t> *gvt = as_global((const uint32_t *)rec_vt(w));
-    bool bad = false;
-    for (uint32_t i = lane; i < n; i += 64) {
-        const uint32_t vt = gvt[i];
-        bad |= (vt & 1023u) >= (1u << lgp) || (vt >> 10) >= nt;
-        ec[i] = (uint16_t)ecode_of_vt(vt, lgp);
-    }
-    return __ballot(bad) == 0;
-}
-
-// In-place vt -> ecode conversion of the global records (RecG path).
-__device__ bool k2_stage_global(const DevWalker &w, const DevModel &m)
-{
-    const int lane = threadIdx.x;
-    const uint32_t n = (uint32_t)w.n, lgp = (uint32_t)m.dt_lgp, nt = (uint32_t)m.n_types;
-    uint32_t *gvt = rec_vt(w);
-    bool bad = false;
-    for (uint32_t i = lane; i < n; i += 64) {
-        const uint32_t vt = gvt[i];
-        bad |= (vt & 1023u) >= (1u << lgp) || (vt >> 10) >= nt;
-        gvt[i] = ecode_of_vt(vt, lgp);
-    }
-    return __ballot(bad) == 0;
-}
-
-// Worm update of walker wi.  LDS holds the records only (the Philox words are
-// in registers).  RecG reads links through the scalar cache, which is
-// valid because K1 wrote them in an earlier kernel launch.
-// kFused: called inside the persistent launch (global link records read by
-// vector loads, RecHV / RecGV)
-template <bool kFused>
-__device__ __forceinline__ void k2_walker(DevWalker *W, const DevModel *models, DevPool *pool, int wi,
-                                          int full_sweep, int lds_bytes, int rec_mode, char *lds,
-                                          int chase)
-{
-    const int lane = threadIdx.x;
-    DevWalker w = W[wi];
-    if (w.error || !w.active || w.retire)
-        return;
-    const DevModel &m = models[w.model];
-    const bool therm = w.sweeps > w.thermalization;
-    K2Stream rs;
-    rs.init(w.key, w.ctr);
-    const bool small_codes = ((int64_t)m.n_types << m.dt_lgp) <= 256;
-    const bool u16_codes = ((int64_t)m.n_types << m.dt_lgp) <= 65536;
-    int fmt = 0;
-    if (rec_mode == 0 && w.n <= 4096 && small_codes && k2_lds_need(w.n, w.L, 8) <= (size_t)lds_bytes)
-        fmt = 8;
-    else if (rec_mode <= 1 && w.n <= 16384 && u16_codes && k2_lds_need(w.n, w.L, 10) <= (size_t)lds_bytes)
-        fmt = 10;
-    else if ((rec_mode <= 1 || rec_mode == 3) && u16_codes && k2_lds_need(w.n, w.L, 2) <= (size_t)lds_bytes)
-        fmt = 2;
-    // chunk masks and bases stay in global memory (worm starts and write-back)
-    const gmem<uint64_t> *gmask = as_global((const uint64_t *)rec_mask(w));
-    const gmem<uint32_t> *gbase = as_global((const uint32_t *)rec_base(w));
-    double total = 1.0;
-    int64_t scat = 0;
-    int err = 0;
-    // records at the start of the walker's LDS
-    char *q = lds;
-    if (fmt == 2) {
-        lds_u16 *lec = (lds_u16 *)(uint16_t *)q;
-        const bool ok = k2_stage_codes(w, m, lec);
-        __syncthreads();
-        if (!ok) {
-            err = SSE_ERR_STATE;
-        } else {
-            if constexpr (kFused) {
-                RecHV rec{lec, (const uint32_t *)rec_link(w)};
-                err = m.dt_mw == 1 ? worm_chase<RecHV, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase<RecHV, false>(w, m, rs, rec, gmask, gbase, total, scat);
-                __syncthreads();
-                if (!err)
-                    worm_finish(w, m, rs, rec, gmask, gbase);
-            } else {
-                RecH rec{lec, (const_u4 *)(const void *)rec_link(w)};
-                err = m.dt_mw == 1 ? worm_chase<RecH, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase<RecH, false>(w, m, rs, rec, gmask, gbase, total, scat);
-                __syncthreads();
-                if (!err)
-                    worm_finish(w, m, rs, rec, gmask, gbase);
-            }
-        }
-    } else if (fmt) {
-        lds_u64 *llk = (lds_u64 *)(uint64_t *)q;
-        lds_u16 *lec = (lds_u16 *)(uint16_t *)(q + w.n * 8);
-        const bool ok = fmt == 8 ? k2_stage<8>(w, m, llk, lec) : k2_stage<10>(w, m, llk, lec);
-        __syncthreads();
-        if (!ok) {
-            err = SSE_ERR_STATE;
-        } else if (fmt == 8) {
-            Rec8 rec{llk};
-            if (chase == 1)
-                err = m.dt_mw == 1 ? worm_chase_la<Rec8, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase_la<Rec8, false>(w, m, rs, rec, gmask, gbase, total, scat);
-            else
-                err = m.dt_mw == 1 ? worm_chase<Rec8, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase<Rec8, false>(w, m, rs, rec, gmask, gbase, total, scat);
-            __syncthreads();
-            if (!err)
-                worm_finish(w, m, rs, rec, gmask, gbase);
-        } else {
-            Rec10 rec{llk, lec};
-            if (chase == 1)
-                err = m.dt_mw == 1 ? worm_chase_la<Rec10, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase_la<Rec10, false>(w, m, rs, rec, gmask, gbase, total, scat);
-            else
-                err = m.dt_mw == 1 ? worm_chase<Rec10, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase<Rec10, false>(w, m, rs, rec, gmask, gbase, total, scat);
-            __syncthreads();
-            if (!err)
-                worm_finish(w, m, rs, rec, gmask, gbase);
-        }
-    } else {
-        if (!k2_stage_global(w, m)) {
-            err = SSE_ERR_STATE;
-        } else {
-            // one-worm tables carry 14 * leg in the worm field: the one-worm chase
-            if constexpr (kFused) {
-                RecGV rec{rec_vt(w), (const uint32_t *)rec_link(w)};
-                err = m.dt_mw == 1 ? worm_chase<RecGV, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase<RecGV, false>(w, m, rs, rec, gmask, gbase, total, scat);
-                __syncthreads();
-                if (!err)
-                    worm_finish(w, m, rs, rec, gmask, gbase);
-            } else {
-                RecG rec{rec_vt(w), (const_u4 *)(const void *)rec_link(w)};
-                err = m.dt_mw == 1 ? worm_chase<RecG, true>(w, m, rs, rec, gmask, gbase, total, scat)
-                                   : worm_chase<RecG, false>(w, m, rs, rec, gmask, gbase, total, scat);
-                __syncthreads();
-                if (!err)
-                    worm_finish(w, m, rs, rec, gmask, gbase);
-            }
-        }
-    }
-    if (err) {
-        if (lane == 0) {
-            W[wi].error = err;
-            flag_error(pool, err);
-        }
-        return;
-    }
-    w.last_scatter = scat;
-    worm_controller(w, total, therm);
-    if (lane == 0) {
-        DevWalker &o = W[wi];
-        o.ctr = rs.ctr();
-        o.avg_worm_length = w.avg_worm_length;
-        o.num_worms = w.num_worms;
-        o.last_scatter = w.last_scatter;
-        o.last_total = w.last_total;
-        o.last_wlf = w.last_wlf;
-        if (full_sweep) {
-            o.sweeps = w.sweeps + 1;
-            o.acc_L = w.acc_L + w.L;
-            o.acc_n = w.acc_n + w.n;
-            o.acc_W = w.acc_W + scat;
-            o.acc_sweeps = w.acc_sweeps + 1;
-            if (w.remaining > 0) {
-                o.remaining = w.remaining - 1;
-                if (w.remaining == 1)
-                    o.retire = 1;
-            }
-        }
-    }
-}
-
-// K2.  rec_mode 0 picks the smallest record layout that fits (Rec8, Rec10,
-// RecH, then RecG); 1 skips Rec8; 2 forces RecG; 3 forces RecH.  chase 1
-// runs the LDS layouts with record lookahead, 0 without.
+// LDS holds the walker's worm records and exit table when they fit lds_bytes;
+// rec_mode as worm_walker's mode.
 __global__ __launch_bounds__(64) void wave_worm_kernel(DevWalker *W, const DevModel *models,
                                                        DevPool *pool, int w_begin, int w_end,
                                                        int full_sweep, int lds_bytes, int rec_mode,
-                                                       const int32_t *order, int chase)
+                                                       const int32_t *order)
 {
     extern __shared__ __align__(16) char lds[];
     const int pos = w_begin + (int)blockIdx.x;
     if (pos < w_end)
-        k2_walker<false>(W, models, pool, walker_at(order, pos), full_sweep, lds_bytes, rec_mode, lds,
-                         chase);
+        worm_walker<2>(W, models, pool, walker_at(order, pos), full_sweep, lds_bytes, rec_mode, lds);
 }
 
 // ------------------------------------------------------------------ init
@@ -1823,7 +843,6 @@ __device__ __forceinline__ void k3_finish(const DevWalker &w, const DevModel &m,
                                           bool want_sign, int neg, int64_t cnt, const double *tmp0,
                                           const double *mag, const double *absmag, const double *mag2,
                                           const double *mag4, double &sign, double *o);
-template <bool kTable = true>
 __device__ __forceinline__ void k3_pass(const DevWalker &w, const DevModel &m, int e0, int ne,
                                         bool want_sign, double &sign, double *o)
 {
@@ -1847,7 +866,7 @@ __device__ __forceinline__ void k3_pass(const DevWalker &w, const DevModel &m, i
     int neg = 0;
     int64_t cnt = 0;
     const gmem<uint32_t> *ops = as_global((const uint32_t *)w.ops);
-    if (kTable && m.est_dtab) {
+    if (m.est_dtab) {
         // per-(bond, vertex) tables: an operator's estimator changes and sign
         // are one gather each; the operator is loaded two chunks ahead, its
         // table values one ahead
@@ -2028,7 +1047,6 @@ __device__ __forceinline__ void k3_finish(const DevWalker &w, const DevModel &m,
 // mode 1: thermalized walkers only, accumulated into the per-walker sums
 // (fused sweep+measure loop).  Estimators are taken K3_MAXE per pass over the
 // operator string; the first pass also computes the sign.
-template <bool kTable = true>
 __device__ __forceinline__ void k3_walker(DevWalker *W, const DevModel *models, double *out, double *sum,
                                           double *sumsq, int64_t *count, double *wlf, int wi, int mode,
                                           int32_t *done)
@@ -2052,7 +1070,7 @@ __device__ __forceinline__ void k3_walker(DevWalker *W, const DevModel *models, 
     int e0 = 0;
     do {
         const int ne = m.n_est - e0 < K3_MAXE ? m.n_est - e0 : K3_MAXE;
-        k3_pass<kTable>(w, m, e0, ne, e0 == 0, sign, o);
+        k3_pass(w, m, e0, ne, e0 == 0, sign, o);
         e0 += K3_MAXE;
     } while (e0 < m.n_est);
     const double nn = (double)w.n;
@@ -2098,21 +1116,19 @@ __global__ __launch_bounds__(64) void wave_measure_kernel(DevWalker *W, const De
 // measurement runs inside the launch's worm tail instead of after it.  The
 // measurement reads the operator string, spins and DevWalker that the worm
 // phase of the same wave has just stored, through vector loads after the
-// barrier (nothing of it goes through the scalar cache).  Its measurement
-// gathers the estimator values (no per-(bond, vertex) tables): with those the
-// compiler cannot keep the chase's operands in scalar registers.
+// barrier (nothing of it goes through the scalar cache).
 __global__ __launch_bounds__(64) void wave_worm_measure_kernel(
     DevWalker *W, const DevModel *models, DevPool *pool, int w_begin, int w_end, int lds_bytes,
-    int rec_mode, const int32_t *order, int chase, double *out, double *sum, double *sumsq,
-    int64_t *count, double *wlf, int32_t *done)
+    int rec_mode, const int32_t *order, double *out, double *sum, double *sumsq, int64_t *count,
+    double *wlf, int32_t *done)
 {
     extern __shared__ __align__(16) char lds[];
     const int pos = w_begin + (int)blockIdx.x;
     if (pos < w_end) {
         const int wi = walker_at(order, pos);
-        k2_walker<false>(W, models, pool, wi, 1, lds_bytes, rec_mode, lds, chase);
+        worm_walker<2>(W, models, pool, wi, 1, lds_bytes, rec_mode, lds);
         __syncthreads();
-        k3_walker<false>(W, models, out, sum, sumsq, count, wlf, wi, 1, done);
+        k3_walker(W, models, out, sum, sumsq, count, wlf, wi, 1, done);
     }
 }
 
@@ -2174,15 +1190,12 @@ static inline int wave_configure(WaveConfig &c, const std::vector<DevModel> &mod
         c.lds_limit = (size_t)lim;
     if (c.lds_k1 > c.lds_limit || (c.generic && c.lds_k1n > c.lds_limit))
         return SSE_ERR_INVALID;
-    c.small_codes = true;
-    for (const DevModel &m : models) {
-        c.max_wtab = std::max(c.max_wtab, (int)m.dtab_bytes);
-        if (((int64_t)m.n_types << m.dt_lgp) > 256)
-            c.small_codes = false;
-    }
     c.lds_k2 = 4096;
-    c.lds_k2n = 4096;
     if (c.lds_limit > 65536) {
+        (void)hipFuncSetAttribute((const void *)waven_worm_kernel,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds_limit);
+        (void)hipFuncSetAttribute((const void *)wave_worm_measure_kernel,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds_limit);
         (void)hipFuncSetAttribute((const void *)wave_worm_kernel,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds_limit);
         (void)hipFuncSetAttribute((const void *)wave_diag_vlist_kernel,
@@ -2191,21 +1204,21 @@ static inline int wave_configure(WaveConfig &c, const std::vector<DevModel> &mod
     return SSE_OK;
 }
 
-// Worm-kernel LDS per walker for the largest walker of the last call (max n,
-// max L) with a little headroom; walkers that do not fit take a slower record
-// layout for that sweep.  The allocation is then widened to the largest size
-// that keeps the same number of walkers per CU (more headroom at no cost in
-// residency).
-static inline size_t wave_k2_lds_for(const WaveConfig &c, unsigned long long max_n,
-                                     unsigned long long max_L)
+// LDS per walker the worm kernel is sized for at most: beyond it a walker keeps
+// its records in global memory instead of lowering every walker's residency
+constexpr size_t K2_LDS_CAP = 65536;
+
+// Worm-kernel LDS per walker for the largest need (worm_lds_need) among the
+// last call's walkers, with a little headroom; walkers that do not fit keep
+// their records in global memory for that sweep.  The allocation is then
+// widened to the largest size that keeps the same number of walkers per CU
+// (more headroom at no cost in residency).
+static inline size_t wave_k2_lds_for(const WaveConfig &c, unsigned long long max_need)
 {
     if (c.lds_k2_fixed)
         return c.lds_k2_fixed;
-    const int64_t nh = (int64_t)(max_n + 16);
-    size_t need = k2_lds_need(nh, (int64_t)max_L, nh <= 4096 && c.small_codes && c.rec_mode == 0 ? 8
-                                                  : c.rec_mode == 3                           ? 2
-                                                                                              : 10);
-    if (need > K2_LDS_CAP)  // larger walkers take the hybrid or global records
+    size_t need = (size_t)max_need + (size_t)max_need / 64 + 256;
+    if (need > K2_LDS_CAP)
         need = K2_LDS_CAP;
     need = (need + 255) & ~(size_t)255;
     if (need > c.lds_limit)
@@ -2223,13 +1236,9 @@ static inline size_t wave_k2_lds_for(const WaveConfig &c, unsigned long long max
     return wide;
 }
 
-static inline void wave_resize_lds(WaveConfig &c, unsigned long long max_n, unsigned long long max_L)
+static inline void wave_resize_lds(WaveConfig &c, unsigned long long max_need)
 {
-    c.lds_k2 = wave_k2_lds_for(c, max_n, max_L);
-    // generic worm kernel: the chase codes of the largest walker and some
-    // headroom, at most 64 KiB (larger walkers chase the global records)
-    size_t g = (2 * ((size_t)max_n + 64) + 255) & ~(size_t)255;
-    c.lds_k2n = g > 65536 ? 65536 : g;
+    c.lds_k2 = wave_k2_lds_for(c, max_need);
 }
 
 static inline int wave_launch_init(WaveConfig &c, hipStream_t s, DevWalker *W, const DevModel *M,
@@ -2259,6 +1268,7 @@ static inline int wave_launch_sweep(WaveConfig &c, hipStream_t s, DevWalker *W, 
     const int n = w1 - w0;
     const int k1 = phases & (1 | 2 | 8);
     const int g = grp >= 0 && grp < 7 ? grp : 7;  // slot 7 collects the rest
+    const size_t lds2 = g < 7 && c.lds_k2_group[g] ? c.lds_k2_group[g] : c.lds_k2;
     if (c.generic) {
         if (k1 & 3)
             hipLaunchKernelGGL(waven_diag_vlist_kernel, dim3(n), dim3(64), c.lds_k1n, s, W, M, pool, w0,
@@ -2266,14 +1276,13 @@ static inline int wave_launch_sweep(WaveConfig &c, hipStream_t s, DevWalker *W, 
         if (ev)
             (void)hipEventRecord(ev[1], s);
         if (phases & 4)
-            hipLaunchKernelGGL(waven_worm_kernel, dim3(n), dim3(64), c.lds_k2n, s, W, M, pool, w0, w1,
+            hipLaunchKernelGGL(waven_worm_kernel, dim3(n), dim3(64), lds2, s, W, M, pool, w0, w1,
                                (phases & 7) == 7 ? 1 : 0, order, (const int32_t *)nullptr, 0,
-                               (int)c.lds_k2n);
+                               (int)lds2, c.rec_mode);
         if (ev)
             (void)hipEventRecord(ev[2], s);
         return hipGetLastError() == hipSuccess ? SSE_OK : SSE_ERR_HIP;
     }
-    const size_t lds2 = g < 7 && c.lds_k2_group[g] ? c.lds_k2_group[g] : c.lds_k2;
     if (k1 & 3) {
         hipLaunchKernelGGL(wave_diag_vlist_kernel, dim3(n), dim3(64), c.lds_k1, s, W, M, pool, w0, w1, k1,
                            -1, (int)c.lds_k1, order, g);
@@ -2282,7 +1291,7 @@ static inline int wave_launch_sweep(WaveConfig &c, hipStream_t s, DevWalker *W, 
         (void)hipEventRecord(ev[1], s);
     if (phases & 4)
         hipLaunchKernelGGL(wave_worm_kernel, dim3(n), dim3(64), lds2, s, W, M, pool, w0, w1,
-                           (phases & 7) == 7 ? 1 : 0, (int)lds2, c.rec_mode, order, c.chase);
+                           (phases & 7) == 7 ? 1 : 0, (int)lds2, c.rec_mode, order);
     if (ev)
         (void)hipEventRecord(ev[2], s);
     return hipGetLastError() == hipSuccess ? SSE_OK : SSE_ERR_HIP;
@@ -2312,7 +1321,7 @@ static inline int wave_launch_sweep_measure(WaveConfig &c, hipStream_t s, DevWal
     if (ev)
         (void)hipEventRecord(ev[1], s);
     hipLaunchKernelGGL(wave_worm_measure_kernel, dim3(n), dim3(64), lds2, s, W, M, pool, w0, w1,
-                       (int)lds2, c.rec_mode, order, c.chase, out, sum, sumsq, count, wlf, done);
+                       (int)lds2, c.rec_mode, order, out, sum, sumsq, count, wlf, done);
     if (ev)
         (void)hipEventRecord(ev[2], s);
     return hipGetLastError() == hipSuccess ? SSE_OK : SSE_ERR_HIP;

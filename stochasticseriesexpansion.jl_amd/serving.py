@@ -92,7 +92,7 @@ def footprint_bytes(n_sites, n_bonds, T):
     n_est = beta * n_bonds * 0.375 * 2.5 + 64
     L = int(2.2 * n_est) + 128
     cap = L + L // 2 + 100
-    return 24 * cap + 16 * (cap // 64 + 1)
+    return 24 * cap + 12 * n_sites
 
 
 def latency_stats(jobs, t_end):
