@@ -662,27 +662,63 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
         o_esg = put(sgb.data(), sgb.size());
     }
     // diagonal-update table (layout: DevModel::k1tab)
-    std::vector<char> k1((size_t)16 * m.n_types);
-    for (int t = 0; t < m.n_types && ns == 2; ++t) {
-        const sse_vertex_data_desc &vd = m.types[t];
-        auto align8 = [&]() { k1.resize((k1.size() + 7) & ~(size_t)7); };
-        align8();
-        const uint32_t w_off = (uint32_t)k1.size();
-        k1.resize(k1.size() + 8 * (size_t)vd.n_vertices);
-        memcpy(k1.data() + w_off, vd.weights, 8 * (size_t)vd.n_vertices);
-        const uint32_t dv_off = (uint32_t)k1.size();
-        const int ndv = vd.dims[0] * vd.dims[1];
-        k1.resize(k1.size() + 2 * (size_t)ndv);
-        for (int i = 0; i < ndv; ++i) {
-            const int16_t c = (int16_t)vd.diagonal_vertices[i];
-            memcpy(k1.data() + dv_off + 2 * i, &c, 2);
+    std::vector<char> k1;
+    std::vector<int> k1group(m.n_types, 0);
+    int k1_groups = 0;
+    uint32_t k1_boff = 0;
+    if (ns == 2) {
+        std::map<std::string, int> seen;
+        std::vector<int> rep;
+        for (int t = 0; t < m.n_types; ++t) {
+            const sse_vertex_data_desc &vd = m.types[t];
+            std::string key;
+            auto add = [&](const void *p, size_t bytes) { key.append((const char *)p, bytes); };
+            add(vd.dims, 2 * sizeof vd.dims[0]);
+            add(&vd.n_vertices, sizeof vd.n_vertices);
+            add(vd.weights, 8 * (size_t)vd.n_vertices);
+            add(vd.leg_states, 4 * (size_t)vd.n_vertices);
+            add(vd.diagonal_vertices, 4 * (size_t)vd.dims[0] * vd.dims[1]);
+            auto it = seen.emplace(std::move(key), k1_groups);
+            k1group[t] = it.first->second;
+            if (it.second) {
+                rep.push_back(t);
+                ++k1_groups;
+            }
         }
-        const uint32_t ls_off = (uint32_t)k1.size();
-        k1.resize(k1.size() + 4 * (size_t)vd.n_vertices);
-        memcpy(k1.data() + ls_off, vd.leg_states, 4 * (size_t)vd.n_vertices);
-        const uint32_t h[4] = {w_off, dv_off, ls_off,
-                               (uint32_t)vd.n_vertices | ((uint32_t)vd.dims[0] << 16)};
-        memcpy(k1.data() + 16 * (size_t)t, h, 16);
+        k1.resize((size_t)16 * k1_groups);
+        for (int g = 0; g < k1_groups; ++g) {
+            const sse_vertex_data_desc &vd = m.types[rep[g]];
+            const int ndv = vd.dims[0] * vd.dims[1];
+            k1.resize((k1.size() + 15) & ~(size_t)15);
+            const uint32_t dw_off = (uint32_t)k1.size();
+            k1.resize(k1.size() + 16 * (size_t)ndv);
+            for (int i = 0; i < ndv; ++i) {
+                const int32_t dv = vd.diagonal_vertices[i];
+                const double wt0 = dv < 0 ? 0.0 : vd.weights[dv >> 1];
+                memcpy(k1.data() + dw_off + 16 * i, &wt0, 8);
+                memcpy(k1.data() + dw_off + 16 * i + 8, &dv, 4);
+            }
+            const uint32_t w_off = (uint32_t)k1.size();
+            k1.resize(k1.size() + 8 * (size_t)vd.n_vertices);
+            memcpy(k1.data() + w_off, vd.weights, 8 * (size_t)vd.n_vertices);
+            const uint32_t up_off = (uint32_t)k1.size();
+            k1.resize(k1.size() + 2 * (size_t)vd.n_vertices);
+            for (int v = 0; v < vd.n_vertices; ++v) {
+                const uint16_t up = (uint16_t)(vd.leg_states[4 * v + 2] | vd.leg_states[4 * v + 3] << 8);
+                memcpy(k1.data() + up_off + 2 * v, &up, 2);
+            }
+            const uint32_t h[4] = {dw_off, w_off, up_off, (uint32_t)vd.n_vertices | ((uint32_t)vd.dims[0] << 16)};
+            memcpy(k1.data() + 16 * (size_t)g, h, 16);
+        }
+        k1.resize((k1.size() + 7) & ~(size_t)7);
+        k1_boff = (uint32_t)k1.size();
+        const size_t per = k1_groups == 1 ? 4 : 8;
+        k1.resize(k1.size() + per * m.n_bonds);
+        for (int bd = 0; bd < m.n_bonds; ++bd) {
+            const uint32_t rec[2] = {((uint32_t)m.bond_sites[2 * bd] & 0xFFFFu) | (uint32_t)m.bond_sites[2 * bd + 1] << 16,
+                                     16u * (uint32_t)k1group[m.bond_type[bd]]};
+            memcpy(k1.data() + k1_boff + per * bd, rec, per);
+        }
     }
     k1.resize((k1.size() + 15) & ~(size_t)15);
     size_t o_k1 = put(k1.data(), k1.size());
@@ -787,6 +823,8 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     dm.w_dim = wt.dim;
     dm.k1tab = (const uint8_t *)(d + o_k1);
     dm.k1tab_bytes = (int32_t)k1.size();
+    dm.k1tab_boff = (int32_t)k1_boff;
+    dm.k1tab_one = k1_groups == 1;
     dm.pad_k1 = 0;
     dm.k1ntab = (const uint8_t *)(d + o_kn);
     dm.k1ntab_bytes = (int32_t)kn.size();

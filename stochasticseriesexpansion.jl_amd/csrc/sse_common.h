@@ -67,12 +67,14 @@ struct DevModel {
     int32_t w_nent;            // exit entries: ((w_ncode << w_lg) + 1) * 2 * w_mw
     int32_t w_dim;             // local dimension of every site, 0 when they differ
     int32_t w_rank, pad_w;     // bytes of the threshold search image, 0 for up to 8 thresholds
-    // diagonal-update table, copied to LDS by K1 next to the bond records:
-    //   per type a 16-byte header {weights off, diag-vertex off, leg-state off,
-    //   nv | dims0 << 16}, then f64 weights[nv], i16 diagonal vertex codes
-    //   [dims0*dims1] (or -1), u8 leg states [nv][4]; offsets from the table start
+    // diagonal-update table, copied to LDS by K1: per group of bond types with
+    // equal tables a 16-byte header {diagonal off, weights off, upper-state off,
+    // nv | dims0 << 16}, then per group {f64 weight, i32 vertex code or -1, 0}
+    // [dims0*dims1], f64 weights[nv], u16 upper leg states [nv]; from k1tab_boff the
+    // bonds' sites (u16 each) and, with more than one group, the header's offset
+    // (u32); offsets from the table start
     const uint8_t *k1tab;
-    int32_t k1tab_bytes, pad_k1;
+    int32_t k1tab_bytes, k1tab_boff, k1tab_one, pad_k1;
     // lookups of the generic diagonal-update kernel, copied to LDS when they
     // fit (any bond size): per type a 32-byte header {weights off, diagonal-
     // vertex off, upper-states off, nv, dims packed one byte each}, then per

@@ -46,6 +46,15 @@ __device__ __forceinline__ uint64_t above_mask(int lane) { return lane >= 63 ? 0
 __device__ __forceinline__ int hi_bit(uint64_t x) { return 63 - __clzll((long long)x); }
 __device__ __forceinline__ int popc(uint64_t x) { return __popcll(x); }
 
+// Orders the LDS accesses of the lanes of a one-wave workgroup.  The LDS runs
+// a wave's instructions in order, so only code motion must be prevented; unlike
+// __syncthreads this does not wait for global loads still in flight.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Philox words of one walker staged in LDS: buf holds words
 // [bbase, bbase+256) and the next word to draw is bbase+off.  All members are
 // wave-uniform; every call must be made by the whole wave.
@@ -53,7 +62,7 @@ template <int NW>
 __device__ __noinline__ void wave_refill(uint64_t *buf, uint64_t key, uint64_t base)
 {
     const int l = threadIdx.x;
-    __syncthreads();
+    wave_lds_sync();
 #pragma unroll
     for (int j = l; j < NW / 2; j += 64) {
         uint32_t o0, o1, o2, o3;
@@ -61,7 +70,7 @@ __device__ __noinline__ void wave_refill(uint64_t *buf, uint64_t key, uint64_t b
         buf[2 * j] = (uint64_t)o0 | ((uint64_t)o1 << 32);
         buf[2 * j + 1] = (uint64_t)o2 | ((uint64_t)o3 << 32);
     }
-    __syncthreads();
+    wave_lds_sync();
 }
 
 template <int NW>
@@ -229,79 +238,109 @@ __device__ __forceinline__ uint64_t uni64(uint64_t x)
 
 // LDS layout of K1 (per workgroup = one walker):
 //   rbuf  u64[256]        Philox words
-//   tm0   u64[N]          per-site lane mask, bond position 0
-//   tm1   u64[N]          per-site lane mask, bond position 1
+//   tm    {u64, u64}[N]   per-site lane masks, bond positions 0 and 1
 //   cnt   u32[N]          operators on the site so far
-//   cups  u16[64]         upper-leg states of this chunk's operators
 //   sp    u8[N]           spins at the current slot
 __host__ __device__ inline size_t k1_lds_bytes(int N)
 {
-    size_t b = 2048 + 16 * (size_t)N + 4 * (size_t)N + 128 + (size_t)N;
+    size_t b = 2048 + 16 * (size_t)N + 4 * (size_t)N + (size_t)N;
     return (b + 15) & ~(size_t)15;
 }
 
 constexpr int K1_BLOCK = 16;  // 64-slot chunks per block of operator-string loads
 
-// Orders the LDS accesses of the lanes of a one-wave workgroup.  The LDS runs
-// a wave's instructions in order, so only code motion must be prevented; unlike
-// __syncthreads this does not wait for global loads still in flight.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// Model lookups of the diagonal update / vertex list: from the LDS copies of
-// the bond records and of DevModel::k1tab (K1Staged), or from global memory.
+// Model lookups of the diagonal update / vertex list: from the LDS copy of
+// DevModel::k1tab (K1Staged), or from the model's global arrays (K1Global).  A
+// type token comes with a bond: K1Staged's is the byte offset of the type's
+// header; with one table for all bonds (kOne: bond types with equal weights,
+// diagonal vertices and upper states share one) the header is in registers.
+struct K1Bond {
+    uint32_t s0, s1, t;
+};
+struct K1Weight {
+    double w;   // weight of the diagonal vertex, 0 without one
+    int32_t dv; // its vertex code, -1 without one
+};
 struct K1Global {
+    static constexpr bool kChecked = true;  // lookups need indexes in range
     const DevModel *m;
-    __device__ __forceinline__ void stage(const DevModel &) const {}
-    __device__ __forceinline__ int2 bond(uint32_t b) const { return m->bond_rec[b]; }
-    __device__ __forceinline__ int nv(int t) const { return m->types[t].nv; }
-    __device__ __forceinline__ int dims0(int t) const { return m->types[t].dims0; }
-    __device__ __forceinline__ int diag(int t, int i) const { return m->types[t].diag_vertex[i]; }
-    __device__ __forceinline__ double weight(int t, int v) const { return m->types[t].weights[v]; }
-    __device__ __forceinline__ uint32_t upper(int t, int v) const
+    __device__ __forceinline__ void stage(const DevModel &) {}
+    __device__ __forceinline__ K1Bond bond(uint32_t b) const
+    {
+        const int2 r = m->bond_rec[b];
+        return K1Bond{(uint32_t)r.x & 0xFFFFFu, (uint32_t)r.y, (uint32_t)r.x >> 20};
+    }
+    __device__ __forceinline__ uint32_t nv(uint32_t t) const { return (uint32_t)m->types[t].nv; }
+    __device__ __forceinline__ K1Weight diag(uint32_t t, uint32_t v0, uint32_t v1) const
+    {
+        const DevVD &vd = m->types[t];
+        const int32_t dv = vd.diag_vertex[(v0 - 1u) + (uint32_t)vd.dims0 * (v1 - 1u)];
+        return K1Weight{dv < 0 ? 0.0 : vd.weights[dv >> 1], dv};
+    }
+    __device__ __forceinline__ double weight(uint32_t t, uint32_t v) const { return m->types[t].weights[v]; }
+    __device__ __forceinline__ uint32_t upper(uint32_t t, uint32_t v) const
     {
         const uint8_t *ls = m->types[t].leg_states + 4 * v;
         return ls[2] | ((uint32_t)ls[3] << 8);
     }
 };
+template <bool kOne>
 struct K1Staged {
-    const int2 *br;
-    const uint8_t *kt;
-    // copy the bond records and the model's k1tab into LDS (whole wave)
-    __device__ __forceinline__ void stage(const DevModel &m) const
+    static constexpr bool kChecked = false;  // an index out of range reads another LDS word
+    uint32_t kt;                             // LDS byte address of the k1tab copy
+    uint32_t boff;                           // bond records in it
+    uint32_t h0, h1, h2, h3;                 // the only type's header (kOne)
+    // copy the model's k1tab into LDS (whole wave)
+    __device__ __forceinline__ void stage(const DevModel &m)
     {
-        int2 *b = (int2 *)br;
-        for (int i = threadIdx.x; i < m.n_bonds; i += 64)
-            b[i] = m.bond_rec[i];
-        uint32_t *k = (uint32_t *)kt;
+        worm_copy_table(kt, m.k1tab, (size_t)m.k1tab_bytes);
+        boff = (uint32_t)m.k1tab_boff;
         const uint32_t *g = (const uint32_t *)m.k1tab;
-        for (int i = threadIdx.x; i < m.k1tab_bytes / 4; i += 64)
-            k[i] = g[i];
+        h0 = uni(g[0]);
+        h1 = uni(g[1]);
+        h2 = uni(g[2]);
+        h3 = uni(g[3]);
     }
-    __device__ __forceinline__ int2 bond(uint32_t b) const { return br[b]; }
-    __device__ __forceinline__ uint4 hdr(int t) const { return ((const uint4 *)kt)[t]; }
-    __device__ __forceinline__ int nv(int t) const { return (int)(hdr(t).w & 0xFFFFu); }
-    __device__ __forceinline__ int dims0(int t) const { return (int)(hdr(t).w >> 16); }
-    __device__ __forceinline__ int diag(int t, int i) const { return ((const int16_t *)(kt + hdr(t).y))[i]; }
-    __device__ __forceinline__ double weight(int t, int v) const
+    __device__ __forceinline__ K1Bond bond(uint32_t b) const
     {
-        return ((const double *)(kt + hdr(t).x))[v];
+        if constexpr (kOne) {
+            const uint32_t s = *lds_at<lds_u32>(kt + boff + 4u * b);
+            return K1Bond{s & 0xFFFFu, s >> 16, 0u};
+        } else {
+            const uint64_t s = *lds_at<lds_u64>(kt + boff + 8u * b);
+            return K1Bond{(uint32_t)s & 0xFFFFu, (uint32_t)s >> 16, (uint32_t)(s >> 32)};
+        }
     }
-    __device__ __forceinline__ uint32_t upper(int t, int v) const
+    __device__ __forceinline__ u32x4 hdr(uint32_t t) const
     {
-        const uint8_t *ls = kt + hdr(t).z + 4 * v;
-        return ls[2] | ((uint32_t)ls[3] << 8);
+        if constexpr (kOne)
+            return u32x4{h0, h1, h2, h3};
+        else
+            return *lds_at<lds_u32x4>(kt + t);
+    }
+    __device__ __forceinline__ uint32_t nv(uint32_t t) const { return hdr(t).w & 0xFFFFu; }
+    __device__ __forceinline__ K1Weight diag(uint32_t t, uint32_t v0, uint32_t v1) const
+    {
+        const u32x4 h = hdr(t);
+        const uint32_t i = (v0 - 1u) + __umul24(h.w >> 16, v1 - 1u);
+        const u32x4 x = *lds_at<lds_u32x4>(kt + h.x + 16u * i);
+        return K1Weight{__hiloint2double((int)x.y, (int)x.x), (int32_t)x.z};
+    }
+    __device__ __forceinline__ double weight(uint32_t t, uint32_t v) const
+    {
+        const uint64_t x = *lds_at<lds_u64>(kt + hdr(t).y + 8u * v);
+        return __longlong_as_double((long long)x);
+    }
+    __device__ __forceinline__ uint32_t upper(uint32_t t, uint32_t v) const
+    {
+        return *lds_at<lds_u16>(kt + hdr(t).z + 2u * v);
     }
 };
 
-// LDS bytes of K1 with the model's lookups staged: the base layout, then the
-// bond records and the k1tab of the model
-__host__ __device__ inline size_t k1_lds_staged(int N, int n_bonds, int k1tab_bytes)
+// LDS bytes of K1 with the model's lookups staged behind the base layout
+__host__ __device__ inline size_t k1_lds_staged(int N, int k1tab_bytes)
 {
-    return k1_lds_bytes(N) + ((8 * (size_t)n_bonds + 15) & ~(size_t)15) + (size_t)k1tab_bytes;
+    return k1_lds_bytes(N) + (size_t)k1tab_bytes;
 }
 
 // Slot-by-slot processing of one chunk (reference order).  Used when a bond
@@ -388,9 +427,32 @@ __device__ __noinline__ K1SerialOut k1_serial_chunk_ool(DevWalker w, const DevMo
     return K1SerialOut{n, rs.bbase, rs.off};
 }
 
+// bits of a per-lane mask below this lane
+__device__ __forceinline__ uint32_t bits_below(uint64_t x)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(x >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)x, 0u));
+}
+// value of lane q's x (all lanes active)
+__device__ __forceinline__ uint32_t from_lane(uint32_t x, uint32_t q)
+{
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(q << 2), (int)x);
+}
+
 // phases: 1 diagonal update, 2 vertex list, 8 force the slot-by-slot path.
 // warm >= 0: init warm-up round (diagonal only; walkers with fewer warm-up
 // sweeps are skipped).
+//
+// A chunk of 64 slots is a chain of LDS lookups (words -> bond -> lane masks ->
+// states -> weight), a decision and the stores; with few walkers its latency
+// bounds the kernel, with many the instructions it issues.  So every lane runs
+// one path, whatever its slot holds, states of earlier operators come straight
+// from their lanes' registers, and the make test multiplies where the
+// reference divides: u < (pm / d) w is decided by u d against pm w unless the
+// two are within 2^-40 of each other, and then exactly, in slot order.
+// Measured on 16x16 Heisenberg at beta = 8 (137 chunks), one wave to a SIMD:
+// 300 -> 199 us per sweep against divides, branches by slot kind and a table
+// per lookup; 383 -> 265 us with 1536 walkers.  Blocks of 8 chunks at three waves
+// per SIMD (168 registers) against 16 at two (193): 194 and 268 us, no gain.
 template <class Tab>
 __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models, DevPool *pool, int wi,
                                             int phases, int warm, char *lds, Tab tab, int grp)
@@ -407,21 +469,17 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
     tab.stage(m);
     const int N = m.n_sites;
     uint64_t *rbuf = (uint64_t *)lds;
-    uint64_t *tm0 = (uint64_t *)(lds + 2048);
-    uint64_t *tm1 = tm0 + N;
-    uint32_t *cnt = (uint32_t *)(tm1 + N);
-    uint16_t *cups = (uint16_t *)(cnt + N);
-    uint8_t *sp = (uint8_t *)(cups + 64);
-    uint32_t *tm0w = (uint32_t *)tm0;
-    uint32_t *tm1w = (uint32_t *)tm1;
+    uint32_t *cnt = (uint32_t *)(lds + 2048 + 16 * (size_t)N);
+    uint8_t *sp = (uint8_t *)(cnt + N);
+    const uint32_t lbase = (uint32_t)(uintptr_t)(lds_u8 *)lds;
+    const uint32_t tmb = lbase + 2048u, cntb = tmb + 16u * (uint32_t)N, spb = cntb + 4u * (uint32_t)N;
 
     const bool do_diag = phases & 1;
     const bool do_vl = (phases & 2) && warm < 0;
     const bool force_serial = phases & 8;
 
     for (int i = lane; i < N; i += 64) {
-        tm0[i] = 0ull;
-        tm1[i] = 0ull;
+        *lds_at<lds_u32x4>(tmb + 16u * i) = u32x4{0u, 0u, 0u, 0u};
         cnt[i] = 0u;
         sp[i] = w.spins[i];
     }
@@ -459,10 +517,8 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
     rs.init(rbuf, w.key, w.ctr);
     const double pm_raw = (double)m.n_bonds / w.T;
     const double pr_raw = w.T / (double)m.n_bonds;
-    const uint64_t Nb = (uint64_t)m.n_bonds;
-    const int64_t L = w.L;
-    int64_t n0 = w.n;
-    const uint64_t below = below_mask(lane), above = above_mask(lane);
+    const uint32_t L = (uint32_t)w.L;
+    uint32_t n0 = uni((uint32_t)w.n);
     gmem<uint64_t> *gidx = as_global((uint64_t *)w.links);  // both sites' idx words of a slot
     gmem<uint32_t> *ops = as_global(w.ops);
 
@@ -476,174 +532,144 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
     // The chunk index within the block is wave-uniform, so cur[slot] is a
     // register-indexed move.  Model scalars are read once, before the loop,
     // for the same reason (a read inside it would wait for the stores).
-    const uint32_t nbonds = (uint32_t)m.n_bonds;
+    const uint32_t nbonds = uni((uint32_t)m.n_bonds);
     uint32_t cur[K1_BLOCK], pf[K1_BLOCK];
 #pragma unroll
     for (int u = 0; u < K1_BLOCK; ++u) {
-        const int64_t q = 64 * u + lane;
+        const uint32_t q = 64u * u + lane;
         cur[u] = q < L ? ops[q] : 0u;
     }
 #pragma unroll
     for (int u = 0; u < K1_BLOCK; ++u) {
-        const int64_t q = 64 * (K1_BLOCK + u) + lane;
+        const uint32_t q = 64u * (K1_BLOCK + u) + lane;
         pf[u] = q < L ? ops[q] : 0u;
     }
-    for (int64_t base = 0; base < L; base += 64) {
-        const int64_t p = base + lane;
+    bool bad = false;
+    for (uint32_t base = 0; base < L; base += 64) {
+        const uint32_t p = base + lane;
         const bool valid = p < L;
-        const int64_t chunk = base >> 6;
-        const int slot = (int)uni((uint32_t)(chunk % K1_BLOCK));
+        const uint32_t chunk = base >> 6;
+        const int slot = (int)uni(chunk % K1_BLOCK);
         if (slot == 0 && chunk > 0) {
 #pragma unroll
             for (int u = 0; u < K1_BLOCK; ++u)
                 cur[u] = pf[u];
 #pragma unroll
             for (int u = 0; u < K1_BLOCK; ++u) {
-                const int64_t q = base + 64 * (K1_BLOCK + u) + lane;
+                const uint32_t q = base + 64u * (K1_BLOCK + u) + lane;
                 pf[u] = q < L ? ops[q] : 0u;
             }
         }
         const uint32_t op = cur[slot];
         const uint32_t vc = op_vcode(op);
         const bool ident = valid && op == 0u;
-        const bool isop = valid && op != 0u;
-        const bool dia = isop && (vc & 1u);
-        const bool offd = isop && !(vc & 1u);
+        const bool dia = op != 0u && (vc & 1u);
+        const bool offd = op != 0u && !(vc & 1u);
         const uint64_t identm = __ballot(ident), diam = __ballot(dia), offm = __ballot(offd);
         uint32_t b = op_bond(op);
+        // an operator outside the model (a corrupted string): reported when the
+        // walker ends, its bond replaced by one that exists
+        bad |= b >= nbonds;
+        b = b < nbonds ? b : 0u;
         double u = 0.0;
-        {
-            bool bad = false;
-            if (isop) {
-                bad = b >= nbonds;
-                if (!bad)
-                    bad = (int)(vc >> 1) >= tab.nv(tab.bond(b).x >> 20);
-            }
-            if (__ballot(bad)) {
-                if (lane == 0) {
-                    W[wi].error = SSE_ERR_STATE;
-                    flag_error(pool, SSE_ERR_STATE);
-                }
-                return;
-            }
-        }
-
         if (do_diag) {
-            const int D = 2 * popc(identm) + popc(diam);
-            const int off = 2 * popc(identm & below) + popc(diam & below);
-            bool reject = force_serial;
-            if (D > 0) {
-                rs.ensure((uint32_t)D);
-                if (ident) {
-                    uint64_t x = rs.peek((uint32_t)off);
-                    uint64_t lo = x * Nb;
-                    b = (uint32_t)__umul64hi(x, Nb);
-                    if (lo < Nb && lo < (0ull - Nb) % Nb)
-                        reject = true;
-                    u = word_to_float(rs.peek((uint32_t)off + 1));
-                } else if (dia) {
-                    u = word_to_float(rs.peek((uint32_t)off));
-                }
-            }
-            if (__ballot(reject)) {
+            // draws of the slots before this one: two per identity, one per
+            // diagonal operator
+            const uint32_t D = 2u * (uint32_t)popc(identm) + (uint32_t)popc(diam);
+            const uint32_t off = 2u * bits_below(identm) + bits_below(diam);
+            if (D > 0u)
+                rs.ensure(D);
+            // identity: bond, then the test's number; diagonal: the number
+            const uint64_t x0 = rs.peek(D ? off : 0u), x1 = rs.peek(D ? off + 1u : 0u);
+            // rand(1:n_bonds): high half of word * n_bonds, rejected where the low
+            // half could be below 2^64 mod n_bonds
+            const uint64_t pl = (uint64_t)(uint32_t)x0 * nbonds;
+            const uint64_t ph = (uint64_t)(uint32_t)(x0 >> 32) * nbonds + (pl >> 32);
+            const bool maybe = ident && (uint32_t)ph == 0u && (uint32_t)pl < nbonds;
+            if (__builtin_expect(force_serial || wave_any(maybe), 0)) {
                 const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, pm_raw, pr_raw, do_diag,
                                                            do_vl, sp, cnt);
-                n0 = so.n;
+                n0 = uni((uint32_t)so.n);
                 rs.bbase = so.bbase;
                 rs.off = so.off;
                 continue;
             }
-            rs.advance((uint32_t)D);
+            b = ident ? (uint32_t)(ph >> 32) : b;
+            u = word_to_float(ident ? x1 : x0);
+            rs.advance(D);
         } else if (force_serial) {
             const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, pm_raw, pr_raw, do_diag,
                                                        do_vl, sp, cnt);
-            n0 = so.n;
+            n0 = uni((uint32_t)so.n);
             rs.bbase = so.bbase;
             rs.off = so.off;
             continue;
         }
 
-        const bool has = isop || (ident && do_diag);
-        int s0 = 0, s1 = 0, type = 0;
+        const K1Bond br = tab.bond(b);
+        const uint32_t s0 = br.s0, s1 = br.s1;
+        const uint32_t vx = vc >> 1;
+        uint32_t vi = vx;
+        if (Tab::kChecked) {
+            const uint32_t nv = tab.nv(br.t);
+            bad |= op != 0u && vx >= nv;
+            vi = vx < nv ? vx : 0u;
+        } else {
+            bad |= op != 0u && vx >= tab.nv(br.t);
+        }
+        // per-site lane masks of the slots that hold or may get an operator
+        const bool has = op != 0u || (ident && do_diag);
+        const uint32_t t0 = tmb + 16u * s0, t1 = tmb + 16u * s1;
         if (has) {
-            int2 br = tab.bond(b);
-            s0 = br.x & 0xFFFFF;
-            s1 = br.y;
-            type = br.x >> 20;
+            const uint32_t half = (lane >> 5) * 4u, bit = 1u << (lane & 31);
+            atomicOr((uint32_t *)(lds + (t0 - lbase) + half), bit);
+            atomicOr((uint32_t *)(lds + (t1 - lbase) + 8u + half), bit);
         }
-        // per-site lane masks
-        if (has) {
-            atomicOr(&tm0w[2 * s0 + (lane >> 5)], 1u << (lane & 31));
-            atomicOr(&tm1w[2 * s1 + (lane >> 5)], 1u << (lane & 31));
-        }
-        if (offd) {
-            cups[lane] = (uint16_t)tab.upper(type, vc >> 1);
-        }
+        const uint32_t up = tab.upper(br.t, vi);      // an off-diagonal operator's states after it
+        double wgt = tab.weight(br.t, vi);            // a diagonal operator's weight
+        const uint32_t sp0 = *lds_at<lds_u8>(spb + s0), sp1 = *lds_at<lds_u8>(spb + s1);
+        const uint32_t c0 = *lds_at<lds_u32>(cntb + 4u * s0), c1 = *lds_at<lds_u32>(cntb + 4u * s1);
         wave_lds_sync();
-        uint64_t a0 = 0, a1 = 0, c0 = 0, c1 = 0;  // site0: pos-0/pos-1 masks; site1: same
-        if (has) {
-            a0 = tm0[s0];
-            a1 = tm1[s0];
-            c0 = tm0[s1];
-            c1 = tm1[s1];
-        }
+        const u32x4 ma = *lds_at<lds_u32x4>(t0), mc = *lds_at<lds_u32x4>(t1);
+        const uint64_t a0 = (uint64_t)ma.x | (uint64_t)ma.y << 32, a1 = (uint64_t)ma.z | (uint64_t)ma.w << 32;
+        const uint64_t e0 = (uint64_t)mc.x | (uint64_t)mc.y << 32, e1 = (uint64_t)mc.z | (uint64_t)mc.w << 32;
+        const uint64_t A = a0 | a1, C = e0 | e1;  // lanes on site 0, on site 1
+        const uint64_t below = below_mask(lane), above = above_mask(lane);
 
         uint64_t plus = 0, minus = 0;
         uint32_t fop = op;
         if (do_diag) {
-            double wgt = 0.0;
-            int32_t dv = -1;
-            if (ident) {
-                int v0, v1;
-                uint64_t cand = (a0 | a1) & offm & below;
-                if (cand) {
-                    int q = hi_bit(cand);
-                    v0 = (cups[q] >> (((a0 >> q) & 1ull) ? 0 : 8)) & 255;
-                } else {
-                    v0 = sp[s0];
-                }
-                cand = (c0 | c1) & offm & below;
-                if (cand) {
-                    int q = hi_bit(cand);
-                    v1 = (cups[q] >> (((c0 >> q) & 1ull) ? 0 : 8)) & 255;
-                } else {
-                    v1 = sp[s1];
-                }
-                dv = tab.diag(type, (v0 - 1) + tab.dims0(type) * (v1 - 1));
-                wgt = dv < 0 ? 0.0 : tab.weight(type, dv >> 1);
-            } else if (dia) {
-                wgt = tab.weight(type, vc >> 1);
-            }
-            bool amb = false, dec = false;
-            if (ident) {
-                int64_t lo = n0 - lane < 0 ? 0 : n0 - lane;
-                int64_t hi = n0 + lane > L - 1 ? L - 1 : n0 + lane;
-                bool d_lo = u < (pm_raw / (double)(L - lo)) * wgt;
-                bool d_hi = u < (pm_raw / (double)(L - hi)) * wgt;
-                amb = d_lo != d_hi;
-                dec = d_lo;
-            } else if (dia) {
-                int64_t lo = n0 - lane < 1 ? 1 : n0 - lane;
-                int64_t hi = n0 + lane > L ? L : n0 + lane;
-                double uw = u * wgt;
-                bool d_lo = uw < (double)(L - lo + 1) * pr_raw;
-                bool d_hi = uw < (double)(L - hi + 1) * pr_raw;
-                amb = d_lo != d_hi;
-                dec = d_lo;
-            }
-            plus = __ballot(ident && !amb && dec);
-            minus = __ballot(dia && !amb && dec);
-            uint64_t ambm = __ballot(amb);
+            // states at the slot: of the latest off-diagonal operator on the
+            // site earlier in the chunk, else at the chunk's start
+            const uint64_t oa = A & offm & below, oc = C & offm & below;
+            const uint32_t qa = oa ? (uint32_t)hi_bit(oa) : 0u, qc = oc ? (uint32_t)hi_bit(oc) : 0u;
+            const uint32_t ua = from_lane(up, qa), uc = from_lane(up, qc);
+            const uint32_t v0 = oa ? (((a0 >> qa) & 1ull) ? ua & 255u : ua >> 8) : sp0;
+            const uint32_t v1 = oc ? (((e0 >> qc) & 1ull) ? uc & 255u : uc >> 8) : sp1;
+            const K1Weight dw = tab.diag(br.t, v0, v1);
+            wgt = ident ? dw.w : wgt;
+            // the window of n that earlier slots of the chunk leave open; each
+            // test is monotone in n, so a decision at both ends holds between
+            const uint32_t room = L - n0 + (ident ? 0u : 1u);
+            const uint32_t dl = room + (uint32_t)lane < L ? room + (uint32_t)lane : L;
+            const uint32_t dh = room > (uint32_t)lane ? room - (uint32_t)lane : 1u;
+            const double fl = (double)dl, fh = (double)dh;
+            const double pmw = pm_raw * wgt, uw = u * wgt;
+            const bool yes = ident ? (u * fl) * (1.0 + 0x1p-40) < pmw : uw < fh * pr_raw;
+            const bool no = ident ? (u * fh) * (1.0 - 0x1p-40) > pmw : !(uw < fl * pr_raw);
+            plus = __ballot(ident && yes);
+            minus = __ballot(dia && yes);
+            uint64_t ambm = __ballot((ident || dia) && !yes && !no);
             while (ambm) {
                 const int a = __ffsll((long long)ambm) - 1;
                 const uint64_t ba = below_mask(a);
-                const int64_t na = n0 + popc(plus & ba) - popc(minus & ba);
+                const int64_t na = (int64_t)n0 + popc(plus & ba) - popc(minus & ba);
                 bool d = false;
                 if (lane == a) {
                     if (ident)
-                        d = u < (pm_raw / (double)(L - na)) * wgt;
+                        d = u < (pm_raw / (double)((int64_t)L - na)) * wgt;
                     else
-                        d = u * wgt < (double)(L - na + 1) * pr_raw;
+                        d = u * wgt < (double)((int64_t)L - na + 1) * pr_raw;
                 }
                 const uint64_t dm = __ballot(d);
                 if ((identm >> a) & 1ull)
@@ -652,48 +678,43 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
                     minus |= dm;
                 ambm &= ambm - 1;
             }
-            n0 += popc(plus) - popc(minus);
+            n0 += (uint32_t)popc(plus) - (uint32_t)popc(minus);
             if (ident && ((plus >> lane) & 1ull))
-                fop = op_make(b, (uint32_t)dv);
+                fop = op_make(b, (uint32_t)dw.dv);
             if (dia && ((minus >> lane) & 1ull))
                 fop = 0u;
-            if (valid && fop != op)
+            if (fop != op)
                 ops[p] = fop;
         }
 
         // vertex list over the chunk's final non-identity operators: how many
         // earlier operators act on each of the operator's sites
         const uint64_t NI = do_diag ? ((identm & plus) | (diam & ~minus) | offm) : (diam | offm);
-        const bool isni = do_vl && ((NI >> lane) & 1ull);
-        uint32_t i0 = 0, i1 = 0;
-        bool last0 = false, last1 = false;
-        if (isni) {
-            const uint64_t m0 = (a0 | a1) & NI, m1 = (c0 | c1) & NI;
-            i0 = cnt[s0] + (uint32_t)popc(m0 & below);
-            i1 = cnt[s1] + (uint32_t)popc(m1 & below);
-            last0 = (m0 & above) == 0ull;
-            last1 = (m1 & above) == 0ull;
-        }
-        wave_lds_sync();
-        if (isni) {
+        if (do_vl && ((NI >> lane) & 1ull)) {
+            const uint32_t i0 = c0 + bits_below(A & NI), i1 = c1 + bits_below(C & NI);
             gidx[p] = (uint64_t)i0 | (uint64_t)i1 << 32;
-            if (last0)
-                cnt[s0] = i0 + 1u;
-            if (last1)
-                cnt[s1] = i1 + 1u;
+            atomicAdd(cnt + s0, 1u);
+            atomicAdd(cnt + s1, 1u);
         }
         // spins after the chunk: the last off-diagonal operator on a site wins
         if (do_diag && offd) {
-            if ((((a0 | a1) & offm) & above) == 0ull)
-                sp[s0] = (uint8_t)(cups[lane] & 255);
-            if ((((c0 | c1) & offm) & above) == 0ull)
-                sp[s1] = (uint8_t)(cups[lane] >> 8);
+            if (((A & offm) & above) == 0ull)
+                *lds_at<lds_u8>(spb + s0) = (uint8_t)(up & 255u);
+            if (((C & offm) & above) == 0ull)
+                *lds_at<lds_u8>(spb + s1) = (uint8_t)(up >> 8);
         }
         if (has) {
-            tm0[s0] = 0ull;
-            tm1[s1] = 0ull;
+            *lds_at<lds_u64>(t0) = 0ull;
+            *lds_at<lds_u64>(t1 + 8u) = 0ull;
         }
         wave_lds_sync();
+    }
+    if (wave_any(bad)) {
+        if (lane == 0) {
+            W[wi].error = SSE_ERR_STATE;
+            flag_error(pool, SSE_ERR_STATE);
+        }
+        return;
     }
 
     if (do_vl) {
@@ -724,13 +745,14 @@ __device__ __forceinline__ void k1_walker(DevWalker *W, const DevModel *models, 
 {
     const DevModel &m = models[W[wi].model];
     const size_t base = k1_lds_bytes(m.n_sites);
-    if (k1_lds_staged(m.n_sites, m.n_bonds, m.k1tab_bytes) <= (size_t)lds_bytes) {
-        K1Staged tab{(const int2 *)(lds + base),
-                     (const uint8_t *)(lds + base + ((8 * (size_t)m.n_bonds + 15) & ~(size_t)15))};
-        k1_walker_t(W, models, pool, wi, phases, warm, lds, tab, grp);
+    if (k1_lds_staged(m.n_sites, m.k1tab_bytes) <= (size_t)lds_bytes) {
+        const uint32_t kt = (uint32_t)(uintptr_t)(lds_u8 *)lds + (uint32_t)base;
+        if (m.k1tab_one)
+            k1_walker_t(W, models, pool, wi, phases, warm, lds, K1Staged<true>{kt, 0, 0, 0, 0, 0}, grp);
+        else
+            k1_walker_t(W, models, pool, wi, phases, warm, lds, K1Staged<false>{kt, 0, 0, 0, 0, 0}, grp);
     } else {
-        K1Global tab{&m};
-        k1_walker_t(W, models, pool, wi, phases, warm, lds, tab, grp);
+        k1_walker_t(W, models, pool, wi, phases, warm, lds, K1Global{&m}, grp);
     }
 }
 
@@ -1179,7 +1201,7 @@ static inline int wave_configure(WaveConfig &c, const std::vector<DevModel> &mod
     // stage each model's lookups in LDS if that keeps K1 within 32 KiB (high
     // occupancy matters more than the lookups of larger models)
     for (const DevModel &m : models) {
-        const size_t st = (k1_lds_staged(m.n_sites, m.n_bonds, m.k1tab_bytes) + 15) & ~(size_t)15;
+        const size_t st = (k1_lds_staged(m.n_sites, m.k1tab_bytes) + 15) & ~(size_t)15;
         if (st <= 32768 && st > c.lds_k1)
             c.lds_k1 = st;
     }

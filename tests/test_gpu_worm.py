@@ -1,9 +1,11 @@
-"""The worm update's record layouts and exit tables, each against the oracle.
+"""The worm update's record layouts and exit tables, and the diagonal update's
+lookups, each against the oracle.
 
 Bit-exact after every sweep (whole numbers, and the worm controller's FP64
 bits): the layouts hold the same operators, so nothing may differ.  T = 8 leaves
 sites with one operator or none (guards next to each other), T = 0.15 gives
 chains of many 64-word buffers and worms that cross the periodic closure."""
+import numpy as np
 import pytest
 
 from fixtures import (field_spins, job_bilayer, job_honeycomb, ladder_dimer, plaquette_ring,
@@ -48,4 +50,43 @@ def test_worm_layouts(sse_pkg, oracle_mod, kind, records, k2_lds):
         for o in oracles:
             o.sweep(1)
         _compare(batch, oracles, f"{kind} sweep {s}")
+    batch.close()
+
+
+@pytest.mark.parametrize("kind,size,T,cutoff", [
+    ("square", 4, 0.3, 63), ("square", 4, 0.3, 64), ("square", 4, 0.3, 65),  # one table; ragged chunks
+    ("square", 4, 0.05, 0),      # grown from nothing; over 64 draws of a chunk, chunks of one site's bonds
+    ("ladder", 8, 0.1, 0),       # a table per bond type
+    ("bilayer", 0, 0.1, 1000),   # vertices without a diagonal partner
+    ("square", 40, 1.5, 0),      # lookups past the staging limit: read from global memory
+])
+def test_diagonal_update(sse_pkg, oracle_mod, kind, size, T, cutoff):
+    """Diagonal update and vertex list alone, both as chunks and slot by slot
+    (8): strings, draws and lists equal the oracle's after each."""
+    model = {"square": lambda: square_heisenberg(sse_pkg, size, d=-0.3, hz=0.1),
+             "ladder": lambda: ladder_dimer(sse_pkg, size, 0.6),
+             "bilayer": lambda: job_bilayer(sse_pkg, T)}[kind]()
+    flat = model.flat()
+    walkers = [sse_pkg.walker_desc(T=T * f, seed=90 + k, init_opstring_cutoff=cutoff)
+               for k, f in enumerate((1.0, 4.0))]
+    _say(f"diagonal update: {kind} {size} T={T} cutoff={cutoff}")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    oracles = [oracle_mod.OracleWalker(sse_pkg.capi, flat, w) for w in walkers]
+    batch.init()
+    for o in oracles:
+        o.init()
+    for s in range(10):
+        batch.sweep_phases(3 if s % 4 else 11)
+        for k, o in enumerate(oracles):
+            assert o.sweep_phases(3) == 0
+            gs, gops, gspins = batch.get_walker(k)
+            os_, oops, ospins = o.state()
+            assert gs["rng_counter"] == os_["rng_counter"]
+            assert np.array_equal(gops, oops) and np.array_equal(gspins, ospins)
+            for got, want in zip(batch.vertex_list(k), o.vertex_list()):
+                assert np.array_equal(got, want)
+        batch.sweep(1)
+        for o in oracles:
+            o.sweep(1)
+        _compare(batch, oracles, f"sweep {s}")
     batch.close()
