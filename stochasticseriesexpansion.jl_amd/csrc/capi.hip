@@ -47,7 +47,7 @@ int fail(int code, const std::string &msg)
 // while every field is unchanged.  Compared bytewise (constructed zeroed).
 struct GraphKey {
     int32_t kind;       // 1 one stream, 2 stream groups, 3 persistent launch
-    int32_t sweeps, measure, groups, rec_mode, chase, use_order, n_tasks, fuse, lane_width, generic;
+    int32_t sweeps, measure, groups, rec_mode, chase, use_order, n_tasks, segments, fuse, lane_width, generic;
     size_t lds[9];      // worm-kernel LDS (one stream / per group), persistent LDS
     const void *models, *budgets, *order;
     GraphKey() { memset(this, 0, sizeof *this); }
@@ -1110,7 +1110,7 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
     if (!rc)
         rc = dev_alloc(b, &b->d_walkers, (size_t)n_walkers);
     if (!rc)
-        rc = dev_alloc(b, &b->d_queue, 1);
+        rc = dev_alloc(b, &b->d_queue, (size_t)n_walkers + 1);
     if (!rc)
         rc = dev_alloc(b, &b->d_work, 1);
     if (!rc)
@@ -1593,22 +1593,25 @@ static int groups_graph_many(sse_batch *b, int n_sweeps, int measure)
     return done < n_sweeps ? groups_run(b, n_sweeps - done, measure) : SSE_OK;
 }
 
-// The persistent work-queue launch: n_tasks tasks in the order `order`,
-// budgets per walker or n_sweeps each (sse_persist.h), captured as a graph
-// when graphs are on.
-static int persist_issue(sse_batch *b, int n_sweeps, int measure, const int32_t *budgets,
+// The persistent work-queue launch: n_tasks walkers in the order `order`,
+// budgets per walker (the largest is most) or n_sweeps each (sse_persist.h),
+// captured as a graph when graphs are on.
+static int persist_issue(sse_batch *b, int n_sweeps, int measure, const int32_t *budgets, int64_t most,
                          int n_tasks, const int32_t *order)
 {
+    const int segments = persist_segments(b->wave, n_tasks, budgets ? most : n_sweeps, b->n_cu);
     auto issue = [&]() {
         int rc = wave_launch_persist(b->wave, b->stream, b->d_walkers, b->d_models, b->d_pool, b->d_out,
                                      b->d_sum, b->d_sumsq, b->d_count, b->d_wlf, b->d_done, order,
-                                     n_tasks, budgets, n_sweeps, measure, b->d_queue, b->n_cu);
+                                     n_tasks, budgets, n_sweeps, segments, measure, b->d_queue,
+                                     b->n_walkers + 1, b->n_cu);
         return rc ? fail(rc, "persistent launch failed") : SSE_OK;
     };
     if (!b->use_graph)
         return issue();
     GraphKey k = graph_key(b, 3, n_sweeps, measure);
     k.n_tasks = n_tasks;
+    k.segments = segments;
     k.budgets = budgets;
     k.order = order;
     k.lds[0] = persist_lds_bytes(b->wave);
@@ -1678,7 +1681,7 @@ static int issue_sweeps(sse_batch *b, int n_sweeps, int measure, bool grouped, b
 {
     if (b->mode == SSE_MODE_WAVE && b->persistent) {
         if (!b->kernel_timing)
-            return persist_issue(b, n_sweeps, measure, nullptr, b->n_walkers,
+            return persist_issue(b, n_sweeps, measure, nullptr, n_sweeps, b->n_walkers,
                                  b->use_order ? b->d_order : nullptr);
         const size_t ev0 = b->kern_ev.size() * 4;
         int rc = ensure_kernel_events(b, ev0 + 4);
@@ -1689,7 +1692,7 @@ static int issue_sweeps(sse_batch *b, int n_sweeps, int measure, bool grouped, b
         HIPCHECK(hipEventRecord(e[0], b->stream));
         const bool graph = b->use_graph;
         b->use_graph = false;
-        rc = persist_issue(b, n_sweeps, measure, nullptr, b->n_walkers,
+        rc = persist_issue(b, n_sweeps, measure, nullptr, n_sweeps, b->n_walkers,
                            b->use_order ? b->d_order : nullptr);
         b->use_graph = graph;
         HIPCHECK(hipEventRecord(e[1], b->stream));
@@ -2194,7 +2197,7 @@ int sse_run_budgets(sse_batch *b, const int64_t *sweeps, int32_t measure)
             b->use_graph = false;
             HIPCHECK(hipEventRecord(e[0], b->stream));
         }
-        rc = persist_issue(b, 0, measure ? 1 : 0, b->d_budget, (int)order.size(), b->d_task_order);
+        rc = persist_issue(b, 0, measure ? 1 : 0, b->d_budget, most, (int)order.size(), b->d_task_order);
         b->use_graph = graph_k;
         if (rc)
             return rc;
@@ -2233,10 +2236,11 @@ int sse_run_budgets(sse_batch *b, const int64_t *sweeps, int32_t measure)
 
 // ---------------------------------------------------------------- no-alloc
 // Device scratch of sse_run_budgets_noalloc, one copy per GPU for the life of
-// the process: [0, 256) the task counter, then the caller's budgets as int64
-// [SSE_NOALLOC_MAX_WALKERS], then the same narrowed to int32.  Host code uses
-// only the per-device address from hipGetSymbolAddress, never the name.
-constexpr size_t kNoAllocBudget64 = 256;
+// the process: the work queue (task counter, sweeps due per walker), then the
+// caller's budgets as int64 [SSE_NOALLOC_MAX_WALKERS], then the same narrowed to
+// int32.  Host code uses only the per-device address from hipGetSymbolAddress,
+// never the name.
+constexpr size_t kNoAllocBudget64 = 256 + 4 * (size_t)SSE_NOALLOC_MAX_WALKERS;
 constexpr size_t kNoAllocBudget32 = kNoAllocBudget64 + 8 * (size_t)SSE_NOALLOC_MAX_WALKERS;
 constexpr size_t kNoAllocBytes = kNoAllocBudget32 + 4 * (size_t)SSE_NOALLOC_MAX_WALKERS;
 static __device__ __align__(256) char scratch[kNoAllocBytes];
@@ -2290,9 +2294,12 @@ int sse_run_budgets_noalloc(sse_batch *b, const int64_t *sweeps, int32_t measure
         return fail(SSE_ERR_INVALID, "sse_run_budgets_noalloc: walkers of a temperature ladder "
                                      "advance together (sse_run)");
     const int n = b->n_walkers;
-    for (int w = 0; w < n; ++w)
+    int64_t most = 0;
+    for (int w = 0; w < n; ++w) {
         if (sweeps[w] < 0 || sweeps[w] > INT32_MAX)
             return fail(SSE_ERR_INVALID, "sse_run_budgets_noalloc: sweep counts must be in 0..2^31-1");
+        most = std::max(most, sweeps[w]);
+    }
     char *sc = noalloc_scratch(b->device);
     if (!sc)
         return fail(SSE_ERR_HIP, "sse_run_budgets_noalloc: no address for the device scratch");
@@ -2312,8 +2319,9 @@ int sse_run_budgets_noalloc(sse_batch *b, const int64_t *sweeps, int32_t measure
     // by the launch's reset kernel.
     int rc = wave_launch_persist(b->wave, b->stream, b->d_walkers, b->d_models, b->d_pool, b->d_out,
                                  b->d_sum, b->d_sumsq, b->d_count, b->d_wlf, b->d_done,
-                                 b->use_order ? b->d_order : nullptr, n, bud32, 0, measure ? 1 : 0,
-                                 (int32_t *)sc, b->n_cu);
+                                 b->use_order ? b->d_order : nullptr, n, bud32, 0,
+                                 persist_segments(b->wave, n, most, b->n_cu), measure ? 1 : 0,
+                                 (int32_t *)sc, n + 1, b->n_cu);
     if (rc)
         return fail(rc, "persistent launch failed");
     if (!measure && b->any_budget) {

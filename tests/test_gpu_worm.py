@@ -1,5 +1,6 @@
 """The worm update's record layouts and exit tables, and the diagonal update's
-lookups, each against the oracle.
+lookups, each against the oracle; and the work-queue launch with more walkers
+than it has workgroups.
 
 Bit-exact after every sweep (whole numbers, and the worm controller's FP64
 bits): the layouts hold the same operators, so nothing may differ.  T = 8 leaves
@@ -89,4 +90,54 @@ def test_diagonal_update(sse_pkg, oracle_mod, kind, size, T, cutoff):
         for o in oracles:
             o.sweep(1)
         _compare(batch, oracles, f"sweep {s}")
+    batch.close()
+
+
+@pytest.mark.parametrize("call", ["run", "budgets", "noalloc"])
+def test_work_queue_hands_walkers_over(sse_pkg, oracle_mod, call):
+    """2600 walkers, more than the card holds workgroups (at most 8 to each of
+    256 compute units), so a walker's sweeps pass between workgroups: all equal
+    the one-stream launches, some the oracle.  Budgets of 0, 1, the segment
+    count 16, one past it and 33."""
+    n, T = 2600, 0.7
+    flat = square_heisenberg(sse_pkg, 4, d=-0.3, hz=0.1).flat()
+    walkers = [sse_pkg.walker_desc(T=T, seed=300 + k, thermalization=2) for k in range(n)]
+    budgets = np.full(n, 5, dtype=np.int64)
+    if call != "run":
+        budgets = np.array([0, 1, 16, 17, 33, 2], dtype=np.int64)[np.arange(n) % 6]
+    _say(f"work queue: {n} walkers, {call}")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    batch.set_option(sse_pkg.capi.SSE_OPT_PERSISTENT, 1)
+    batch.init()
+    for rep in range(2):
+        if call == "run":
+            batch.run(5, measure=True)
+        elif call == "budgets":
+            batch.run_budgets(budgets, measure=True)
+        else:
+            batch.run_budgets_noalloc(budgets, measure=True)
+    sums, sumsq, counts = batch.accumulators_raw()
+    assert np.array_equal(counts, np.maximum(2 * budgets - 2, 0))
+    for k in list(range(6)) + [1300, n - 1]:
+        o = oracle_mod.OracleWalker(sse_pkg.capi, flat, walkers[k])
+        o.init()
+        o.sweep(int(2 * budgets[k]))
+        gs, gops, gspins = batch.get_walker(k)
+        os_, oops, ospins = o.state()
+        assert np.array_equal(gops, oops) and np.array_equal(gspins, ospins)
+        for key in ("cutoff", "num_operators", "num_worms", "rng_counter", "sweeps"):
+            assert gs[key] == os_[key], key
+    one = sse_pkg.Batch([flat], walkers, mode=0)
+    one.set_option(sse_pkg.capi.SSE_OPT_STREAMS, 1)
+    one.init()
+    for s in range(int(2 * budgets.max())):
+        one.run(1, measure=True)
+        for k in np.nonzero(2 * budgets == s + 1)[0]:
+            a, b = batch.get_walker(int(k)), one.get_walker(int(k))
+            assert a[0]["rng_counter"] == b[0]["rng_counter"] and np.array_equal(a[1], b[1])
+            assert np.array_equal(a[2], b[2])
+    if call == "run":
+        for a, b in zip((sums, sumsq, counts), one.accumulators_raw()):
+            assert np.array_equal(a, b)
+    one.close()
     batch.close()
