@@ -67,8 +67,8 @@ enum sse_status {
  * kernel families take any n_sites.  In wave mode a batch whose models all
  * have two-site bonds runs the two-site kernels (and the work-queue
  * launch); a batch with any other model runs every
- * walker through the generic wave kernels, which have no work-queue launch
- * (SSE_OPT_PERSISTENT and sse_run_budgets_noalloc are refused;
+ * walker through the generic wave kernels, whose work-queue launch is the
+ * autotuner's alone (SSE_OPT_PERSISTENT and sse_run_budgets_noalloc are refused;
  * sse_run_budgets issues one launch per sweep index).                      */
 #define SSE_MAX_BOND_SITES 4
 typedef struct sse_vertex_data_desc {
@@ -408,7 +408,8 @@ int sse_pt_get_ladders(sse_batch *b, int32_t *slot_walkers, int64_t *accepted,
  *                0 = walker index order.  Results are identical.
  * SSE_OPT_GENERIC (wave mode): 1 = run every model, two-site bonds included,
  *                through the generic wave kernels (the ones that bonds of one,
- *                three and four sites always take; no work-queue launch);
+ *                three and four sites always take; SSE_OPT_PERSISTENT is
+ *                refused, the autotuner may choose the work-queue launch);
  *                0 = the two-site kernels (an error while a model has bonds
  *                of other sizes).
  *                Default: 0 unless such a model is present.  Restarts tuning.

@@ -1197,9 +1197,9 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
             b->seen_need = std::max(b->seen_need, expected_need(b, walkers[w]));
         wave_resize_lds(b->wave, b->seen_need);
         if (!rc && b->wave.lds_limit > 65536)
-            (void)hipFuncSetAttribute((const void *)wave_persist_kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)b->wave.lds_limit);
+            for (const void *k : {(const void *)wave_persist_kernel, (const void *)waven_persist_kernel})
+                (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)b->wave.lds_limit);
         if (hipDeviceGetAttribute(&b->n_cu, hipDeviceAttributeMultiprocessorCount, b->device) !=
                 hipSuccess ||
             b->n_cu <= 0)
@@ -1747,7 +1747,7 @@ static int work_sum(sse_batch *b, unsigned long long *v)
 
 static void tune_apply(sse_batch *b, const sse_batch::TuneCfg &c)
 {
-    b->persistent = c.persistent != 0 && !b->wave.generic;
+    b->persistent = c.persistent != 0;
     b->n_groups = c.groups;
     b->wave.lds_k2_fixed = c.k2_lds;
     wave_resize_lds(b->wave, b->seen_need);
@@ -1776,12 +1776,8 @@ static void tune_init(sse_batch *b, sse_batch::Tuner &t, bool budgets)
         if (t.cands.empty())
             t.cands.push_back({0, 1, 0});
     }
-    if (!b->wave.generic) {  // the generic kernels have no work-queue launch
-        t.cands.push_back({1, 0, 0});
-        t.cands.push_back({1, 0, 32768});
-    }
-    if (t.cands.empty())
-        t.cands.push_back({0, 1, 0});
+    t.cands.push_back({1, 0, 0});
+    t.cands.push_back({1, 0, 32768});
     t.rate.assign(t.cands.size(), 0.0);
     t.runs.assign(t.cands.size(), 0);
     t.best = -1;
@@ -2619,7 +2615,7 @@ int sse_add_model(sse_batch *b, const sse_model_desc *model, int32_t *index)
     b->d_models = nd;
     if (dm.nsb != 2 || b->wave.generic) {
         // bonds of other than two sites: the generic wave kernels from now on
-        // (they take two-site models too), never the work-queue launch
+        // (they take two-site models too)
         b->wave.generic = 1;
         {
             int max_ns = 2;

@@ -477,7 +477,7 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
 // over the operator string, then one pass per magnetization estimator.  mode
 // as in k3_walker.
 template <int NS>
-__device__ void k3n_walker(DevWalker *W, const DevModel *models, double *out, double *sum,
+__device__ __forceinline__ void k3n_walker(DevWalker *W, const DevModel *models, double *out, double *sum,
                            double *sumsq, int64_t *count, double *wlf, int wi, int mode,
                            int32_t *done)
 {

@@ -141,3 +141,33 @@ def test_work_queue_hands_walkers_over(sse_pkg, oracle_mod, call):
             assert np.array_equal(a, b)
     one.close()
     batch.close()
+
+
+@pytest.mark.parametrize("kinds", [("trimer",), ("plaquette", "field", "trimer"), ("square", "trimer")])
+def test_generic_work_queue(sse_pkg, oracle_mod, kinds):
+    """Bonds of any site count, batches of one size and of several: the tuner's
+    calls run every launch form (stream groups, the work queue at two LDS sizes)
+    over the same chains, which stay the oracle's, sums included."""
+    flats = [MODELS[k](sse_pkg) for k in kinds]
+    walkers = [sse_pkg.walker_desc(model=k % len(flats), T=(0.3, 0.7, 1.5)[k % 3], seed=500 + k,
+                                   thermalization=3) for k in range(70)]
+    _say(f"generic work queue: {kinds}")
+    batch = sse_pkg.Batch(flats, walkers, mode=0)
+    batch.init()
+    sweeps = 0
+    while batch.tuning(0) is None and sweeps < 80:
+        batch.run(8, measure=True)
+        sweeps += 8
+    assert batch.tuning(0) is not None and batch.tuning(0)["candidates_measured"] >= 3
+    batch.run(6, measure=True)
+    sweeps += 6
+    for k in (0, 1, 2, 3, 4, 5, 69):
+        o = oracle_mod.OracleWalker(sse_pkg.capi, flats[k % len(flats)], walkers[k])
+        o.init()
+        o.sweep(sweeps)
+        gs, gops, gspins = batch.get_walker(k)
+        os_, oops, ospins = o.state()
+        assert np.array_equal(gops, oops) and np.array_equal(gspins, ospins)
+        assert gs["rng_counter"] == os_["rng_counter"] and gs["sweeps"] == sweeps
+    assert (batch.accumulators_raw()[2] == sweeps - 3).all()
+    batch.close()
