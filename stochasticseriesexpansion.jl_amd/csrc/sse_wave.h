@@ -828,6 +828,20 @@ __device__ __forceinline__ double wave_sum(double x)
     return x;
 }
 
+__device__ __forceinline__ int wave_sum_int(int x)
+{
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1)
+        x += __shfl_xor(x, o);
+    return x;
+}
+// lane q's x, wave-uniform
+__device__ __forceinline__ double lane_f64(double x, int q)
+{
+    const long long b = __double_as_longlong(x);
+    return __hiloint2double(__builtin_amdgcn_readlane((int)(b >> 32), q), __builtin_amdgcn_readlane((int)b, q));
+}
+
 // x moved across lanes by one DPP pattern, both 32-bit halves; lanes without
 // a source (or outside the row mask) read 0
 template <int kCtrl, int kRowMask>
@@ -853,95 +867,148 @@ __device__ __forceinline__ double wave_incl_scan(double x)
     return x;
 }
 
-// mode 0: explicit measure of every walker; mode 1: thermalized walkers only,
-// accumulated into the per-walker sums (fused sweep+measure loop).
-// One pass over the operator string: the sign (sse.jl:305-314) when
-// want_sign, and estimators e0 .. e0+ne-1 (ne <= K3_MAXE) of the
-// MagnetizationEstimator family (magnetization_estimator.jl:96-230), whose
-// running sums over the operator positions are wave prefix sums.  Writes the
-// five outputs of each of its estimators.
-constexpr int K3_MAXE = 4;
+// One pass over the operator string: the sign (sse.jl:305-314) when want_sign,
+// and estimators e0 .. e0+ne-1 of the MagnetizationEstimator family
+// (magnetization_estimator.jl:96-230), whose running sums over the operator
+// positions are wave prefix sums.  Writes the five outputs of each of its
+// estimators.  Estimators per pass: with the tables, whose pass holds eight
+// values of each at a time, and without.
+constexpr int K3_TABLE_E = 2, K3_MAXE = 4;
+template <int E>
 __device__ __forceinline__ void k3_finish(const DevWalker &w, const DevModel &m, int e0, int ne,
                                           bool want_sign, int neg, int64_t cnt, const double *tmp0,
                                           const double *mag, const double *absmag, const double *mag2,
                                           const double *mag4, double &sign, double *o);
-__device__ __forceinline__ void k3_pass(const DevWalker &w, const DevModel &m, int e0, int ne,
-                                        bool want_sign, double &sign, double *o)
+// The estimators' values before the first operator.
+template <int E>
+__device__ __forceinline__ void k3_start(const DevWalker &w, const DevModel &m, int e0, int ne, double *tmp0)
+{
+    const int N = m.n_sites, D = m.est_max_dim;
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+        double t0 = 0.0;
+        if (k < ne) {
+            const double *cf = m.est_coef + (size_t)(e0 + k) * N, *mk = m.est_mval + (size_t)(e0 + k) * N * D;
+            for (int i = threadIdx.x; i < N; i += 64)
+                t0 += cf[i] * mk[i * D + w.spins[i] - 1];
+        }
+        tmp0[k] = k < ne ? wave_sum(t0) : 0.0;
+    }
+}
+
+// From per-(bond, vertex) tables: an operator's estimator changes and sign are
+// one gather each.  A lane takes four slots in a row, so one prefix sum over the
+// wave, which was most of a chunk's work, serves 256 slots instead of 64; the
+// operators are loaded two chunks ahead, their table values one ahead.  Measured
+// on 16x16 Heisenberg at beta = 8 (8711 slots, two estimators): 88 -> 52 us of a
+// lone wave, 125 -> 77 us with 1536 walkers.  Four estimators in a pass (173
+// registers) gave half of that back in the work-queue kernel.
+__device__ __forceinline__ void k3_table_pass(const DevWalker &w, const DevModel &m, int e0, int ne,
+                                              bool want_sign, double &sign, double *o)
+{
+    constexpr int E = K3_TABLE_E;
+    const int lane = threadIdx.x;
+    const int64_t L = w.L;
+    double tmp0[E], run[E], mag[E] = {}, absmag[E] = {}, mag2[E] = {}, mag4[E] = {};
+    k3_start<E>(w, m, e0, ne, tmp0);
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+        run[k] = tmp0[k];
+    const gmem<uint32_t> *ops = as_global((const uint32_t *)w.ops);
+    constexpr int K = 4;
+    const gmem<double> *DT = as_global(m.est_dtab);
+    const gmem<int8_t> *SG = as_global(m.est_dsgn);
+    const uint32_t dnv = (uint32_t)m.est_dnv, NE = (uint32_t)m.n_est;
+    const bool sgn = want_sign && m.any_neg;
+    // slots past L (the vector may hold up to three) read as identities
+    auto ops_at = [&](int64_t q, uint32_t (&op)[K]) {
+        u32x4 x = {0u, 0u, 0u, 0u};
+        if (q < L)
+            x = *(const gmem<u32x4> *)(ops + q);
+        op[0] = x.x;
+        op[1] = q + 1 < L ? x.y : 0u;
+        op[2] = q + 2 < L ? x.z : 0u;
+        op[3] = q + 3 < L ? x.w : 0u;
+    };
+    auto vals_of = [&](const uint32_t (&op)[K], double (&d)[E][K], int &ng) {
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const uint32_t ix = op_bond(op[j]) * dnv + (op_vcode(op[j]) >> 1);
+            const bool offd = op[j] != 0u && !(op_vcode(op[j]) & 1u);
+#pragma unroll
+            for (int k = 0; k < E; ++k)
+                d[k][j] = k < ne && offd ? DT[(size_t)ix * NE + e0 + k] : 0.0;
+            if (sgn && op[j] != 0u)
+                ng += SG[ix] < 0;
+        }
+    };
+    int ngl = 0, cntl = 0;
+    uint32_t op0[K], op1[K];
+    ops_at(K * lane, op0);
+    ops_at(64 * K + K * lane, op1);
+    double d0[E][K];
+    vals_of(op0, d0, ngl);
+    for (int64_t base = 0; base < L; base += 64 * K) {
+        uint32_t op2[K];
+        ops_at(base + 128 * K + K * lane, op2);
+        double d1[E][K];
+        vals_of(op1, d1, ngl);
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            cntl += op0[j] != 0u;
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+            if (k < ne) {
+                const double own = (d0[k][0] + d0[k][1]) + (d0[k][2] + d0[k][3]);
+                const double inc = wave_incl_scan(own);
+                double t = run[k] + (inc - own);
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    t += d0[k][j];
+                    const double u = op0[j] != 0u ? t : 0.0;
+                    const double u2 = u * u;
+                    mag[k] += u;
+                    absmag[k] += fabs(u);
+                    mag2[k] += u2;
+                    mag4[k] += u2 * u2;
+                }
+                run[k] += lane_f64(inc, 63);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            op0[j] = op1[j];
+            op1[j] = op2[j];
+#pragma unroll
+            for (int k = 0; k < E; ++k)
+                d0[k][j] = d1[k][j];
+        }
+    }
+    k3_finish<E>(w, m, e0, ne, want_sign, wave_sum_int(ngl), wave_sum_int(cntl), tmp0, mag, absmag, mag2,
+                 mag4, sign, o);
+}
+
+// The same from the bonds' and vertices' own tables, for models without the
+// per-(bond, vertex) ones.
+__device__ __forceinline__ void k3_gather_pass(const DevWalker &w, const DevModel &m, int e0, int ne,
+                                               bool want_sign, double &sign, double *o)
 {
     const int lane = threadIdx.x;
     const int64_t L = w.L;
     const int N = m.n_sites, D = m.est_max_dim;
     const double *coef[K3_MAXE], *mv[K3_MAXE];
-    double tmp0[K3_MAXE], run[K3_MAXE], mag[K3_MAXE], absmag[K3_MAXE], mag2[K3_MAXE], mag4[K3_MAXE];
+    double tmp0[K3_MAXE], run[K3_MAXE], mag[K3_MAXE] = {}, absmag[K3_MAXE] = {}, mag2[K3_MAXE] = {},
+                                        mag4[K3_MAXE] = {};
+    k3_start<K3_MAXE>(w, m, e0, ne, tmp0);
 #pragma unroll
     for (int k = 0; k < K3_MAXE; ++k) {
         coef[k] = m.est_coef + (size_t)(e0 + k) * N;
         mv[k] = m.est_mval + (size_t)(e0 + k) * N * D;
-        double t0 = 0.0;
-        if (k < ne)
-            for (int i = lane; i < N; i += 64)
-                t0 += coef[k][i] * mv[k][i * D + w.spins[i] - 1];
-        tmp0[k] = k < ne ? wave_sum(t0) : 0.0;
         run[k] = tmp0[k];
-        mag[k] = absmag[k] = mag2[k] = mag4[k] = 0.0;
     }
     int neg = 0;
     int64_t cnt = 0;
     const gmem<uint32_t> *ops = as_global((const uint32_t *)w.ops);
-    if (m.est_dtab) {
-        // per-(bond, vertex) tables: an operator's estimator changes and sign
-        // are one gather each; the operator is loaded two chunks ahead, its
-        // table values one ahead
-        const gmem<double> *DT = as_global(m.est_dtab);
-        const gmem<int8_t> *SG = as_global(m.est_dsgn);
-        const uint32_t dnv = (uint32_t)m.est_dnv, NE = (uint32_t)m.n_est;
-        const bool sgn = want_sign && m.any_neg;
-        auto op_at = [&](int64_t q) -> uint32_t { return q < L ? ops[q] : 0u; };
-        auto vals_of = [&](uint32_t op, double *d, int8_t &sg) {
-            const uint32_t ix = op_bond(op) * dnv + (op_vcode(op) >> 1);
-            const bool offd = op != 0u && !(op_vcode(op) & 1u);
-#pragma unroll
-            for (int k = 0; k < K3_MAXE; ++k)
-                d[k] = k < ne && offd ? DT[(size_t)ix * NE + e0 + k] : 0.0;
-            sg = sgn && op != 0u ? SG[ix] : (int8_t)0;
-        };
-        uint32_t op0 = op_at(lane), op1 = op_at(64 + lane);
-        double d0[K3_MAXE];
-        int8_t sg0;
-        vals_of(op0, d0, sg0);
-        for (int64_t base = 0; base < L; base += 64) {
-            const uint32_t op2 = op_at(base + 128 + lane);
-            double d1[K3_MAXE];
-            int8_t sg1;
-            vals_of(op1, d1, sg1);
-            if (sgn)
-                neg += popc(__ballot(op0 != 0u && sg0 < 0));
-            cnt += popc(__ballot(op0 != 0u));
-#pragma unroll
-            for (int k = 0; k < K3_MAXE; ++k) {
-                if (k < ne) {
-                    const double inc = wave_incl_scan(d0[k]);
-                    if (op0 != 0u) {
-                        const double t = run[k] + inc;
-                        const double t2 = t * t;
-                        mag[k] += t;
-                        absmag[k] += fabs(t);
-                        mag2[k] += t2;
-                        mag4[k] += t2 * t2;
-                    }
-                    run[k] += __shfl(inc, 63);
-                }
-            }
-            op0 = op1;
-            op1 = op2;
-#pragma unroll
-            for (int k = 0; k < K3_MAXE; ++k)
-                d0[k] = d1[k];
-            sg0 = sg1;
-        }
-        k3_finish(w, m, e0, ne, want_sign, neg, cnt, tmp0, mag, absmag, mag2, mag4, sign, o);
-        return;
-    }
     const gmem<uint64_t> *brec = as_global((const uint64_t *)m.bond_rec);  // int2 pairs
     // Software pipeline over the 64-slot chunks: the operator is loaded three
     // chunks ahead, its bond record two ahead, the vertex's sign and leg states
@@ -1025,10 +1092,11 @@ __device__ __forceinline__ void k3_pass(const DevWalker &w, const DevModel &m, i
         sg0 = sg1;
         lg0 = lg1;
     }
-    k3_finish(w, m, e0, ne, want_sign, neg, cnt, tmp0, mag, absmag, mag2, mag4, sign, o);
+    k3_finish<K3_MAXE>(w, m, e0, ne, want_sign, neg, cnt, tmp0, mag, absmag, mag2, mag4, sign, o);
 }
 
 // The five outputs of each estimator of a pass (and the sign of the first).
+template <int E>
 __device__ __forceinline__ void k3_finish(const DevWalker &w, const DevModel &m, int e0, int ne,
                                           bool want_sign, int neg, int64_t cnt, const double *tmp0,
                                           const double *mag, const double *absmag, const double *mag2,
@@ -1041,7 +1109,7 @@ __device__ __forceinline__ void k3_finish(const DevWalker &w, const DevModel &m,
     const double en = 1.0 + (double)cnt;
     const double norm = 1.0 / Nn;
 #pragma unroll
-    for (int k = 0; k < K3_MAXE; ++k) {
+    for (int k = 0; k < E; ++k) {
         if (k < ne) {
             double smag = tmp0[k] + wave_sum(mag[k]);
             double sabs = fabs(tmp0[k]) + wave_sum(absmag[k]);
@@ -1067,7 +1135,7 @@ __device__ __forceinline__ void k3_finish(const DevWalker &w, const DevModel &m,
 
 // measure (sse.jl:70-87, 305-376) of walker wi.  mode 0: explicit measure;
 // mode 1: thermalized walkers only, accumulated into the per-walker sums
-// (fused sweep+measure loop).  Estimators are taken K3_MAXE per pass over the
+// (fused sweep+measure loop).  Estimators are taken a few per pass over the
 // operator string; the first pass also computes the sign.
 __device__ __forceinline__ void k3_walker(DevWalker *W, const DevModel *models, double *out, double *sum,
                                           double *sumsq, int64_t *count, double *wlf, int wi, int mode,
@@ -1091,9 +1159,13 @@ __device__ __forceinline__ void k3_walker(DevWalker *W, const DevModel *models, 
     double sign = 1.0;
     int e0 = 0;
     do {
-        const int ne = m.n_est - e0 < K3_MAXE ? m.n_est - e0 : K3_MAXE;
-        k3_pass(w, m, e0, ne, e0 == 0, sign, o);
-        e0 += K3_MAXE;
+        const int E = m.est_dtab ? K3_TABLE_E : K3_MAXE;
+        const int ne = m.n_est - e0 < E ? m.n_est - e0 : E;
+        if (m.est_dtab)
+            k3_table_pass(w, m, e0, ne, e0 == 0, sign, o);
+        else
+            k3_gather_pass(w, m, e0, ne, e0 == 0, sign, o);
+        e0 += E;
     } while (e0 < m.n_est);
     const double nn = (double)w.n;
     if (lane == 0) {

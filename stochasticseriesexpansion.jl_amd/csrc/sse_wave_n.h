@@ -552,7 +552,7 @@ __device__ __forceinline__ void k3n_walker(DevWalker *W, const DevModel *models,
             }
             run += __shfl(inc, 63);
         }
-        // as k3_pass: the estimator's five values (magnetization_estimator.jl:125-165,205-230)
+        // as k3_finish: the estimator's five values (magnetization_estimator.jl:125-165,205-230)
         const double Nn = m.norm;
         const double en = 1.0 + (double)cnt;
         const double norm = 1.0 / Nn;

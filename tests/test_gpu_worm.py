@@ -171,3 +171,29 @@ def test_generic_work_queue(sse_pkg, oracle_mod, kinds):
         assert gs["rng_counter"] == os_["rng_counter"] and gs["sweeps"] == sweeps
     assert (batch.accumulators_raw()[2] == sweeps - 3).all()
     batch.close()
+
+
+@pytest.mark.parametrize("cutoff", [255, 256, 257, 511, 1023])
+@pytest.mark.parametrize("n_est", [1, 2, 4])
+def test_measure_chunks(sse_pkg, oracle_mod, cutoff, n_est):
+    """The measurement at operator strings about its 256-slot chunks, one pass of
+    estimators and two: the oracle's values to 1e-12 (sums in another order)."""
+    if n_est == 4:
+        flat = job_honeycomb(sse_pkg, 0.5).flat()
+    else:
+        flat = square_heisenberg(sse_pkg, 4, measure=("magnetization", "staggered_magnetization")[:n_est]).flat()
+    walkers = [sse_pkg.walker_desc(T=T, seed=700 + k, init_opstring_cutoff=cutoff)
+               for k, T in enumerate((0.6, 2.0))]
+    _say(f"measure chunks: cutoff={cutoff} estimators={n_est}")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    oracles = [oracle_mod.OracleWalker(sse_pkg.capi, flat, w) for w in walkers]
+    batch.init()
+    for o in oracles:
+        o.init()
+    for s in range(4):
+        batch.sweep(2)
+        gm = batch.measure()
+        for k, o in enumerate(oracles):
+            o.sweep(2)
+            assert np.allclose(gm[k], o.measure(), rtol=1e-12, atol=1e-13)
+    batch.close()
