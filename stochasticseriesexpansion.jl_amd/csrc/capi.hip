@@ -83,6 +83,7 @@ struct sse_batch {
     DevWalker *d_walkers = nullptr;
     std::vector<DevWalker> h_walkers;
     DevPool *d_pool = nullptr;
+    PoolReport *report = nullptr, *d_report = nullptr;  // pinned host memory, host and device address
     char *pool_base = nullptr;
     size_t pool_size = 0;
     size_t pool_host_next = 0;
@@ -889,11 +890,33 @@ static int sync_pool_from_device(sse_batch *b)
     return SSE_OK;
 }
 
-static int check_walker_errors(sse_batch *b)
+// Writes the report of a call (and n_out values of out behind it) and restarts
+// the pool's maxima.
+__global__ void pool_report_kernel(DevPool *pool, PoolReport *r, const double *out, int n_out)
 {
-    DevPool p;
+    const int i = threadIdx.x;
+    if (i < 8) {
+        r->max_need[i] = pool->max_need[i];
+        pool->max_need[i] = 0ull;
+    }
+    if (i == 0) {
+        r->overflow = pool->overflow;
+        r->status = pool->status;
+    }
+    for (int k = i; k < n_out; k += (int)blockDim.x)
+        r->out[k] = out[k];
+}
+
+// Ends a call: waits for the stream once and turns the walkers' error words into
+// a status.  With copies of the pool to pageable memory (and of the zeroed
+// maxima back) each call waited three times, a call that measures four.
+static int check_walker_errors(sse_batch *b, const double *out = nullptr, int n_out = 0)
+{
+    hipLaunchKernelGGL(pool_report_kernel, dim3(1), dim3(256), 0, b->stream, b->d_pool, b->d_report, out,
+                       n_out);
+    HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(b->stream));
-    HIPCHECK(bmemcpy(b, &p, b->d_pool, sizeof p, hipMemcpyDeviceToHost));
+    const PoolReport &p = *b->report;
     if (p.overflow)
         return fail(SSE_ERR_OOM, "slab pool exhausted; raise SSE_POOL_MB");
     unsigned long long need = 0;
@@ -904,9 +927,6 @@ static int check_walker_errors(sse_batch *b)
         // sweeps (the device maxima restart at zero for the next call): one
         // size for single-stream launches, one per stream group
         b->seen_need = need;
-        const unsigned long long zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        static_assert(sizeof zero == sizeof p.max_need, "pool maxima layout");
-        HIPCHECK(bmemcpy(b, b->d_pool->max_need, zero, sizeof zero, hipMemcpyHostToDevice));
         wave_resize_lds(b->wave, b->seen_need);
         for (int g = 0; g < 7; ++g)
             if (p.max_need[g])
@@ -1086,6 +1106,9 @@ int sse_batch_create(const sse_model_desc *models, int32_t n_models, const sse_w
         rc = dev_alloc(b, &b->pool_base, b->pool_size);
     if (!rc)
         rc = dev_alloc(b, &b->d_pool, 1);
+    if (!rc && (hipHostMalloc((void **)&b->report, sizeof(PoolReport), hipHostMallocDefault) != hipSuccess ||
+                hipHostGetDevicePointer((void **)&b->d_report, b->report, 0) != hipSuccess))
+        rc = fail(SSE_ERR_OOM, "hipHostMalloc failed");
     size_t nsp = (size_t)n_walkers * b->max_sites;
     if (!rc)
         rc = dev_alloc(b, &b->d_spins, nsp);
@@ -1232,6 +1255,8 @@ int sse_batch_destroy(sse_batch *b)
         (void)hipStreamSynchronize(b->stream);
     for (void *p : b->allocs)
         (void)hipFree(p);
+    if (b->report)
+        (void)hipHostFree(b->report);
     for (int i = 0; i < 4; ++i)
         if (b->ev[i])
             (void)hipEventDestroy(b->ev[i]);
@@ -2031,11 +2056,16 @@ int sse_measure(sse_batch *b, double *out)
     int rc = launch_measure(b, 0);
     if (rc)
         return rc;
-    if (out) {
-        HIPCHECK(hipMemcpyAsync(out, b->d_out, sizeof(double) * b->total_width,
-                                hipMemcpyDeviceToHost, b->stream));
+    const size_t width = (size_t)b->total_width;
+    if (!out || width > kReportOut) {
+        if (out)
+            HIPCHECK(hipMemcpyAsync(out, b->d_out, sizeof(double) * width, hipMemcpyDeviceToHost, b->stream));
+        return check_walker_errors(b);
     }
-    return check_walker_errors(b);
+    // small results come with the report
+    rc = check_walker_errors(b, b->d_out, (int)width);
+    memcpy(out, b->report->out, sizeof(double) * width);
+    return rc;
 }
 
 int sse_run(sse_batch *b, int32_t n_sweeps, int32_t measure)

@@ -186,6 +186,15 @@ struct DevPool {
     unsigned long long max_need[8];
 };
 
+// What the host reads after a call, in pinned host memory: the pool's error words
+// and maxima, then (doubles) the measurement of a call that returns one.
+constexpr size_t kReportOut = 8192;
+struct PoolReport {
+    int32_t overflow, status;
+    unsigned long long max_need[8];
+    double out[kReportOut];
+};
+
 __device__ __forceinline__ void flag_error(DevPool *pool, int code)
 {
     atomicOr(&pool->status, 1 << code);

@@ -1323,7 +1323,9 @@ static inline size_t wave_k2_lds_for(const WaveConfig &c, unsigned long long max
     // occupancy query says).
     const size_t per_cu = std::min(c.lds_limit, (size_t)162816);
     auto alloc = [](size_t b) { return (b + 256 + 511) & ~(size_t)511; };
-    const size_t k = std::max((size_t)1, per_cu / alloc(need));  // walkers per CU
+    // walkers per CU: as many as fit, at most the 8 that the registers allow.  So
+    // batches of small walkers keep one size, and a captured launch stays valid.
+    const size_t k = std::min((size_t)8, std::max((size_t)1, per_cu / alloc(need)));
     size_t wide = ((per_cu / k) & ~(size_t)511) - 256;
     if (wide < need)
         wide = need;

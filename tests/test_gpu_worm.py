@@ -197,3 +197,22 @@ def test_measure_chunks(sse_pkg, oracle_mod, cutoff, n_est):
             o.sweep(2)
             assert np.allclose(gm[k], o.measure(), rtol=1e-12, atol=1e-13)
     batch.close()
+
+
+@pytest.mark.parametrize("n", [546, 547])
+def test_measure_returns_every_walker(sse_pkg, oracle_mod, n):
+    """15 values a walker: 8190 come with the call's report, 8205 by a copy."""
+    flat = square_heisenberg(sse_pkg, 4).flat()
+    walkers = [sse_pkg.walker_desc(T=1.0, seed=900 + k) for k in range(n)]
+    _say(f"measure of {n} walkers")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    batch.init()
+    batch.sweep(3)
+    gm = batch.measure()
+    assert len(gm) == n and len(gm[0]) == 15
+    for k in (0, 1, n // 2, n - 1):
+        o = oracle_mod.OracleWalker(sse_pkg.capi, flat, walkers[k])
+        o.init()
+        o.sweep(3)
+        assert np.allclose(gm[k], o.measure(), rtol=1e-12, atol=1e-13)
+    batch.close()
