@@ -16,11 +16,10 @@
 #pragma once
 
 // LDS of K1n (one walker): Philox words u64[256], lane masks u64[NS][N],
-// operators on the site so far u32[N], upper leg states of the chunk's
-// operators u32[64] (one byte per bond position), spins u8[N]
+// operators on the site so far u32[N], spins u8[N]
 __host__ __device__ inline size_t k1n_lds_bytes(int N, int NS)
 {
-    size_t b = 2048 + 8 * (size_t)NS * N + 4 * (size_t)N + 256 + (size_t)N;
+    size_t b = 2048 + 8 * (size_t)NS * N + 4 * (size_t)N + (size_t)N;
     return (b + 15) & ~(size_t)15;
 }
 
@@ -176,8 +175,7 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
     uint64_t *rbuf = (uint64_t *)lds;
     uint64_t *tm = (uint64_t *)(lds + 2048);  // tm[k * N + site]
     uint32_t *cnt = (uint32_t *)(tm + (size_t)NS * N);
-    uint32_t *cups = cnt + N;
-    uint8_t *sp = (uint8_t *)(cups + 64);
+    uint8_t *sp = (uint8_t *)(cnt + N);
     uint32_t *tmw = (uint32_t *)tm;
 
     const bool do_diag = phases & 1;
@@ -225,93 +223,106 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
     rs.init(rbuf, w.key, w.ctr);
     const double pm_raw = (double)m.n_bonds / w.T;
     const double pr_raw = w.T / (double)m.n_bonds;
-    const uint64_t Nb = (uint64_t)m.n_bonds;
     const int64_t L = w.L;
+    const uint32_t Lu = (uint32_t)L;
     int64_t n0 = w.n;
     const uint64_t below = below_mask(lane), above = above_mask(lane);
     gmem<uint32_t> *gidx = as_global((uint32_t *)w.links);
     gmem<uint32_t> *ops = as_global(w.ops);
 
-    // read once: a read of the model inside the loop would wait for the
-    // chunk's global stores
-    const uint32_t nbonds = (uint32_t)m.n_bonds;
-    uint32_t op_next = (int64_t)lane < L ? ops[lane] : 0u;
-    for (int64_t base = 0; base < L; base += 64) {
-        const int64_t p = base + lane;
-        const bool valid = p < L;
-        const uint32_t op = op_next;
-        op_next = p + 64 < L ? ops[p + 64] : 0u;
+    // As in k1_walker_t: the operators come in blocks of K1_BLOCK chunks, a block
+    // ahead (an operator loaded in one chunk for the next would be waited on with
+    // the chunk's stores), the model's scalars are read before the loop, and the
+    // lanes run one path.  Measured on 64 walkers: ring of three-site bonds (8711
+    // slots) 343 -> 246 us per sweep, of four-site bonds (1439 slots) 78 -> 59 us.
+    const uint32_t nbonds = uni((uint32_t)m.n_bonds);
+    uint32_t cur[K1_BLOCK], pf[K1_BLOCK];
+#pragma unroll
+    for (int u = 0; u < K1_BLOCK; ++u) {
+        const uint32_t q = 64u * u + lane;
+        cur[u] = q < Lu ? ops[q] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < K1_BLOCK; ++u) {
+        const uint32_t q = 64u * (K1_BLOCK + u) + lane;
+        pf[u] = q < Lu ? ops[q] : 0u;
+    }
+    bool bad = false;
+    for (uint32_t base = 0; base < Lu; base += 64) {
+        const uint32_t p = base + lane;
+        const bool valid = p < Lu;
+        const uint32_t chunk = base >> 6;
+        const int slot = (int)uni(chunk % K1_BLOCK);
+        if (slot == 0 && chunk > 0) {
+#pragma unroll
+            for (int u = 0; u < K1_BLOCK; ++u)
+                cur[u] = pf[u];
+#pragma unroll
+            for (int u = 0; u < K1_BLOCK; ++u) {
+                const uint32_t q = base + 64u * (K1_BLOCK + u) + lane;
+                pf[u] = q < Lu ? ops[q] : 0u;
+            }
+        }
+        const uint32_t op = cur[slot];
         const uint32_t vc = op_vcode(op);
         const bool ident = valid && op == 0u;
-        const bool isop = valid && op != 0u;
+        const bool isop = op != 0u;
         const bool dia = isop && (vc & 1u);
         const bool offd = isop && !(vc & 1u);
         const uint64_t identm = __ballot(ident), diam = __ballot(dia), offm = __ballot(offd);
         uint32_t b = op_bond(op);
+        // an operator outside the model (a corrupted string): reported when the
+        // walker ends, its bond and vertex replaced by ones that exist
+        bad |= b >= nbonds;
+        b = b < nbonds ? b : 0u;
         double u = 0.0;
-        {
-            bool bad = false;
-            if (isop) {
-                bad = b >= nbonds;
-                if (!bad)
-                    bad = (int)(vc >> 1) >= tab.nv(tab.type(b));
-            }
-            if (__ballot(bad)) {
-                if (lane == 0) {
-                    W[wi].error = SSE_ERR_STATE;
-                    flag_error(pool, SSE_ERR_STATE);
-                }
-                return;
-            }
-        }
-
         if (do_diag) {
-            const int D = 2 * popc(identm) + popc(diam);
-            const int off = 2 * popc(identm & below) + popc(diam & below);
-            bool reject = force_serial;
-            if (D > 0) {
-                rs.ensure((uint32_t)D);
-                if (ident) {
-                    uint64_t x = rs.peek((uint32_t)off);
-                    uint64_t lo = x * Nb;
-                    b = (uint32_t)__umul64hi(x, Nb);
-                    if (lo < Nb && lo < (0ull - Nb) % Nb)
-                        reject = true;
-                    u = word_to_float(rs.peek((uint32_t)off + 1));
-                } else if (dia) {
-                    u = word_to_float(rs.peek((uint32_t)off));
-                }
-            }
-            if (__ballot(reject)) {
+            const uint32_t D = 2u * (uint32_t)popc(identm) + (uint32_t)popc(diam);
+            const uint32_t off = 2u * bits_below(identm) + bits_below(diam);
+            if (D > 0u)
+                rs.ensure(D);
+            const uint64_t x0 = rs.peek(D ? off : 0u), x1 = rs.peek(D ? off + 1u : 0u);
+            // rand(1:n_bonds): high half of word * n_bonds, rejected where the low
+            // half could be below 2^64 mod n_bonds
+            const uint64_t pl = (uint64_t)(uint32_t)x0 * nbonds;
+            const uint64_t ph = (uint64_t)(uint32_t)(x0 >> 32) * nbonds + (pl >> 32);
+            const bool maybe = ident && (uint32_t)ph == 0u && (uint32_t)pl < nbonds;
+            if (__builtin_expect(force_serial || wave_any(maybe), 0)) {
                 k1n_serial_chunk<NS>(w, m, rs, base, n0, pm_raw, pr_raw, do_diag, do_vl, sp, cnt);
                 continue;
             }
-            rs.advance((uint32_t)D);
+            b = ident ? (uint32_t)(ph >> 32) : b;
+            u = word_to_float(ident ? x1 : x0);
+            rs.advance(D);
         } else if (force_serial) {
             k1n_serial_chunk<NS>(w, m, rs, base, n0, pm_raw, pr_raw, do_diag, do_vl, sp, cnt);
             continue;
         }
 
         const bool has = isop || (ident && do_diag);
+        const int type = tab.type(b);
         int st[NS];
-        int type = 0;
 #pragma unroll
         for (int k = 0; k < NS; ++k)
-            st[k] = 0;
-        if (has) {
-            type = tab.type(b);
-#pragma unroll
-            for (int k = 0; k < NS; ++k)
-                st[k] = tab.site(b, k);
-        }
+            st[k] = tab.site(b, k);
         // per-site lane masks, one per bond position
         if (has) {
 #pragma unroll
             for (int k = 0; k < NS; ++k)
                 atomicOr(&tmw[2 * ((size_t)k * N + st[k]) + (lane >> 5)], 1u << (lane & 31));
         }
-        if (offd)
-            cups[lane] = tab.upper(type, (int)(vc >> 1));
+        int vx = (int)(vc >> 1);
+        const bool vbad = vx >= tab.nv(type);
+        bad |= isop && vbad;
+        vx = vbad ? 0 : vx;
+        const uint32_t up = tab.upper(type, vx);  // an off-diagonal operator's states after it
+        double wgt = tab.weight(type, vx);        // a diagonal operator's weight
+        uint32_t s0[NS], c0[NS];
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+            s0[j] = sp[st[j]];
+            c0[j] = cnt[st[j]];
+        }
         wave_lds_sync();
         // M[j][k]: lanes whose bond has the site of this lane's position j at
         // position k; A[j]: lanes whose bond touches that site at all
@@ -321,65 +332,44 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
             A[j] = 0ull;
 #pragma unroll
             for (int k = 0; k < NS; ++k) {
-                M[j][k] = has ? tm[(size_t)k * N + st[j]] : 0ull;
+                M[j][k] = tm[(size_t)k * N + st[j]];
                 A[j] |= M[j][k];
             }
         }
-        // position of this lane's site j in the bond of lane q
-        auto pos_in = [&](int j, int q) -> int {
-            int r = 0;
-#pragma unroll
-            for (int k = 0; k < NS; ++k)
-                if ((M[j][k] >> q) & 1ull)
-                    r = k;
-            return r;
-        };
 
         uint64_t plus = 0, minus = 0;
         uint32_t fop = op;
         if (do_diag) {
-            double wgt = 0.0;
-            int32_t dv = -1;
-            if (ident) {
-                int idx = 0, stride = 1;
+            // states at the slot: of the latest off-diagonal operator on the site
+            // earlier in the chunk, else at the chunk's start
+            int idx = 0, stride = 1;
 #pragma unroll
-                for (int j = 0; j < NS; ++j) {
-                    int v;
-                    const uint64_t cand = A[j] & offm & below;
-                    if (cand) {
-                        const int q = hi_bit(cand);
-                        v = (int)((cups[q] >> (8 * pos_in(j, q))) & 255u);
-                    } else {
-                        v = sp[st[j]];
-                    }
-                    idx += (v - 1) * stride;
-                    stride *= tab.dim(type, j);
-                }
-                dv = tab.diag(type, idx);
-                wgt = dv < 0 ? 0.0 : tab.weight(type, dv >> 1);
-            } else if (dia) {
-                wgt = tab.weight(type, (int)(vc >> 1));
+            for (int j = 0; j < NS; ++j) {
+                const uint64_t cand = A[j] & offm & below;
+                const uint32_t q = cand ? (uint32_t)hi_bit(cand) : 0u;
+                const uint32_t uq = from_lane(up, q);
+                uint32_t pos = 0;  // of the site in that operator's bond
+#pragma unroll
+                for (int k = 1; k < NS; ++k)
+                    pos = ((M[j][k] >> q) & 1ull) ? 8u * k : pos;
+                const int v = (int)(cand ? (uq >> pos) & 255u : s0[j]);
+                idx += (v - 1) * stride;
+                stride *= tab.dim(type, j);
             }
-            bool amb = false, dec = false;
-            if (ident) {
-                int64_t lo = n0 - lane < 0 ? 0 : n0 - lane;
-                int64_t hi = n0 + lane > L - 1 ? L - 1 : n0 + lane;
-                bool d_lo = u < (pm_raw / (double)(L - lo)) * wgt;
-                bool d_hi = u < (pm_raw / (double)(L - hi)) * wgt;
-                amb = d_lo != d_hi;
-                dec = d_lo;
-            } else if (dia) {
-                int64_t lo = n0 - lane < 1 ? 1 : n0 - lane;
-                int64_t hi = n0 + lane > L ? L : n0 + lane;
-                double uw = u * wgt;
-                bool d_lo = uw < (double)(L - lo + 1) * pr_raw;
-                bool d_hi = uw < (double)(L - hi + 1) * pr_raw;
-                amb = d_lo != d_hi;
-                dec = d_lo;
-            }
-            plus = __ballot(ident && !amb && dec);
-            minus = __ballot(dia && !amb && dec);
-            uint64_t ambm = __ballot(amb);
+            const int32_t dv = ident ? tab.diag(type, idx) : -1;
+            const double wd = tab.weight(type, dv < 0 ? 0 : dv >> 1);
+            wgt = ident ? (dv < 0 ? 0.0 : wd) : wgt;
+            // as in k1_walker_t
+            const uint32_t room = Lu - (uint32_t)n0 + (ident ? 0u : 1u);
+            const uint32_t dl = room + (uint32_t)lane < Lu ? room + (uint32_t)lane : Lu;
+            const uint32_t dh = room > (uint32_t)lane ? room - (uint32_t)lane : 1u;
+            const double fl = (double)dl, fh = (double)dh;
+            const double pmw = pm_raw * wgt, uw = u * wgt;
+            const bool yes = ident ? (u * fl) * (1.0 + 0x1p-40) < pmw : uw < fh * pr_raw;
+            const bool no = ident ? (u * fh) * (1.0 - 0x1p-40) > pmw : !(uw < fl * pr_raw);
+            plus = __ballot(ident && yes);
+            minus = __ballot(dia && yes);
+            uint64_t ambm = __ballot((ident || dia) && !yes && !no);
             while (ambm) {
                 const int a = __ffsll((long long)ambm) - 1;
                 const uint64_t ba = below_mask(a);
@@ -403,36 +393,18 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
                 fop = op_make(b, (uint32_t)dv);
             if (dia && ((minus >> lane) & 1ull))
                 fop = 0u;
-            if (valid && fop != op)
+            if (fop != op)
                 ops[p] = fop;
         }
 
         // vertex list over the chunk's final non-identity operators: how many
         // earlier operators act on each of the operator's sites
         const uint64_t NI = do_diag ? ((identm & plus) | (diam & ~minus) | offm) : (diam | offm);
-        const bool isni = do_vl && ((NI >> lane) & 1ull);
-        uint32_t ix[NS];
-        bool last[NS];
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            ix[j] = 0u;
-            last[j] = false;
-        }
-        if (isni) {
+        if (do_vl && ((NI >> lane) & 1ull)) {
 #pragma unroll
             for (int j = 0; j < NS; ++j) {
-                const uint64_t mm = A[j] & NI;
-                ix[j] = cnt[st[j]] + (uint32_t)popc(mm & below);
-                last[j] = (mm & above) == 0ull;
-            }
-        }
-        wave_lds_sync();
-        if (isni) {
-#pragma unroll
-            for (int j = 0; j < NS; ++j) {
-                gidx[(size_t)NS * p + j] = ix[j];
-                if (last[j])
-                    cnt[st[j]] = ix[j] + 1u;
+                gidx[(size_t)NS * p + j] = c0[j] + bits_below(A[j] & NI);
+                atomicAdd(cnt + st[j], 1u);
             }
         }
         // spins after the chunk: the last off-diagonal operator on a site wins
@@ -440,7 +412,7 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
 #pragma unroll
             for (int j = 0; j < NS; ++j)
                 if (((A[j] & offm) & above) == 0ull)
-                    sp[st[j]] = (uint8_t)(cups[lane] >> (8 * j));
+                    sp[st[j]] = (uint8_t)(up >> (8 * j));
         }
         if (has) {
 #pragma unroll
@@ -448,6 +420,13 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
                 tm[(size_t)k * N + st[k]] = 0ull;
         }
         wave_lds_sync();
+    }
+    if (wave_any(bad)) {
+        if (lane == 0) {
+            W[wi].error = SSE_ERR_STATE;
+            flag_error(pool, SSE_ERR_STATE);
+        }
+        return;
     }
 
     if (do_vl) {
