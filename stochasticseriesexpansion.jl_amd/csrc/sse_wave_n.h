@@ -2,9 +2,8 @@
 // any site count NS = 1..4 (SSEData{NSites}, sse_data.jl:15-42; vertices of
 // 2*NS legs, vertex_list.jl:24-62).
 //
-// The two-site kernels of sse_wave.h pack four legs into their records and
-// chase tables; these kernels take the site count as a template parameter and
-// keep the same structure where it carries over:
+// These kernels take the site count as a template parameter and keep the
+// structure of the two-site ones of sse_wave.h where it carries over:
 //   K1n  diagonal update + vertex list, 64 slots per step (as K1: the same
 //        draws, acceptance windows and slot-by-slot fallback), with one
 //        per-site lane mask per bond position;
