@@ -216,3 +216,25 @@ def test_measure_returns_every_walker(sse_pkg, oracle_mod, n):
         o.sweep(3)
         assert np.allclose(gm[k], o.measure(), rtol=1e-12, atol=1e-13)
     batch.close()
+
+
+@pytest.mark.parametrize("n_walkers", [2, 600])
+def test_large_walkers(sse_pkg, oracle_mod, n_walkers):
+    """Records of more than 64 KB (some 10^4 operators), where each walker has a
+    compute unit to itself and where three share one."""
+    flat = square_heisenberg(sse_pkg, 32).flat()
+    walkers = [sse_pkg.walker_desc(T=0.13 if k < 2 else 8.0, seed=40 + k, thermalization=3)
+               for k in range(n_walkers)]
+    _say(f"large walkers: {n_walkers}")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    oracles = [oracle_mod.OracleWalker(sse_pkg.capi, flat, w) for w in walkers[:2]]
+    batch.init()
+    for o in oracles:
+        o.init()
+    for s in range(14):
+        batch.sweep(1)
+        for o in oracles:
+            o.sweep(1)
+        _compare(batch, oracles, f"sweep {s}")
+    assert batch.get_walker(0)[0]["num_operators"] > 10500
+    batch.close()
