@@ -110,6 +110,8 @@ struct __align__(16) WormEntry {
     uint32_t tail[4];
 };
 #define kWormSpecial (1ull << 63)
+// words (of 53 bits) from here on are looked up exactly
+constexpr uint64_t kWormTail = (1ull << 53) - 4096u;
 
 // Leg selector of an exit: for one and two sites per bond other | upper << 1
 // (other: not the entering site), else (position - entering position) mod sites

@@ -1,0 +1,239 @@
+// worm_tables.h -- host side of the worm update's exit tables: the images that
+// sse_worm.h reads, from the transition lists of a model.
+#pragma once
+#include <algorithm>
+#include <array>
+#include <cmath>
+#include <cstddef>
+#include <cstdint>
+#include <cstring>
+#include <map>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "../../include/ssegpu.h"
+#include "sse_common.h"
+
+// Host image of a model's worm tables (DevModel::w*).
+struct WormTables {
+    std::vector<uint4> bond;
+    std::vector<uint2> code;
+    std::vector<uint64_t> thr;
+    std::vector<uint32_t> row;
+    std::vector<uint4> exit;
+    std::vector<WormEntry> wide;
+    int nthr = 0, lg = 0, mw = 1, dim = 0;
+};
+
+// Exit rows take LDS beside every walker's records, which the step without a
+// compare has to be worth.
+constexpr size_t kWormRowBytes = 16384;
+// 16-byte exit entries beyond this are read from the global wide table.
+constexpr size_t kWormExitBytes = 16384;
+
+// Builds t; returns the reason why the model is refused, or null.
+inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
+{
+    const int ns = m.bond_n_sites, legs = 2 * ns;
+    t.lg = ns == 1 ? 0 : ns == 2 ? 1 : 2;
+    for (int i = 0; i < m.n_types; ++i)
+        t.mw = std::max(t.mw, (int)m.types[i].max_worm_count);
+    t.dim = m.site_dims[0];
+    for (int i = 1; i < m.n_sites; ++i)
+        if (m.site_dims[i] != t.dim)
+            t.dim = 0;
+    // r < c  <=>  (word >> 11) < ceil(c * 2^53)
+    auto thr = [](double c) {
+        return c <= 0.0 ? 0ull : c >= 1.0 ? (1ull << 53) : (uint64_t)std::ceil(std::ldexp(c, 53));
+    };
+    // bond types with equal vertices and transitions share a range of codes
+    std::map<std::string, int> seen;
+    std::vector<int> base(m.n_types), rep;  // code base per type; representative types
+    for (int i = 0; i < m.n_types; ++i) {
+        const sse_vertex_data_desc &vd = m.types[i];
+        std::string key;
+        auto add = [&](const void *p, size_t bytes) { key.append((const char *)p, bytes); };
+        const int nt = vd.n_vertices * vd.max_worm_count * legs;
+        add(&vd.n_vertices, sizeof vd.n_vertices);
+        add(&vd.max_worm_count, sizeof vd.max_worm_count);
+        add(vd.leg_states, (size_t)legs * vd.n_vertices);
+        for (int k = 0; k < nt; ++k) {
+            const int off = vd.transition_offset[k], cnt = off < 0 ? -1 : vd.transition_count[k];
+            if (cnt >= 4096)
+                return "transition with more than 4095 exits";
+            add(&cnt, sizeof cnt);
+            for (int j = 0; j < cnt; ++j) {
+                add(vd.exit_cumprob + off + j, sizeof(double));
+                add(vd.exit_target + off + j, sizeof(int32_t));
+                add(vd.exit_leg + off + j, 1);
+                add(vd.exit_worm + off + j, 1);
+            }
+        }
+        auto it = seen.find(key);
+        if (it != seen.end()) {
+            base[i] = it->second;
+            continue;
+        }
+        base[i] = (int)t.code.size();
+        seen.emplace(std::move(key), base[i]);
+        rep.push_back(i);
+        for (int v = 0; v < vd.n_vertices; ++v) {
+            const uint8_t *ls = vd.leg_states + (size_t)legs * v;
+            uint32_t lower = 0;
+            bool diag = true;
+            for (int k = 0; k < ns; ++k) {
+                lower |= (uint32_t)ls[k] << (8 * k);
+                diag &= ls[k] == ls[ns + k];
+            }
+            t.code.push_back(make_uint2(lower, (uint32_t)diag | (uint32_t)v << 1 | (uint32_t)i << 10));
+        }
+        // a vertex's diagonal flag is the one its exits' targets carry (equal to
+        // the comparison of its leg states in the reference's tables,
+        // vertex_data.jl:171-187)
+        for (int e = 0; e < vd.n_exits; ++e) {
+            uint32_t &y = t.code[(size_t)base[i] + ((uint32_t)vd.exit_target[e] >> 1)].y;
+            y = (y & ~1u) | ((uint32_t)vd.exit_target[e] & 1u);
+        }
+    }
+    const size_t nc = t.code.size(), ports = 2 * (size_t)t.mw;
+    const size_t nent = ((nc << t.lg) + 1) * ports;
+    if (nent >= ((size_t)1 << 30))
+        return "too many worm table entries";
+    for (int i : rep) {
+        const sse_vertex_data_desc &vd = m.types[i];
+        for (int e = 0; e < vd.n_exits; ++e) {
+            const uint64_t k = thr(vd.exit_cumprob[e]);
+            if (k < kWormTail)
+                t.thr.push_back(k);
+        }
+    }
+    std::sort(t.thr.begin(), t.thr.end());
+    t.thr.erase(std::unique(t.thr.begin(), t.thr.end()), t.thr.end());
+    t.nthr = (int)t.thr.size();
+    // m < k  <=>  q < rank(k), for words below kWormTail
+    auto rank = [&](uint64_t k) {
+        return k >= kWormTail ? 0xFFFFFFFFu
+                                 : (uint32_t)(std::lower_bound(t.thr.begin(), t.thr.begin() + t.nthr, k) -
+                                              t.thr.begin()) + 1u;
+    };
+    WormEntry none;
+    memset(&none, 0, sizeof none);
+    none.r[0] = none.r[1] = none.r[2] = 0xFFFFFFFFu;
+    for (int j = 0; j < 4; ++j)
+        none.out[j] = kWormSpecial;
+    t.wide.assign(nent, none);
+    bool rows = ns <= 2 && ports <= 128 && (nc << t.lg) <= 255 &&
+                (size_t)(t.nthr + 1) * nent * 4 <= kWormRowBytes;
+    std::map<size_t, std::array<uint64_t, 3>> fifth;  // fourth rank, exits 3 and 4
+    std::vector<uint32_t> row(rows ? (size_t)(t.nthr + 1) * nent : 0, 0u);
+    for (int i : rep) {
+        const sse_vertex_data_desc &vd = m.types[i];
+        for (int v = 0; v < vd.n_vertices; ++v)
+            for (int wv = 0; wv < vd.max_worm_count; ++wv)
+                for (int l = 0; l < legs; ++l) {
+                    const int src = (v * vd.max_worm_count + wv) * legs + l;
+                    const int off = vd.transition_offset[src], cnt = off < 0 ? 0 : vd.transition_count[src];
+                    const uint32_t pos = (uint32_t)(l % ns), side = (uint32_t)(l / ns);
+                    const size_t ix = ((((size_t)base[i] + v) << t.lg) + pos) * ports + 2 * (size_t)wv + side;
+                    WormEntry &x = t.wide[ix];
+                    auto word = [&](int j) {
+                        const uint32_t lo = vd.exit_leg[off + j], up = lo >= (uint32_t)ns;
+                        return worm_word(worm_leg(ns, pos, lo),
+                                         2u * ((uint32_t)vd.exit_worm[off + j] - 1u) + (up ^ 1u),
+                                         ((uint32_t)base[i] + ((uint32_t)vd.exit_target[off + j] >> 1)) << t.lg);
+                    };
+                    // exit 3 stands for every word past the first three
+                    // thresholds: the fourth exit if it ends the list at 1,
+                    // else none (the exact search decides)
+                    for (int j = 0; j < 3 && j < cnt; ++j) {
+                        x.r[j] = rank(thr(vd.exit_cumprob[off + j]));
+                        if (j && x.r[j] < x.r[j - 1])
+                            x.r[j] = x.r[j - 1];
+                        x.out[j] = word(j);
+                    }
+                    if (cnt > 0 && cnt < 3)  // past the last exit: none
+                        for (int j = cnt; j < 3; ++j)
+                            x.r[j] = 0xFFFFFFFFu;
+                    if (cnt >= 4) {
+                        const uint32_t r3 = rank(thr(vd.exit_cumprob[off + 3]));
+                        if (cnt == 4 && r3 == 0xFFFFFFFFu)
+                            x.out[3] = word(3);
+                        if (ns == 4 && cnt == 5 && rank(thr(vd.exit_cumprob[off + 4])) == 0xFFFFFFFFu)
+                            fifth[ix] = {r3, word(3), word(4)};
+                    }
+                    if (cnt > 0)
+                        rows = rows && thr(vd.exit_cumprob[off + cnt - 1]) == (1ull << 53);
+                    if (rows)
+                        for (int q = 0; q <= t.nthr && rows; ++q) {
+                            int j = 0;
+                            while (j < cnt && (uint32_t)q >= rank(thr(vd.exit_cumprob[off + j])))
+                                ++j;
+                            if (j >= cnt) {
+                                rows = false;  // a word without an exit
+                                break;
+                            }
+                            const uint64_t o = word(j);
+                            const uint32_t nc0 = (uint32_t)(o >> 32);
+                            row[(size_t)q * nent + ix] =
+                                ((uint32_t)o & 0x3Fu) | (((uint32_t)o >> 8) & 255u) << 8 | (nc0 | pos) << 16 |
+                                (nc0 | (pos ^ 1u)) << 24;
+                        }
+                }
+    }
+    if (rows) {
+        t.row.swap(row);
+    } else {
+        // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none),
+        // ranks in three 10-bit fields (511: always), for four sites per bond
+        // a fifth exit
+        const int lcb = ns <= 2 ? 2 : 3;
+        if (t.nthr <= 509 && nc <= 128 && ports <= ((size_t)1 << (8 - lcb)) && nent * 16 <= kWormExitBytes) {
+            t.exit.resize(nent);
+            for (size_t e = 0; e < nent; ++e) {
+                const WormEntry &x = t.wide[e];
+                auto narrow = [&](uint64_t w) {
+                    return (w & kWormSpecial) ? 0xFFFFu
+                                              : (uint32_t)((w >> 4) & 7u) | (uint32_t)(w >> 8 & 0xFFFFFFu) << lcb |
+                                                    (uint32_t)(w >> (32 + t.lg)) << 8;
+                };
+                uint32_t r = 0, o[4], last = 511u | 0xFFFFu << 16;
+                for (int j = 0; j < 3; ++j)
+                    r |= std::min(x.r[j], 511u) << (10 * j);
+                for (int j = 0; j < 4; ++j)
+                    o[j] = narrow(x.out[j]);
+                const auto f = fifth.find(e);
+                if (f != fifth.end()) {
+                    o[3] = narrow(f->second[1]);
+                    last = std::min((uint32_t)f->second[0], 511u) | narrow(f->second[2]) << 16;
+                }
+                t.exit[e] = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, r, last);
+            }
+        }
+    }
+    std::vector<uint16_t> bkt;
+    if (t.nthr > 8) {
+        bkt.resize(256);  // saturated where it must be: the search goes on from there
+        for (uint64_t b = 0; b < 256; ++b)
+            bkt[b] = (uint16_t)std::min<ptrdiff_t>(
+                65535, std::upper_bound(t.thr.begin(), t.thr.end(), b << 45) - t.thr.begin());
+    }
+    do
+        t.thr.push_back(~0ull);
+    while (t.thr.size() % 8);
+    if (!bkt.empty()) {
+        const size_t at = t.thr.size();
+        t.thr.resize(at + 64);
+        memcpy(t.thr.data() + at, bkt.data(), 512);
+    }
+    // sites two per word: the wave kernels take lattices far below 65536 sites
+    t.bond.resize(m.n_bonds);
+    for (int b = 0; b < m.n_bonds; ++b) {
+        uint32_t s[4] = {0, 0, 0, 0};
+        for (int k = 0; k < ns; ++k)
+            s[k] = (uint32_t)m.bond_sites[(size_t)ns * b + k];
+        t.bond[b] = make_uint4((s[0] & 0xFFFFu) | s[1] << 16, (s[2] & 0xFFFFu) | s[3] << 16,
+                               (uint32_t)base[m.bond_type[b]], 0u);
+    }
+    return nullptr;
+}

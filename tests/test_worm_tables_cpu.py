@@ -1,0 +1,181 @@
+"""The worm update's exit tables against the transition lists they are made
+from: for every vertex, worm type and leg, and for words at and beside every
+threshold, at both ends of the range and inside the tail, the exit that a table
+gives is the list's first with r < cumulative probability (vertex_data.jl:113-125).
+The tables are built by the library's own host code (csrc/worm_tables.h) and
+looked up here as the kernels do (csrc/sse_worm.h); where a table leaves a word to
+the exact search, the search is the list itself and there is nothing to compare."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from fixtures import (field_spins, job_bilayer, job_honeycomb, ladder_dimer, plaquette_ring,
+                      square_heisenberg, trimer_ring)
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+FULL, TAIL = 1 << 53, (1 << 53) - 4096
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("worm_tables") / "libworm_tables.so")
+    subprocess.run(["hipcc", "--offload-host-only", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-shared", "-w",
+                    "-o", out, os.path.join(ROOT, "tests", "worm_tables_host.cpp")], check=True)
+    lib = C.CDLL(out)
+    lib.wt_build.restype = C.c_void_p
+    lib.wt_build.argtypes = [C.c_void_p, C.POINTER(C.c_char_p)]
+    lib.wt_free.argtypes = [C.c_void_p]
+    lib.wt_info.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
+    lib.wt_image.restype = C.c_void_p
+    lib.wt_image.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_int64)]
+    return lib
+
+
+class Tables:
+    def __init__(self, host, sse, flat):
+        descs = sse.capi.ModelDescs([flat])
+        why = C.c_char_p()
+        h = host.wt_build(C.cast(descs.array, C.c_void_p), C.byref(why))
+        self.refused = why.value
+        if not self.refused:
+            info = (C.c_int64 * 4)()
+            host.wt_info(h, info)
+            self.nthr, self.lg, self.mw, self.nent = info
+
+            def image(which, dtype):
+                n = C.c_int64()
+                p = host.wt_image(h, which, C.byref(n))
+                return np.frombuffer(C.string_at(p, n.value) if n.value else b"", dtype=dtype).copy()
+
+            self.thr = image(0, np.uint64)
+            self.row = image(1, np.uint32)
+            self.exit = image(2, np.uint32).reshape(-1, 4)
+            self.wide = image(3, WIDE)
+            self.code = image(4, np.uint32).reshape(-1, 2)
+            self.bond = image(5, np.uint32).reshape(-1, 4)
+        host.wt_free(h)
+        self.ns, self.ports = flat.bond_n_sites, 2 * getattr(self, "mw", 0)
+
+    def rank(self, m):
+        return int(np.searchsorted(self.thr[:self.nthr], np.uint64(m), side="right"))
+
+    def kind(self):
+        return "rows" if len(self.row) else "exits" if len(self.exit) else "wide"
+
+    # an exit as (selector, port, new code), or None: left to the exact search
+    def rows(self, ix, m):
+        w = int(self.row[self.rank(m) * self.nent + ix])
+        return (w & 63) >> 4, (w >> 8) & 255, ((w >> 16) & 255) >> self.lg
+
+    def exits(self, ix, m):
+        x = [int(v) for v in self.exit[ix]]
+        q = self.rank(m)
+        j = sum(q >= ((x[2] >> (10 * k)) & 511) for k in range(3))
+        o = ((x[0] | x[1] << 32) >> (16 * j)) & 0xFFFF
+        if self.ns == 4 and q >= (x[3] & 0xFFFF):
+            o = x[3] >> 16
+        if m >= TAIL or o & 0x8000:
+            return None
+        lcb = 2 if self.ns <= 2 else 3
+        return o & ((1 << lcb) - 1), (o >> lcb) & ((1 << (8 - lcb)) - 1), o >> 8
+
+    def wides(self, ix, m):
+        x = self.wide[ix]
+        q = self.rank(m)
+        j = sum(q >= int(r) for r in x["r"])
+        o = int(x["out"][j])
+        if m >= TAIL or o >> 63:
+            return None
+        return (o & 127) >> 4, (o >> 8) & 0xFFFFFF, o >> (32 + self.lg)
+
+
+WIDE = np.dtype([("r", np.uint32, 3), ("pad", np.uint32), ("out", np.uint64, 4), ("tail", np.uint32, 4)])
+
+
+def k_of(c):
+    return 0 if c <= 0 else FULL if c >= 1 else -int(-(c * 2.0 ** 53) // 1)
+
+
+def words(ks, rng):
+    near = {k + d for k in ks for d in (-1, 0, 1)}
+    near |= {0, 1, FULL // 2, TAIL - 1, TAIL, TAIL + 1, FULL - 2, FULL - 1}
+    near |= {int(x) for x in rng.integers(0, FULL, size=8)}
+    return sorted(m for m in near if 0 <= m < FULL)
+
+
+def check(tab, flat):
+    """Every lookup of every table of the model; returns how many a table answered."""
+    ns, legs = tab.ns, 2 * tab.ns
+    rng = np.random.default_rng(5)
+    base = {}
+    for b in range(flat.n_bonds):
+        base[int(flat.bond_type[b])] = int(tab.bond[b][2])
+    answered = 0
+    for t, vd in enumerate(flat.types):
+        if t not in base:
+            continue
+        off = np.asarray(vd["transition_offset"]).ravel()
+        cnt = np.asarray(vd["transition_count"]).ravel()
+        cum, tgt = vd["exit_cumprob"], vd["exit_target"]
+        mw = vd["max_worm_count"]
+        for v in range(vd["n_vertices"]):
+            for wv in range(mw):
+                for leg in range(legs):
+                    src = (v * mw + wv) * legs + leg
+                    o, n = int(off[src]), int(cnt[src])
+                    if o < 0:
+                        n = 0
+                    pos, side = leg % ns, leg // ns
+                    if n == 0 and wv >= max(1, vd["dims"][pos] - 1):
+                        continue  # no worm of this type lives on the site
+                    ix = (((base[t] + v) << tab.lg) + pos) * tab.ports + 2 * wv + side
+                    ks = [k_of(cum[o + j]) for j in range(n)]
+                    for m in words(ks, rng):
+                        j = next((j for j in range(n) if m < ks[j]), None)
+                        want = None
+                        if j is not None:
+                            lo = int(vd["exit_leg"][o + j])
+                            rel, up = (lo % ns + ns - pos) % ns, lo // ns
+                            want = (rel | up << (1 if ns <= 2 else 2),
+                                    2 * (int(vd["exit_worm"][o + j]) - 1) + (up ^ 1),
+                                    base[t] + (int(tgt[o + j]) >> 1))
+                        for name in ("rows", "exits", "wides"):
+                            if name != "wides" and name != tab.kind():
+                                continue
+                            got = getattr(tab, name)(ix, m)
+                            if got is not None or name == "rows":
+                                assert got == want, (name, t, v, wv, leg, m)
+                                answered += 1
+    return answered
+
+
+def honeycomb_dz(sse):
+    """Spin-1 honeycomb with single-ion anisotropy: rows with two worm types."""
+    return sse.MagnetModel({"lattice": {"unitcell": sse.UnitCells.honeycomb, "size": (2, 2)}, "S": 1,
+                            "J": 1.0, "Dz": 0.005645, "measure": ["magnetization"]}).flat()
+
+
+MODELS = {
+    "square": (lambda sse: square_heisenberg(sse, 4, d=-0.3, hz=0.1).flat(), "rows"),
+    "honeycomb_dz": (honeycomb_dz, "rows"),
+    "field": (lambda sse: field_spins(sse, 5), None),
+    "honeycomb": (lambda sse: job_honeycomb(sse, 0.3).flat(), "exits"),
+    "ladder": (lambda sse: ladder_dimer(sse, 8, 0.6).flat(), "exits"),
+    "bilayer": (lambda sse: job_bilayer(sse, 0.2).flat(), None),
+    "trimer": (lambda sse: trimer_ring(sse, 7)[0], "exits"),
+    "plaquette": (lambda sse: plaquette_ring(sse, 9)[0], "exits"),
+}
+
+
+@pytest.mark.parametrize("name", MODELS)
+def test_tables_are_the_lists(sse_pkg, host, name):
+    make, kind = MODELS[name]
+    flat = make(sse_pkg)
+    tab = Tables(host, sse_pkg, flat)
+    assert not tab.refused
+    if kind:
+        assert tab.kind() == kind
+    assert check(tab, flat) > 0
