@@ -114,9 +114,10 @@ struct WormRank {
 };
 
 // ------------------------------------------------------------------ exit tables
-// A word within kWormTail of 2^53 is marked in its row's top bit and looked up
-// exactly, so that a table whose last cumulative probability misses 1 by rounding
-// still has an exit for every other word.
+// A word from kWormTail on is marked in its row's top bit and looked up exactly, so
+// that a table whose last cumulative probability misses 1 by rounding still has an
+// exit for every other word.  Exit rows mark nothing: they are built only where no
+// threshold but 1 lies in the tail.
 __device__ __forceinline__ uint32_t worm_tail_bit(uint64_t m) { return m >= kWormTail ? 0x80000000u : 0u; }
 
 // A table gives for an entry's word and the step's row, in two parts so that the

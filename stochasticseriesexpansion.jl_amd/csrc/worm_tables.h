@@ -162,8 +162,13 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
                         if (ns == 4 && cnt == 5 && rank(thr(vd.exit_cumprob[off + 4])) == 0xFFFFFFFFu)
                             fifth[ix] = {r3, word(3), word(4)};
                     }
-                    if (cnt > 0)
-                        rows = rows && thr(vd.exit_cumprob[off + cnt - 1]) == (1ull << 53);
+                    // rows have no exact search behind them: the list has to
+                    // end at 1, and no word of the tail (rank() takes its
+                    // thresholds for 1) may belong to another exit
+                    for (int j = 0; j < cnt; ++j) {
+                        const uint64_t k = thr(vd.exit_cumprob[off + j]);
+                        rows = rows && (k == (1ull << 53) || (j + 1 < cnt && k < kWormTail));
+                    }
                     if (rows)
                         for (int q = 0; q <= t.nthr && rows; ++q) {
                             int j = 0;

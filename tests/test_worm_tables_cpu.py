@@ -158,6 +158,27 @@ def honeycomb_dz(sse):
                             "J": 1.0, "Dz": 0.005645, "measure": ["magnetization"]}).flat()
 
 
+def with_list(flat, n, change):
+    """flat with the first transition of n exits replaced: change(cumulative
+    probabilities) edits them in place; None takes the transition out."""
+    vd = dict(flat.types[0])
+    for key in ("transition_offset", "transition_count", "exit_cumprob"):
+        vd[key] = np.array(vd[key], copy=True)
+    cnt = vd["transition_count"].reshape(-1)
+    i = int(np.nonzero((cnt == n) & (vd["transition_offset"].reshape(-1) >= 0))[0][0])
+    o = int(vd["transition_offset"].reshape(-1)[i])
+    if change is None:
+        vd["transition_offset"].reshape(-1)[i] = -1
+    else:
+        change(vd["exit_cumprob"][o:o + n])
+    flat.types = [vd] + list(flat.types[1:])
+    return flat
+
+
+def inner_tail(c):
+    c[-2], c[-1] = 1.0 - 2.0 ** -50, 1.0
+
+
 MODELS = {
     "square": (lambda sse: square_heisenberg(sse, 4, d=-0.3, hz=0.1).flat(), "rows"),
     "honeycomb_dz": (honeycomb_dz, "rows"),
@@ -179,3 +200,11 @@ def test_tables_are_the_lists(sse_pkg, host, name):
     if kind:
         assert tab.kind() == kind
     assert check(tab, flat) > 0
+
+
+@pytest.mark.parametrize("name,n", [("square", 2), ("honeycomb_dz", 3)])
+def test_inner_threshold_in_the_tail(sse_pkg, host, name, n):
+    """An exit of probability 2^-50 behind the others: words past its threshold
+    lie in the tail that exit rows do not look up exactly."""
+    flat = with_list(MODELS[name][0](sse_pkg), n, inner_tail)
+    check(Tables(host, sse_pkg, flat), flat)
