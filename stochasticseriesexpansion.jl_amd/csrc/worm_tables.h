@@ -127,6 +127,16 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
                 (size_t)(t.nthr + 1) * nent * 4 <= kWormRowBytes;
     std::map<size_t, std::array<uint64_t, 3>> fifth;  // fourth rank, exits 3 and 4
     std::vector<uint32_t> row(rows ? (size_t)(t.nthr + 1) * nent : 0, 0u);
+    // A site of dimension d starts worms of max(d - 1, 1) types; an exit into
+    // another type than its leg's site has makes all types possible.  Rows do not
+    // see that a bond type has no list for a worm.
+    bool foreign = false;
+    for (int i : rep)
+        for (int e = 0; e < m.types[i].n_exits; ++e)
+            foreign |= m.types[i].exit_worm[e] > std::max(1, m.types[i].dims[m.types[i].exit_leg[e] % ns] - 1);
+    for (int i : rep)
+        for (int k = 0; k < ns; ++k)
+            rows = rows && (foreign ? t.mw : std::max(1, m.types[i].dims[k] - 1)) <= m.types[i].max_worm_count;
     for (int i : rep) {
         const sse_vertex_data_desc &vd = m.types[i];
         for (int v = 0; v < vd.n_vertices; ++v)

@@ -122,10 +122,10 @@ def check(tab, flat):
         cum, tgt = vd["exit_cumprob"], vd["exit_target"]
         mw = vd["max_worm_count"]
         for v in range(vd["n_vertices"]):
-            for wv in range(mw):
+            for wv in range(tab.mw):
                 for leg in range(legs):
                     src = (v * mw + wv) * legs + leg
-                    o, n = int(off[src]), int(cnt[src])
+                    o, n = (int(off[src]), int(cnt[src])) if wv < mw else (-1, 0)
                     if o < 0:
                         n = 0
                     pos, side = leg % ns, leg // ns
@@ -208,3 +208,37 @@ def test_inner_threshold_in_the_tail(sse_pkg, host, name, n):
     lie in the tail that exit rows do not look up exactly."""
     flat = with_list(MODELS[name][0](sse_pkg), n, inner_tail)
     check(Tables(host, sse_pkg, flat), flat)
+
+
+@pytest.mark.parametrize("name", ["square", "honeycomb_dz"])
+def test_missing_transition(sse_pkg, host, name):
+    """A vertex and leg without a transition list: the worm that gets there is an
+    error of the chain, which the exact search reports; no table may answer."""
+    for n in (1, 2, 3):
+        flat = MODELS[name][0](sse_pkg)
+        if (np.asarray(flat.types[0]["transition_count"]) == n).any():
+            flat = with_list(flat, n, None)
+            check(Tables(host, sse_pkg, flat), flat)
+
+
+def test_bond_type_without_a_worm_type(sse_pkg, host):
+    """Two bond types of one vertex whose worms only bounce, on spin-1 sites that
+    hold two worm types; the second knows one.  The other worm's arrival there is
+    an error as well."""
+    flat = square_heisenberg(sse_pkg, 4).flat()
+
+    def bounce(mw):
+        n = mw * 4
+        return dict(flat.types[0], dims=(3, 3), n_vertices=1, leg_states=np.ones((1, 4), np.uint8),
+                    weights=np.ones(1), signs=np.ones(1, np.int8), diagonal_vertices=-np.ones(9, np.int32),
+                    max_worm_count=mw, transition_offset=np.arange(n), transition_count=np.ones(n, np.int32),
+                    n_exits=n, exit_cumprob=np.ones(n), exit_target=np.ones(n, np.int32),
+                    exit_leg=np.arange(n) % 4, exit_worm=np.arange(n) // 4 + 1)
+
+    flat.types = [bounce(2), bounce(1)]
+    flat.bond_type = np.arange(flat.n_bonds) % 2
+    flat.site_dims = np.full(flat.n_sites, 3, np.uint8)
+    check(Tables(host, sse_pkg, flat), flat)
+    flat.types = [bounce(2), bounce(2)]
+    tab = Tables(host, sse_pkg, flat)
+    assert tab.kind() == "rows" and check(tab, flat) > 0
