@@ -199,7 +199,8 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
     if (rows) {
         t.row.swap(row);
     } else {
-        // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none),
+        // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none, with
+        // selector and port 0, which the step follows before it sees the bit),
         // ranks in three 10-bit fields (511: always), for four sites per bond
         // a fifth exit
         const int lcb = ns <= 2 ? 2 : 3;
@@ -208,11 +209,11 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
             for (size_t e = 0; e < nent; ++e) {
                 const WormEntry &x = t.wide[e];
                 auto narrow = [&](uint64_t w) {
-                    return (w & kWormSpecial) ? 0xFFFFu
+                    return (w & kWormSpecial) ? 0x8000u
                                               : (uint32_t)((w >> 4) & 7u) | (uint32_t)(w >> 8 & 0xFFFFFFu) << lcb |
                                                     (uint32_t)(w >> (32 + t.lg)) << 8;
                 };
-                uint32_t r = 0, o[4], last = 511u | 0xFFFFu << 16;
+                uint32_t r = 0, o[4], last = 511u | 0x8000u << 16;
                 for (int j = 0; j < 3; ++j)
                     r |= std::min(x.r[j], 511u) << (10 * j);
                 for (int j = 0; j < 4; ++j)

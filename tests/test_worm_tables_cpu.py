@@ -242,3 +242,19 @@ def test_bond_type_without_a_worm_type(sse_pkg, host):
     flat.types = [bounce(2), bounce(2)]
     tab = Tables(host, sse_pkg, flat)
     assert tab.kind() == "rows" and check(tab, flat) > 0
+
+
+@pytest.mark.parametrize("name", ["honeycomb", "ladder", "trimer", "plaquette"])
+def test_word_of_a_missing_exit(sse_pkg, host, name):
+    """The step loads the entry and table word behind an exit before it sees that
+    there is none: the missing exit's word has to name a leg and a port that exist."""
+    flat = MODELS[name][0](sse_pkg)
+    tab = Tables(host, sse_pkg, flat)
+    assert tab.kind() == "exits"
+    lcb = 2 if tab.ns <= 2 else 3
+    words = np.concatenate([tab.exit[:, 0] & 0xFFFF, tab.exit[:, 0] >> 16, tab.exit[:, 1] & 0xFFFF,
+                            tab.exit[:, 1] >> 16] + ([tab.exit[:, 3] >> 16] if tab.ns == 4 else []))
+    none = words[(words & 0x8000) != 0]
+    assert len(none)
+    assert ((none & ((1 << (lcb - 1)) - 1)) < tab.ns).all()
+    assert ((none >> lcb & ((1 << (8 - lcb)) - 1)) < tab.ports).all()
