@@ -334,7 +334,7 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     }
     std::vector<char> blob;
     auto put = [&](const void *src, size_t bytes) {
-        size_t off = (blob.size() + 15) & ~(size_t)15;
+        size_t off = (blob.size() + 63) & ~(size_t)63;
         blob.resize(off + bytes + 16);
         if (bytes)
             memcpy(blob.data() + off, src, bytes);
@@ -589,7 +589,7 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     dm.wcode = (const uint2 *)(d + o_wcode);
     dm.wthr = (const uint64_t *)(d + o_wthr);
     dm.wrow = wt.row.empty() ? nullptr : (const uint32_t *)(d + o_wrow);
-    dm.w_rank = wt.nthr > 8 ? (int32_t)(8 * wt.thr.size()) : 0;
+    dm.w_rank = wt.rank;
     dm.pad_w = 0;
     dm.wexit = wt.exit.empty() ? nullptr : (const uint4 *)(d + o_wexit);
     dm.wwide = (const WormEntry *)(d + o_wwide);

@@ -58,11 +58,11 @@ struct DevModel {
     const uint4 *wbond;        // [n_bonds] sites two per word (u16), code base, 0
     const uint2 *wcode;        // [w_ncode] lower leg states, one byte per site; vcode | type << 10
     // distinct exit thresholds, ascending, ended by ~0 and padded to a multiple of
-    // 8; then (above 8 thresholds) u16[256], the thresholds <= bucket << 45
+    // 8; then (above 8, with one of the next two) u16[256], thresholds <= bucket << 45
     const uint64_t *wthr;
     const uint32_t *wrow;      // exit rows (null: too large, or some word has no exit)
     const uint4 *wexit;        // 16-byte exit entries (null: too many codes or thresholds)
-    const struct WormEntry *wwide;  // exit entries of any table
+    const struct WormEntry *wwide;  // exit entries of any table, 64-byte aligned
     int32_t w_ncode, w_lg, w_nthr, w_mw;
     int32_t w_nent;            // exit entries: ((w_ncode << w_lg) + 1) * 2 * w_mw
     int32_t w_dim;             // local dimension of every site, 0 when they differ
@@ -103,12 +103,21 @@ struct DevModel {
 // c * 2 * w_mw + 2 * (worm - 1) + side.  Its exit word names the leg relative
 // to the entering site, the port 2 * (worm - 1) + side with which the worm
 // enters the next operator, and the new vertex code.
-struct __align__(16) WormEntry {
-    uint32_t r[3];     // exit j < 3: the first with q < r[j] (r ascending); else exit 3
+struct __align__(32) WormEntry {
+    // exit j < 3: the first with the word's top 32 bits below r[j] (ascending; ~0:
+    // always), else exit 3.  Equal top bits are looked up exactly.
+    uint32_t r[3];
+    // selector << 4 in bits 0..6, port in 7..19, new vertex - old one in 20..30
+    // (two's complement); bit 31 alone: no exit here (worm_exact)
+    uint32_t out[4];
     uint32_t pad;
-    uint64_t out[4];   // worm_word(), or kWormSpecial: no exit here (see worm_exact)
-    uint32_t tail[4];
 };
+__host__ __device__ inline uint32_t worm_entry_word(uint32_t leg, uint32_t port, int step)
+{
+    return leg << 4 | port << 7 | ((uint32_t)step & 0x7FFu) << 20;
+}
+__host__ __device__ inline uint32_t worm_entry_port(uint32_t o) { return (o >> 7) & 0x1FFFu; }
+__host__ __device__ inline int32_t worm_entry_step(uint32_t o) { return (int32_t)(o << 1) >> 21; }
 #define kWormSpecial (1ull << 63)
 // words (of 53 bits) from here on are looked up exactly
 constexpr uint64_t kWormTail = (1ull << 53) - 4096u;

@@ -45,6 +45,9 @@ typedef __attribute__((address_space(3))) uint64_t lds_u64;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 typedef const __attribute__((address_space(4))) uint64_t const_u64;
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+typedef const __attribute__((address_space(4))) u32x8 const_u32x8;
+typedef const __attribute__((address_space(4))) uint8_t const_u8;
 
 // LDS by byte address: entry ids and table rows are addresses, so that the step
 // adds no base
@@ -72,16 +75,15 @@ __device__ __forceinline__ uint32_t rdlane(uint32_t v, uint32_t l)
 __device__ __forceinline__ bool wave_any(bool x) { return __builtin_amdgcn_ballot_w64(x) != 0ull; }
 
 // ------------------------------------------------------------------ ranks
-// q = number of the model's thresholds that are <= m.  Up to 8: compared one by
-// one against scalar operands.  More: a 256-bucket start by the mantissa's top
-// bits, then the bucket's own thresholds, few as a rule; from the LDS copy of
-// DevModel::wthr (behind the exit table) or, with a table in global memory, there.
-// In LDS the 64 ranks of a buffer of words take some 300 cycles for 25-35
-// thresholds; from global memory, and by comparing all, 1500-3000.
+// q = number of the model's thresholds that are <= m, for the tables in LDS.  Up to
+// 8: compared one by one against scalar operands.  More: a 256-bucket start by the
+// mantissa's top bits, then the bucket's own thresholds, few as a rule; from the LDS
+// copy of DevModel::wthr behind the exit table.  The 64 ranks of a buffer of words
+// take some 300 cycles for 25-35 thresholds, by comparing all 1500-3000.
 struct WormRank {
     const uint64_t *thr;
     int n;
-    uint32_t lds;  // byte address of the LDS copy, ~0: none
+    uint32_t lds;  // byte address of the LDS copy (n > 8)
     __device__ __forceinline__ uint32_t of(uint64_t m) const
     {
         uint32_t q = 0;
@@ -93,19 +95,9 @@ struct WormRank {
             return q;
         }
         const uint32_t pad = ((uint32_t)n + 8u) & ~7u;  // entries ahead of the buckets
-        if (lds != ~0u) {
-            q = *lds_at<lds_u16>(lds + 8u * pad + 2u * (uint32_t)(m >> 45));
-            for (;;) {
-                const bool up = *lds_at<lds_u64>(lds + 8u * q) <= m;  // ~0 ends the list
-                if (!wave_any(up))
-                    return q;
-                q += up ? 1u : 0u;
-            }
-        }
-        const gmem<uint64_t> *t = as_global(thr);
-        q = ((const gmem<uint16_t> *)(t + pad))[m >> 45];
+        q = *lds_at<lds_u16>(lds + 8u * pad + 2u * (uint32_t)(m >> 45));
         for (;;) {
-            const bool up = t[q] <= m;
+            const bool up = *lds_at<lds_u64>(lds + 8u * q) <= m;  // ~0 ends the list
             if (!wave_any(up))
                 return q;
             q += up ? 1u : 0u;
@@ -136,7 +128,7 @@ struct WormExit {
 // compare at all is left in the step.
 template <int NS>
 struct TabRows {
-    static constexpr bool kNone = false;
+    static constexpr bool kNone = false, kScalar = false;
     WormRank rank;
     uint32_t base, rowbytes, ports;  // ports: 2 * worm types
     typedef uint32_t Word;
@@ -171,7 +163,7 @@ struct TabRows {
 // <= q, which is the exit's index.
 template <int NS>
 struct TabExits {
-    static constexpr bool kNone = true;
+    static constexpr bool kNone = true, kScalar = false;
     static constexpr uint32_t kGuards = 1u << 9 | 1u << 19 | 1u << 29;
     WormRank rank;
     uint32_t base, ports;  // ports: 2 * worm types
@@ -214,37 +206,46 @@ struct TabExits {
     }
 };
 
-// WormEntry in global memory: any number of codes, worm types and thresholds.
+// WormEntry in global memory: any number of codes, worm types and thresholds.  The
+// table is constant, and one load to the scalar unit brings a whole entry; a word is
+// compared by its top 32 bits against the entry's own thresholds, so that no rank is
+// needed, however many bond types a model has.  Where they are equal (2^-32 a
+// compare) and in the tail the exact search decides.  Against ranks searched in global
+// memory and entries of 64 bytes selected through scratch, a step of an XXZ square in
+// a field took, by number of different bonds: 32 320 -> 170 ns, 512 401 -> 181 ns.
 template <int NS>
 struct TabWide {
-    static constexpr bool kNone = true;
-    WormRank rank;
+    static constexpr bool kNone = true, kScalar = true;
     uint32_t ports;
     const WormEntry *t;
-    struct Word {
-        u32x4 r;
-        uint64_t o0, o1, o2, o3;
-    };
-    __device__ __forceinline__ uint32_t row_of(uint64_t m) const { return rank.of(m) | worm_tail_bit(m); }
+    typedef u32x8 Word;
+    __device__ __forceinline__ uint32_t row_of(uint64_t m) const { return (uint32_t)(m >> 21); }
     __device__ __forceinline__ Word load(uint32_t, uint32_t c, uint32_t port) const
     {
-        const gmem<WormEntry> *e = as_global(t) + ((size_t)c * ports + port);
-        return Word{u32x4{e->r[0], e->r[1], e->r[2], 0u}, e->out[0], e->out[1], e->out[2], e->out[3]};
+        // below 4 GB: a 32-bit offset goes into the load instruction
+        const uint32_t at = (uni(c) * ports + uni(port)) * (uint32_t)sizeof(WormEntry);
+        return *(const_u32x8 *)((const_u8 *)(const void *)t + at);
     }
-    typedef uint64_t Pick;
-    __device__ __forceinline__ Pick pick(const Word &w, uint32_t row) const
+    __device__ __forceinline__ static uint32_t unsure(Word w, uint32_t row)
     {
-        return row < w.r.x ? w.o0 : row < w.r.y ? w.o1 : row < w.r.z ? w.o2 : w.o3;
+        return row == w.s0 || row == w.s1 || row == w.s2 || row == ~0u ? 0x80000000u : 0u;
     }
-    __device__ __forceinline__ static uint32_t sh(Pick o) { return (uint32_t)o; }
+    typedef uint32_t Pick;
+    __device__ __forceinline__ Pick pick(Word w, uint32_t row) const
+    {
+        uint32_t o = row < w.s2 ? w.s5 : w.s6;
+        o = row < w.s1 ? w.s4 : o;
+        return row < w.s0 ? w.s3 : o;
+    }
+    __device__ __forceinline__ static uint32_t sh(Pick o) { return o; }
     __device__ __forceinline__ WormExit<NS> exit(Pick o, uint32_t c) const
     {
         constexpr int LG = WormNS<NS>::LG;
         WormExit<NS> x;
-        x.port = (uint32_t)o >> 8;
-        x.none = (uint32_t)(o >> 32);
-        const uint32_t nc = x.none;
+        x.port = worm_entry_port(o);
+        x.none = o;
         uint32_t pos = c & ((1u << LG) - 1u);
+        const uint32_t nc = c - pos + ((uint32_t)worm_entry_step(o) << LG);
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
             x.c[k] = nc | pos;
@@ -783,6 +784,11 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
             uint32_t off = uni(rs.off);
             row = uni(row);
             uint32_t q[NS], cq, pq, rq, none, ends;
+            bool stop;
+            // scalar loads return out of order: with one in flight from before the
+            // loop, its first instruction would wait for the table in every step
+            if constexpr (T::kScalar)
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
             do {
                 q[0] = e;
                 if constexpr (NS > 1)
@@ -793,7 +799,7 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
                 const WormHop<NS, R::kGlobal> hop(q);
                 cq = c;
                 pq = port;
-                rq = row;
+                rq = T::kScalar ? 0u : row;
                 // the exit's own chain starts here, with all that does not
                 // need it done under its load
                 __builtin_amdgcn_sched_barrier(0);
@@ -814,21 +820,33 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
                 c = rec.code(nx);
                 pt = rec.part(nx);
                 __builtin_amdgcn_sched_barrier(0);
+                if constexpr (T::kScalar)
+                    rq = T::unsure(wd, row);
                 const WormExit<NS> ex = tab.exit(pick, cq);
                 none = ex.none;
-#pragma unroll
-                for (int j = 0; j < NS; ++j)
-                    rec.set_code(q[j], ex.c[j]);
                 off += 1u;
                 e = nx;
                 port = ex.port;
                 row = rdlane(rs.row, off & 63u);
-                wd = tab.load(row, c, port);
                 // one condition, one branch: a flag, no exit, or no word left
                 ends = (63u - off) | (T::kNone ? rq : 0u);
                 if constexpr (T::kNone)
                     ends |= none;
-            } while (!wave_any((int32_t)((uint32_t)pt | ends) < 0));
+                // a wait for LDS is a wait for the scalar load too, so that one
+                // leaves after the test of the flag
+                if constexpr (T::kScalar) {
+                    stop = wave_any((int32_t)((uint32_t)pt | ends) < 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    wd = tab.load(row, c, port);
+                }
+#pragma unroll
+                for (int j = 0; j < NS; ++j)
+                    rec.set_code(q[j], ex.c[j]);
+                if constexpr (!T::kScalar) {
+                    wd = tab.load(row, c, port);
+                    stop = wave_any((int32_t)((uint32_t)pt | ends) < 0);
+                }
+            } while (!stop);
             rs.off = off;
             if constexpr (T::kNone) {
                 if (__builtin_expect(wave_any((int32_t)(none | rq) < 0), 0)) {
@@ -1123,7 +1141,7 @@ __device__ __forceinline__ void worm_walker(DevWalker *W, const DevModel *models
     const uint32_t poff = pbase - 2u * id0;
     if (in_lds)
         x.sb = lds_at<lds_u16>(pbase + 2u * (uint32_t)E);
-    const TabWide<NS> wide{rank, ports, m.wwide};
+    const TabWide<NS> wide{ports, m.wwide};
     const bool rows = NS <= 2 && m.wrow != nullptr;
 #define WORM_RUN(R, T) err = worm_update<NS>(w, m, x, R, T, total, scat, ctr)
     if (in_lds && tb) {

@@ -2,7 +2,6 @@
 // sse_worm.h reads, from the transition lists of a model.
 #pragma once
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstddef>
 #include <cstdint>
@@ -23,7 +22,7 @@ struct WormTables {
     std::vector<uint32_t> row;
     std::vector<uint4> exit;
     std::vector<WormEntry> wide;
-    int nthr = 0, lg = 0, mw = 1, dim = 0;
+    int nthr = 0, lg = 0, mw = 1, dim = 0, rank = 0;
 };
 
 // Exit rows take LDS beside every walker's records, which the step without a
@@ -98,7 +97,7 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
     }
     const size_t nc = t.code.size(), ports = 2 * (size_t)t.mw;
     const size_t nent = ((nc << t.lg) + 1) * ports;
-    if (nent >= ((size_t)1 << 30))
+    if (nent * sizeof(WormEntry) >= ((size_t)1 << 32))  // the kernel's offsets have 32 bits
         return "too many worm table entries";
     for (int i : rep) {
         const sse_vertex_data_desc &vd = m.types[i];
@@ -117,15 +116,17 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
                                  : (uint32_t)(std::lower_bound(t.thr.begin(), t.thr.begin() + t.nthr, k) -
                                               t.thr.begin()) + 1u;
     };
-    WormEntry none;
-    memset(&none, 0, sizeof none);
-    none.r[0] = none.r[1] = none.r[2] = 0xFFFFFFFFu;
-    for (int j = 0; j < 4; ++j)
-        none.out[j] = kWormSpecial;
-    t.wide.assign(nent, none);
+    const uint32_t always = 0xFFFFFFFFu;
+    t.wide.assign(nent, WormEntry{{always, always, always}, {1u << 31, 1u << 31, 1u << 31, 1u << 31}, 0u});
+    // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none, with
+    // selector and port 0, which the step follows before it sees the bit), ranks in
+    // three 10-bit fields (511: always), for four sites per bond a fifth exit
+    const int lcb = ns <= 2 ? 2 : 3;
+    const bool small = t.nthr <= 509 && nc <= 128 && ports <= ((size_t)1 << (8 - lcb)) && nent * 16 <= kWormExitBytes;
+    const uint4 none = make_uint4(0x80008000u, 0x80008000u, 511u | 511u << 10 | 511u << 20, 511u | 0x8000u << 16);
+    std::vector<uint4> exits(small ? nent : 0, none);
     bool rows = ns <= 2 && ports <= 128 && (nc << t.lg) <= 255 &&
                 (size_t)(t.nthr + 1) * nent * 4 <= kWormRowBytes;
-    std::map<size_t, std::array<uint64_t, 3>> fifth;  // fourth rank, exits 3 and 4
     std::vector<uint32_t> row(rows ? (size_t)(t.nthr + 1) * nent : 0, 0u);
     // A site of dimension d starts worms of max(d - 1, 1) types; an exit into
     // another type than its leg's site has makes all types possible.  Rows do not
@@ -146,93 +147,74 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
                     const int off = vd.transition_offset[src], cnt = off < 0 ? 0 : vd.transition_count[src];
                     const uint32_t pos = (uint32_t)(l % ns), side = (uint32_t)(l / ns);
                     const size_t ix = ((((size_t)base[i] + v) << t.lg) + pos) * ports + 2 * (size_t)wv + side;
-                    WormEntry &x = t.wide[ix];
-                    auto word = [&](int j) {
-                        const uint32_t lo = vd.exit_leg[off + j], up = lo >= (uint32_t)ns;
-                        return worm_word(worm_leg(ns, pos, lo),
-                                         2u * ((uint32_t)vd.exit_worm[off + j] - 1u) + (up ^ 1u),
-                                         ((uint32_t)base[i] + ((uint32_t)vd.exit_target[off + j] >> 1)) << t.lg);
+                    const auto cum = [&](int j) { return thr(vd.exit_cumprob[off + j]); };
+                    // leg selector, port behind the exit, new vertex
+                    const auto leg = [&](int j) { return worm_leg(ns, pos, vd.exit_leg[off + j]); };
+                    const auto port = [&](int j) {
+                        return 2u * ((uint32_t)vd.exit_worm[off + j] - 1u) + (vd.exit_leg[off + j] < ns ? 1u : 0u);
                     };
-                    // exit 3 stands for every word past the first three
-                    // thresholds: the fourth exit if it ends the list at 1,
-                    // else none (the exact search decides)
-                    for (int j = 0; j < 3 && j < cnt; ++j) {
-                        x.r[j] = rank(thr(vd.exit_cumprob[off + j]));
-                        if (j && x.r[j] < x.r[j - 1])
-                            x.r[j] = x.r[j - 1];
-                        x.out[j] = word(j);
+                    const auto vertex = [&](int j) { return vd.exit_target[off + j] >> 1; };
+                    const auto code = [&](int j) { return (uint32_t)(base[i] + vertex(j)); };
+                    // exits and thresholds 0..2; exit 3 stands for every word past
+                    // the third threshold: the fourth exit if it ends the list at
+                    // 1, else none (the exact search decides)
+                    const int ends = cnt == 4 && cum(3) >= kWormTail ? 4 : std::min(cnt, 3);
+                    WormEntry &x = t.wide[ix];
+                    uint32_t r[3] = {511u, 511u, 511u}, o[5] = {0x8000u, 0x8000u, 0x8000u, 0x8000u, 0x8000u};
+                    const auto narrow = [&](int j) { return leg(j) | port(j) << lcb | code(j) << 8; };
+                    for (int j = 0; j < ends; ++j) {
+                        x.out[j] = worm_entry_word(leg(j), port(j), vertex(j) - v);
+                        if (small)
+                            o[j] = narrow(j);
+                        if (j < 3) {
+                            x.r[j] = cum(j) >= kWormTail ? always : (uint32_t)(cum(j) >> 21);
+                            r[j] = std::min(rank(cum(j)), 511u);
+                        }
+                        if (j > 0 && j < 3) {
+                            x.r[j] = std::max(x.r[j], x.r[j - 1]);
+                            r[j] = std::max(r[j], r[j - 1]);
+                        }
                     }
-                    if (cnt > 0 && cnt < 3)  // past the last exit: none
-                        for (int j = cnt; j < 3; ++j)
-                            x.r[j] = 0xFFFFFFFFu;
-                    if (cnt >= 4) {
-                        const uint32_t r3 = rank(thr(vd.exit_cumprob[off + 3]));
-                        if (cnt == 4 && r3 == 0xFFFFFFFFu)
-                            x.out[3] = word(3);
-                        if (ns == 4 && cnt == 5 && rank(thr(vd.exit_cumprob[off + 4])) == 0xFFFFFFFFu)
-                            fifth[ix] = {r3, word(3), word(4)};
+                    if (small) {
+                        uint32_t r3 = 511u;
+                        if (ns == 4 && cnt == 5 && cum(4) >= kWormTail) {
+                            r3 = std::min(rank(cum(3)), 511u);
+                            o[3] = narrow(3);
+                            o[4] = narrow(4);
+                        }
+                        exits[ix] = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, r[0] | r[1] << 10 | r[2] << 20,
+                                               r3 | o[4] << 16);
                     }
                     // rows have no exact search behind them: the list has to
                     // end at 1, and no word of the tail (rank() takes its
                     // thresholds for 1) may belong to another exit
                     for (int j = 0; j < cnt; ++j) {
-                        const uint64_t k = thr(vd.exit_cumprob[off + j]);
-                        rows = rows && (k == (1ull << 53) || (j + 1 < cnt && k < kWormTail));
+                        rows = rows && (cum(j) == (1ull << 53) || (j + 1 < cnt && cum(j) < kWormTail));
                     }
                     if (rows)
                         for (int q = 0; q <= t.nthr && rows; ++q) {
                             int j = 0;
-                            while (j < cnt && (uint32_t)q >= rank(thr(vd.exit_cumprob[off + j])))
+                            while (j < cnt && (uint32_t)q >= rank(cum(j)))
                                 ++j;
                             if (j >= cnt) {
                                 rows = false;  // a word without an exit
                                 break;
                             }
-                            const uint64_t o = word(j);
-                            const uint32_t nc0 = (uint32_t)(o >> 32);
+                            const uint32_t nc0 = code(j) << t.lg;
                             row[(size_t)q * nent + ix] =
-                                ((uint32_t)o & 0x3Fu) | (((uint32_t)o >> 8) & 255u) << 8 | (nc0 | pos) << 16 |
-                                (nc0 | (pos ^ 1u)) << 24;
+                                leg(j) << 4 | port(j) << 8 | (nc0 | pos) << 16 | (nc0 | (pos ^ 1u)) << 24;
                         }
                 }
     }
-    if (rows) {
+    if (rows)
         t.row.swap(row);
-    } else {
-        // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none, with
-        // selector and port 0, which the step follows before it sees the bit),
-        // ranks in three 10-bit fields (511: always), for four sites per bond
-        // a fifth exit
-        const int lcb = ns <= 2 ? 2 : 3;
-        if (t.nthr <= 509 && nc <= 128 && ports <= ((size_t)1 << (8 - lcb)) && nent * 16 <= kWormExitBytes) {
-            t.exit.resize(nent);
-            for (size_t e = 0; e < nent; ++e) {
-                const WormEntry &x = t.wide[e];
-                auto narrow = [&](uint64_t w) {
-                    return (w & kWormSpecial) ? 0x8000u
-                                              : (uint32_t)((w >> 4) & 7u) | (uint32_t)(w >> 8 & 0xFFFFFFu) << lcb |
-                                                    (uint32_t)(w >> (32 + t.lg)) << 8;
-                };
-                uint32_t r = 0, o[4], last = 511u | 0x8000u << 16;
-                for (int j = 0; j < 3; ++j)
-                    r |= std::min(x.r[j], 511u) << (10 * j);
-                for (int j = 0; j < 4; ++j)
-                    o[j] = narrow(x.out[j]);
-                const auto f = fifth.find(e);
-                if (f != fifth.end()) {
-                    o[3] = narrow(f->second[1]);
-                    last = std::min((uint32_t)f->second[0], 511u) | narrow(f->second[2]) << 16;
-                }
-                t.exit[e] = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, r, last);
-            }
-        }
-    }
+    else
+        t.exit.swap(exits);
     std::vector<uint16_t> bkt;
-    if (t.nthr > 8) {
-        bkt.resize(256);  // saturated where it must be: the search goes on from there
+    if (t.nthr > 8 && (!t.row.empty() || !t.exit.empty())) {  // the wide table needs no ranks
+        bkt.resize(256);
         for (uint64_t b = 0; b < 256; ++b)
-            bkt[b] = (uint16_t)std::min<ptrdiff_t>(
-                65535, std::upper_bound(t.thr.begin(), t.thr.end(), b << 45) - t.thr.begin());
+            bkt[b] = (uint16_t)(std::upper_bound(t.thr.begin(), t.thr.end(), b << 45) - t.thr.begin());
     }
     do
         t.thr.push_back(~0ull);
@@ -241,6 +223,7 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
         const size_t at = t.thr.size();
         t.thr.resize(at + 64);
         memcpy(t.thr.data() + at, bkt.data(), 512);
+        t.rank = (int)(8 * t.thr.size());
     }
     // sites two per word: the wave kernels take lattices far below 65536 sites
     t.bond.resize(m.n_bonds);

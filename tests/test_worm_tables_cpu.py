@@ -83,16 +83,18 @@ class Tables:
         return o & ((1 << lcb) - 1), (o >> lcb) & ((1 << (8 - lcb)) - 1), o >> 8
 
     def wides(self, ix, m):
-        x = self.wide[ix]
-        q = self.rank(m)
-        j = sum(q >= int(r) for r in x["r"])
+        x, w = self.wide[ix], m >> 21
+        r = [int(v) for v in x["r"]]
+        j = next((k for k in range(3) if w < r[k]), 3)
         o = int(x["out"][j])
-        if m >= TAIL or o >> 63:
+        if w in r or w == 0xFFFFFFFF or o >> 31:
             return None
-        return (o & 127) >> 4, (o >> 8) & 0xFFFFFF, o >> (32 + self.lg)
+        step = (o >> 20) & 0x7FF
+        code = (ix // self.ports) >> self.lg
+        return (o & 127) >> 4, (o >> 7) & 0x1FFF, code + (step - 2048 if step >= 1024 else step)
 
 
-WIDE = np.dtype([("r", np.uint32, 3), ("pad", np.uint32), ("out", np.uint64, 4), ("tail", np.uint32, 4)])
+WIDE = np.dtype([("r", np.uint32, 3), ("out", np.uint32, 4), ("pad", np.uint32)])
 
 
 def k_of(c):
@@ -100,7 +102,7 @@ def k_of(c):
 
 
 def words(ks, rng):
-    near = {k + d for k in ks for d in (-1, 0, 1)}
+    near = {k + d for k in ks for d in (-1 << 22, -1 << 21, -1, 0, 1, 1 << 21, 1 << 22)}
     near |= {0, 1, FULL // 2, TAIL - 1, TAIL, TAIL + 1, FULL - 2, FULL - 1}
     near |= {int(x) for x in rng.integers(0, FULL, size=8)}
     return sorted(m for m in near if 0 <= m < FULL)
@@ -179,6 +181,42 @@ def inner_tail(c):
     c[-2], c[-1] = 1.0 - 2.0 ** -50, 1.0
 
 
+def random_bonds(sse, n):
+    """An XXZ square in a field whose bonds have n different anisotropies."""
+    parts = [square_heisenberg(sse, 4, d=-0.3 + 0.6 * k / n, hz=0.1).flat() for k in range(n)]
+    flat = parts[0]
+    flat.types = [p.types[0] for p in parts]
+    flat.bond_type = np.arange(flat.n_bonds) % n
+    return flat
+
+
+def trimer_split(sse):
+    """The three-site ring with the last exit of every list of four cut in three:
+    six exits with the same outcomes, beyond what an entry holds."""
+    flat = trimer_ring(sse, 7)[0]
+    vd = dict(flat.types[0])
+    off = np.array(vd["transition_offset"]).reshape(-1)
+    cnt = np.array(vd["transition_count"]).reshape(-1)
+    keys = ("exit_cumprob", "exit_target", "exit_leg", "exit_worm")
+    lists = {k: [] for k in keys}
+    for i in range(len(off)):
+        if off[i] < 0:
+            continue
+        part = {k: list(vd[k][off[i]:off[i] + cnt[i]]) for k in keys}
+        if cnt[i] == 4:
+            a, b = part["exit_cumprob"][2:4]
+            for k in keys:
+                part[k] = part[k][:3] + [part[k][3]] * 3
+            part["exit_cumprob"][3:5] = [a + (b - a) * 0.25, a + (b - a) * 0.75]
+        off[i], cnt[i] = len(lists["exit_cumprob"]), len(part["exit_cumprob"])
+        for k in keys:
+            lists[k] += part[k]
+    vd.update({k: np.array(lists[k], dtype=np.asarray(vd[k]).dtype) for k in keys})
+    vd.update(transition_offset=off, transition_count=cnt, n_exits=len(lists["exit_cumprob"]))
+    flat.types = [vd]
+    return flat
+
+
 MODELS = {
     "square": (lambda sse: square_heisenberg(sse, 4, d=-0.3, hz=0.1).flat(), "rows"),
     "honeycomb_dz": (honeycomb_dz, "rows"),
@@ -188,6 +226,9 @@ MODELS = {
     "bilayer": (lambda sse: job_bilayer(sse, 0.2).flat(), None),
     "trimer": (lambda sse: trimer_ring(sse, 7)[0], "exits"),
     "plaquette": (lambda sse: plaquette_ring(sse, 9)[0], "exits"),
+    "trimer_split": (trimer_split, "exits"),
+    "random_8": (lambda sse: random_bonds(sse, 8), "exits"),
+    "random_32": (lambda sse: random_bonds(sse, 32), "wide"),
 }
 
 
