@@ -35,6 +35,16 @@
 
 constexpr int kPersistSegments = 16;
 
+// Makes the workgroup's stores visible to the other XCDs: the L2's write-back has to
+// be over before the walker is given away.  The fence alone does not ensure that: the
+// compiler drops the wait behind buffer_wbl2 where it knows of no other access in
+// flight, as it does after a sweep.
+__device__ __forceinline__ void persist_release()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // Runs the tasks of a launch: task t is segment t / n_walkers of the budget of
 // walker order[t % n_walkers] (budgets[w] sweeps, or n_sweeps when budgets is
 // null).  queue[0] is the task counter and due = queue + 1 (segments > 1), all 0
@@ -77,7 +87,7 @@ __device__ __forceinline__ void persist_tasks(int32_t *queue, const int32_t *ord
                     break;
             if (segments == 1)
                 break;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            persist_release();
             int left = 0;
             if (lane == 0)
                 left = atomicSub(due + wi, todo) - todo;
