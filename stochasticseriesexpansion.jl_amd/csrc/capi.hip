@@ -389,7 +389,7 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     size_t o_wthr = put(wt.thr.data(), sizeof(uint64_t) * wt.thr.size());
     size_t o_wrow = put(wt.row.data(), sizeof(uint32_t) * wt.row.size());
     size_t o_wexit = put(wt.exit.data(), sizeof(uint4) * wt.exit.size());
-    size_t o_wwide = put(wt.wide.data(), sizeof(WormEntry) * wt.wide.size());
+    size_t o_wwide = put(wt.wide.data(), sizeof(uint32_t) * wt.wide.size());
     int dnv = 1;
     for (int t = 0; t < m.n_types; ++t)
         dnv = std::max(dnv, (int)m.types[t].n_vertices);
@@ -592,12 +592,12 @@ static int upload_model(sse_batch *b, const sse_model_desc &m, DevModel &dm, Hos
     dm.w_rank = wt.rank;
     dm.pad_w = 0;
     dm.wexit = wt.exit.empty() ? nullptr : (const uint4 *)(d + o_wexit);
-    dm.wwide = (const WormEntry *)(d + o_wwide);
+    dm.wwide = (const uint32_t *)(d + o_wwide);
     dm.w_ncode = (int32_t)wt.code.size();
     dm.w_lg = wt.lg;
     dm.w_nthr = wt.nthr;
     dm.w_mw = wt.mw;
-    dm.w_nent = (int32_t)wt.wide.size();
+    dm.w_nent = (int32_t)wt.nent;
     dm.w_dim = wt.dim;
     dm.k1tab = (const uint8_t *)(d + o_k1);
     dm.k1tab_bytes = (int32_t)k1.size();

@@ -62,7 +62,7 @@ struct DevModel {
     const uint64_t *wthr;
     const uint32_t *wrow;      // exit rows (null: too large, or some word has no exit)
     const uint4 *wexit;        // 16-byte exit entries (null: too many codes or thresholds)
-    const struct WormEntry *wwide;  // exit entries of any table, 64-byte aligned
+    const uint32_t *wwide;     // wide exit entries, of any table; 64-byte aligned
     int32_t w_ncode, w_lg, w_nthr, w_mw;
     int32_t w_nent;            // exit entries: ((w_ncode << w_lg) + 1) * 2 * w_mw
     int32_t w_dim;             // local dimension of every site, 0 when they differ
@@ -103,15 +103,13 @@ struct DevModel {
 // c * 2 * w_mw + 2 * (worm - 1) + side.  Its exit word names the leg relative
 // to the entering site, the port 2 * (worm - 1) + side with which the worm
 // enters the next operator, and the new vertex code.
-struct __align__(32) WormEntry {
-    // exit j < 3: the first with the word's top 32 bits below r[j] (ascending; ~0:
-    // always), else exit 3.  Equal top bits are looked up exactly.
-    uint32_t r[3];
-    // selector << 4 in bits 0..6, port in 7..19, new vertex - old one in 20..30
-    // (two's complement); bit 31 alone: no exit here (worm_exact)
-    uint32_t out[4];
-    uint32_t pad;
-};
+//
+// Wide entry (words): thresholds r0 r1 r2, exits o0 o1 o2 o3, r3, o4 (r3 and o4 with
+// four sites to a bond).  Exit j is the first with the word's top 32 bits below r_j
+// (ascending; ~0: always), else the last.  Equal top bits are looked up exactly.
+// An exit: selector << 4 in bits 0..6, port in 7..19, new vertex - old one in 20..30
+// (two's complement); bit 31 alone: no exit here (worm_exact).
+__host__ __device__ constexpr int worm_wide_words(int ns) { return ns == 4 ? 16 : 8; }
 __host__ __device__ inline uint32_t worm_entry_word(uint32_t leg, uint32_t port, int step)
 {
     return leg << 4 | port << 7 | ((uint32_t)step & 0x7FFu) << 20;

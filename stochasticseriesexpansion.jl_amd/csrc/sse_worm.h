@@ -45,8 +45,6 @@ typedef __attribute__((address_space(3))) uint64_t lds_u64;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 typedef const __attribute__((address_space(4))) uint64_t const_u64;
-typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-typedef const __attribute__((address_space(4))) u32x8 const_u32x8;
 typedef const __attribute__((address_space(4))) uint8_t const_u8;
 
 // LDS by byte address: entry ids and table rows are addresses, so that the step
@@ -206,7 +204,7 @@ struct TabExits {
     }
 };
 
-// WormEntry in global memory: any number of codes, worm types and thresholds.  The
+// Wide entries in global memory: any number of codes, worm types and thresholds.  The
 // table is constant, and one load to the scalar unit brings a whole entry; a word is
 // compared by its top 32 bits against the entry's own thresholds, so that no rank is
 // needed, however many bond types a model has.  Where they are equal (2^-32 a
@@ -217,25 +215,32 @@ template <int NS>
 struct TabWide {
     static constexpr bool kNone = true, kScalar = true;
     uint32_t ports;
-    const WormEntry *t;
-    typedef u32x8 Word;
+    const uint32_t *t;
+    typedef uint32_t Word __attribute__((ext_vector_type(worm_wide_words(NS))));
+    typedef const __attribute__((address_space(4))) Word const_word;
     __device__ __forceinline__ uint32_t row_of(uint64_t m) const { return (uint32_t)(m >> 21); }
     __device__ __forceinline__ Word load(uint32_t, uint32_t c, uint32_t port) const
     {
         // below 4 GB: a 32-bit offset goes into the load instruction
-        const uint32_t at = (uni(c) * ports + uni(port)) * (uint32_t)sizeof(WormEntry);
-        return *(const_u32x8 *)((const_u8 *)(const void *)t + at);
+        const uint32_t at = (uni(c) * ports + uni(port)) * (uint32_t)sizeof(Word);
+        return *(const_word *)((const_u8 *)(const void *)t + at);
     }
     __device__ __forceinline__ static uint32_t unsure(Word w, uint32_t row)
     {
-        return row == w.s0 || row == w.s1 || row == w.s2 || row == ~0u ? 0x80000000u : 0u;
+        bool u = row == w[0] || row == w[1] || row == w[2] || row == ~0u;
+        if constexpr (NS == 4)
+            u = u || row == w[7];
+        return u ? 0x80000000u : 0u;
     }
     typedef uint32_t Pick;
     __device__ __forceinline__ Pick pick(Word w, uint32_t row) const
     {
-        uint32_t o = row < w.s2 ? w.s5 : w.s6;
-        o = row < w.s1 ? w.s4 : o;
-        return row < w.s0 ? w.s3 : o;
+        uint32_t o = w[6];
+        if constexpr (NS == 4)
+            o = row < w[7] ? o : w[8];
+        o = row < w[2] ? w[5] : o;
+        o = row < w[1] ? w[4] : o;
+        return row < w[0] ? w[3] : o;
     }
     __device__ __forceinline__ static uint32_t sh(Pick o) { return o; }
     __device__ __forceinline__ WormExit<NS> exit(Pick o, uint32_t c) const
@@ -256,50 +261,140 @@ struct TabWide {
 };
 
 // ------------------------------------------------------------------ records
-// Entry ids start at id0; part() is signed, negative where flagged.
-struct RecL8 {  // LDS, 8-bit codes: id = byte address of the code
+// Entry ids start at id0.  An entry's partners are a Part: the entry of its operator on
+// the bond's next site, whose own gives the one after that, and the flag.
+template <uint32_t kFlag>
+struct RecNext {
+    typedef int32_t Part;
+    // bit 31: flagged
+    __device__ __forceinline__ static uint32_t top(Part p) { return (uint32_t)p; }
+    __device__ __forceinline__ static Part plain(Part p) { return (Part)((uint32_t)p & (kFlag - 1u)); }
+    __device__ __forceinline__ static Part flagged(Part p) { return (Part)((uint32_t)p | kFlag); }
+    // of a guard, the entry at the other end of the site's range
+    __device__ __forceinline__ static uint32_t other_end(Part p) { return (uint32_t)plain(p); }
+    __device__ __forceinline__ static Part guard(uint32_t to) { return (Part)(to | kFlag); }
+    // partners of entry e[k]
+    template <int NS>
+    __device__ __forceinline__ static Part link(const uint32_t *e, int k)
+    {
+        return NS == 1 ? 0 : (Part)e[(k + 1) % NS];
+    }
+};
+struct RecL8 : RecNext<0x8000u> {  // LDS, 8-bit codes: id = byte address of the code
     static constexpr bool kGlobal = false;
     uint32_t id0, poff;  // partner of id at poff + 2 * id
-    static constexpr uint32_t kFlag = 0x8000u;
+    __device__ __forceinline__ RecL8(uint32_t i, uint32_t p) : id0(i), poff(p) {}
     __device__ __forceinline__ uint32_t code(uint32_t id) const { return *lds_at<lds_u8>(id); }
-    __device__ __forceinline__ int32_t part(uint32_t id) const { return *lds_at<lds_i16>(poff + 2u * id); }
+    __device__ __forceinline__ Part part(uint32_t id) const { return *lds_at<lds_i16>(poff + 2u * id); }
     __device__ __forceinline__ void set_code(uint32_t id, uint32_t c) const
     {
         *lds_at<lds_u8>(id) = (uint8_t)c;
     }
-    __device__ __forceinline__ void set_part(uint32_t id, uint32_t p) const
+    __device__ __forceinline__ void set_part(uint32_t id, Part p) const
     {
         *lds_at<lds_u16>(poff + 2u * id) = (uint16_t)p;
     }
 };
-struct RecL16 {  // LDS, 16-bit codes: id = half the byte address of the code
+struct RecL16 : RecNext<0x8000u> {  // LDS, 16-bit codes: id = half the byte address of the code
     static constexpr bool kGlobal = false;
     uint32_t id0, poff;  // partner of id at poff + 2 * id
-    static constexpr uint32_t kFlag = 0x8000u;
+    __device__ __forceinline__ RecL16(uint32_t i, uint32_t p) : id0(i), poff(p) {}
     __device__ __forceinline__ uint32_t code(uint32_t id) const { return *lds_at<lds_u16>(2u * id); }
-    __device__ __forceinline__ int32_t part(uint32_t id) const { return *lds_at<lds_i16>(poff + 2u * id); }
+    __device__ __forceinline__ Part part(uint32_t id) const { return *lds_at<lds_i16>(poff + 2u * id); }
     __device__ __forceinline__ void set_code(uint32_t id, uint32_t c) const
     {
         *lds_at<lds_u16>(2u * id) = (uint16_t)c;
     }
-    __device__ __forceinline__ void set_part(uint32_t id, uint32_t p) const
+    __device__ __forceinline__ void set_part(uint32_t id, Part p) const
     {
         *lds_at<lds_u16>(poff + 2u * id) = (uint16_t)p;
     }
 };
 template <class C>
-struct RecG {  // global memory; every lane stores, so each lane's own later load is ordered after it
+struct RecG : RecNext<0x80000000u> {  // global memory; every lane stores, so each lane's own later load is ordered after it
     static constexpr bool kGlobal = true;
     gmem<uint32_t> *p;
     gmem<C> *c;
     uint32_t n;  // entries
     static constexpr uint32_t id0 = 0;
-    static constexpr uint32_t kFlag = 0x80000000u;
+    __device__ __forceinline__ RecG(gmem<uint32_t> *p_, gmem<C> *c_, uint32_t n_) : p(p_), c(c_), n(n_) {}
     __device__ __forceinline__ uint32_t code(uint32_t id) const { return c[id]; }
-    __device__ __forceinline__ int32_t part(uint32_t id) const { return (int32_t)p[id]; }
+    __device__ __forceinline__ Part part(uint32_t id) const { return (Part)p[id]; }
     __device__ __forceinline__ void set_code(uint32_t id, uint32_t x) const { c[id] = (C)x; }
-    __device__ __forceinline__ void set_part(uint32_t id, uint32_t x) const { p[id] = x; }
+    __device__ __forceinline__ void set_part(uint32_t id, Part x) const { p[id] = (uint32_t)x; }
 };
+// Global memory, bonds of three and four sites: all partners of an entry in one
+// 8-byte load, where a chain of partners costs one more trip to L2 per site and step.
+// Ids have 31 bits with three sites, 21 with four.
+template <int NS>
+struct RecGAll {
+    static constexpr bool kGlobal = true;
+    static constexpr uint32_t kBits = NS == 3 ? 32 : 21;
+    static constexpr uint32_t kMaxIds = NS == 3 ? 1u << 31 : 1u << 21;
+    typedef uint64_t Part;
+    gmem<uint64_t> *p;
+    gmem<uint16_t> *c;
+    uint32_t n;  // entries
+    static constexpr uint32_t id0 = 0;
+    __device__ __forceinline__ static uint32_t id(Part p, int k)
+    {
+        return (uint32_t)((p >> (kBits * k)) & (kMaxIds - 1u));
+    }
+    __device__ __forceinline__ static uint32_t top(Part p) { return (uint32_t)(p >> 32); }
+    __device__ __forceinline__ static Part plain(Part p) { return p & ~(1ull << 63); }
+    __device__ __forceinline__ static Part flagged(Part p) { return p | 1ull << 63; }
+    __device__ __forceinline__ static uint32_t other_end(Part p) { return id(p, 0); }
+    __device__ __forceinline__ static Part guard(uint32_t to) { return (Part)to | 1ull << 63; }
+    template <int>
+    __device__ __forceinline__ static Part link(const uint32_t *e, int k)
+    {
+        Part x = 0;
+#pragma unroll
+        for (int j = 1; j < NS; ++j)
+            x |= (Part)e[(k + j) % NS] << (kBits * (j - 1));
+        return x;
+    }
+    __device__ __forceinline__ RecGAll(gmem<uint64_t> *p_, gmem<uint16_t> *c_, uint32_t n_) : p(p_), c(c_), n(n_) {}
+    __device__ __forceinline__ uint32_t code(uint32_t id) const { return c[id]; }
+    __device__ __forceinline__ Part part(uint32_t id) const { return p[id]; }
+    __device__ __forceinline__ void set_code(uint32_t id, uint32_t x) const { c[id] = (uint16_t)x; }
+    __device__ __forceinline__ void set_part(uint32_t id, Part x) const { p[id] = x; }
+};
+// The same with the codes in LDS, byte address base on: a step then stores nothing to
+// global memory.  Ring of 1000 three-site bonds at beta = 12 (n = 16400), 64 walkers:
+// 45 ms per sweep with a chain of partners and codes in global memory, 31.6 without the
+// chain, 28.0 with the codes in LDS.
+template <int NS, class C>
+struct RecHAll : RecGAll<NS> {
+    typedef __attribute__((address_space(3))) C lds_c;
+    uint32_t base;
+    __device__ __forceinline__ RecHAll(gmem<uint64_t> *p_, uint32_t b, uint32_t n_)
+        : RecGAll<NS>(p_, nullptr, n_), base(b)
+    {
+    }
+    __device__ __forceinline__ lds_c *at(uint32_t id) const { return lds_at<lds_c>(base + (uint32_t)sizeof(C) * id); }
+    __device__ __forceinline__ uint32_t code(uint32_t id) const { return *at(id); }
+    __device__ __forceinline__ void set_code(uint32_t id, uint32_t x) const { *at(id) = (C)x; }
+};
+// entries of an operator behind q[0], whose partners are pt (not flagged)
+template <int NS, class R>
+__device__ __forceinline__ void rec_others(const R &rec, int32_t pt, uint32_t *q)
+{
+    if constexpr (NS > 1)
+        q[1] = (uint32_t)pt;
+#pragma unroll
+    for (int j = 2; j < NS; ++j)
+        q[j] = (uint32_t)R::plain(rec.part(q[j - 1]));
+}
+template <int NS, class R>
+__device__ __forceinline__ void rec_others(const R &, uint64_t pt, uint32_t *q)
+{
+#pragma unroll
+    for (int j = 1; j < NS; ++j)
+        q[j] = R::id(pt, j - 1);
+}
+__device__ __forceinline__ int32_t uni_part(int32_t p) { return (int32_t)uni((uint32_t)p); }
+__device__ __forceinline__ uint64_t uni_part(uint64_t p) { return uni64(p); }
 
 // ------------------------------------------------------------------ stream
 // The walker's Philox words in registers: lane l holds word bbase + l (bbase
@@ -465,8 +560,8 @@ __device__ __noinline__ bool worm_stage(R rec, WormCtx x)
                 x.sb[s] = (uint16_t)(g + 1u);
             rec.set_code(g, x.guard);
             rec.set_code(g + cnt + 1u, x.guard);
-            rec.set_part(g, (g + cnt) | rec.kFlag);
-            rec.set_part(g + cnt + 1u, (g + 1u) | rec.kFlag);
+            rec.set_part(g, R::guard(g + cnt));
+            rec.set_part(g + cnt + 1u, R::guard(g + 1u));
         }
         run += total;
     }
@@ -529,7 +624,7 @@ __device__ __noinline__ bool worm_stage(R rec, WormCtx x)
 #pragma unroll
                 for (int k = 0; k < NS; ++k) {
                     rec.set_code(e[k], c | (uint32_t)k);
-                    rec.set_part(e[k], NS == 1 ? 0u : e[(k + 1) % NS]);
+                    rec.set_part(e[k], R::template link<NS>(e, k));
                 }
             }
             if constexpr (!R::kGlobal) {
@@ -763,10 +858,10 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
         const uint32_t porta = 2u * (dim0 - wf0 - 2u) + (up0 ^ 1u);
         uint32_t e = e0 + vz, port = port0 + vz;
         uint32_t c = rec.code(e);
-        int32_t pt = rec.part(e);
-        const uint32_t part0 = uni((uint32_t)pt), parta = uni((uint32_t)rec.part(ea + vz));
-        rec.set_part(e0 + vz, part0 | rec.kFlag);
-        rec.set_part(ea + vz, parta | rec.kFlag);
+        typename R::Part pt = rec.part(e);
+        const typename R::Part part0 = uni_part(pt), parta = uni_part(rec.part(ea + vz));
+        rec.set_part(e0 + vz, R::flagged(part0));
+        rec.set_part(ea + vz, R::flagged(parta));
         const uint64_t ctr0 = rs.ctr();
         const uint32_t row0 = rdlane(rs.row, rs.off & 63u);
         uint32_t row = row0;
@@ -784,18 +879,14 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
             uint32_t off = uni(rs.off);
             row = uni(row);
             uint32_t q[NS], cq, pq, rq, none, ends;
-            bool stop;
+            bool stop = false;  // (kScalar)
             // scalar loads return out of order: with one in flight from before the
             // loop, its first instruction would wait for the table in every step
             if constexpr (T::kScalar)
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
             do {
                 q[0] = e;
-                if constexpr (NS > 1)
-                    q[1] = (uint32_t)pt;
-#pragma unroll
-                for (int j = 2; j < NS; ++j)
-                    q[j] = (uint32_t)rec.part(q[j - 1]) & (rec.kFlag - 1u);
+                rec_others<NS>(rec, pt, q);
                 const WormHop<NS, R::kGlobal> hop(q);
                 cq = c;
                 pq = port;
@@ -824,10 +915,17 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
                     rq = T::unsure(wd, row);
                 const WormExit<NS> ex = tab.exit(pick, cq);
                 none = ex.none;
+                if constexpr (!T::kScalar) {
+#pragma unroll
+                    for (int j = 0; j < NS; ++j)
+                        rec.set_code(q[j], ex.c[j]);
+                }
                 off += 1u;
                 e = nx;
                 port = ex.port;
                 row = rdlane(rs.row, off & 63u);
+                if constexpr (!T::kScalar)
+                    wd = tab.load(row, c, port);
                 // one condition, one branch: a flag, no exit, or no word left
                 ends = (63u - off) | (T::kNone ? rq : 0u);
                 if constexpr (T::kNone)
@@ -835,18 +933,14 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
                 // a wait for LDS is a wait for the scalar load too, so that one
                 // leaves after the test of the flag
                 if constexpr (T::kScalar) {
-                    stop = wave_any((int32_t)((uint32_t)pt | ends) < 0);
+                    stop = wave_any((int32_t)(R::top(pt) | ends) < 0);
                     __builtin_amdgcn_sched_barrier(0);
                     wd = tab.load(row, c, port);
-                }
 #pragma unroll
-                for (int j = 0; j < NS; ++j)
-                    rec.set_code(q[j], ex.c[j]);
-                if constexpr (!T::kScalar) {
-                    wd = tab.load(row, c, port);
-                    stop = wave_any((int32_t)((uint32_t)pt | ends) < 0);
+                    for (int j = 0; j < NS; ++j)
+                        rec.set_code(q[j], ex.c[j]);
                 }
-            } while (!stop);
+            } while (T::kScalar ? !stop : !wave_any((int32_t)(R::top(pt) | ends) < 0));
             rs.off = off;
             if constexpr (T::kNone) {
                 if (__builtin_expect(wave_any((int32_t)(none | rq) < 0), 0)) {
@@ -872,17 +966,17 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
                     wd = tab.load(row, c, port);
                 }
             }
-            if (!wave_any(pt < 0))
+            if (!wave_any((int32_t)R::top(pt) < 0))
                 continue;
             // a flagged entry: the worm's end, a guard, or neither
             if (wave_any(e == ea && port == porta))
                 break;
             if (wave_any(c == x.guard)) {
-                e = (uint32_t)pt & (rec.kFlag - 1u);
+                e = R::other_end(pt);
                 c = rec.code(e);
                 pt = rec.part(e);
                 wd = tab.load(row, c, port);
-                if (!wave_any(pt < 0))
+                if (!wave_any((int32_t)R::top(pt) < 0))
                     continue;
                 // the start leg may be the one behind the guard
             }
@@ -890,7 +984,7 @@ __device__ __forceinline__ int worm_chase(const WormCtx &x, const DevModel &m, W
                 reentry = 1u;
                 break;
             }
-            pt &= (int32_t)(rec.kFlag - 1u);
+            pt = R::plain(pt);
         }
         rec.set_part(e0 + vz, part0);
         rec.set_part(ea + vz, parta);
@@ -1180,7 +1274,25 @@ __device__ __forceinline__ void worm_walker(DevWalker *W, const DevModel *models
                 err = SSE_ERR_STATE;
             }
         } else {
-            WORM_RUN((RecG<uint16_t>{gp, (gmem<uint16_t> *)(gp + cofs), ne}), wide);
+            // 8 bytes of partners per entry where the slab, which has 4 per
+            // possible one, holds them: cutoffs are about twice the operator
+            // count and more
+            const size_t room = (4u + (size_t)worm_code_bytes(m)) * ((size_t)NS * w.cap + 2u * (size_t)pool->max_sites);
+            bool all = false;
+            if constexpr (NS >= 3) {
+                all = 10u * E <= room && E <= RecGAll<NS>::kMaxIds;
+                gmem<uint64_t> *ga = (gmem<uint64_t> *)gp;
+                if (all && mode != 2 && E * (size_t)cb <= (size_t)lds_bytes) {
+                    if (small)
+                        WORM_RUN((RecHAll<NS, uint8_t>{ga, lds, ne}), wide);
+                    else
+                        WORM_RUN((RecHAll<NS, uint16_t>{ga, lds, ne}), wide);
+                } else if (all) {
+                    WORM_RUN((RecGAll<NS>{ga, (gmem<uint16_t> *)(ga + ne), ne}), wide);
+                }
+            }
+            if (!all)
+                WORM_RUN((RecG<uint16_t>{gp, (gmem<uint16_t> *)(gp + cofs), ne}), wide);
         }
     }
 #undef WORM_RUN

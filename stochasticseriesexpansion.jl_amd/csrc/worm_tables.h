@@ -21,8 +21,8 @@ struct WormTables {
     std::vector<uint64_t> thr;
     std::vector<uint32_t> row;
     std::vector<uint4> exit;
-    std::vector<WormEntry> wide;
-    int nthr = 0, lg = 0, mw = 1, dim = 0, rank = 0;
+    std::vector<uint32_t> wide;
+    int nthr = 0, lg = 0, mw = 1, dim = 0, rank = 0, nent = 0;
 };
 
 // Exit rows take LDS beside every walker's records, which the step without a
@@ -97,7 +97,8 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
     }
     const size_t nc = t.code.size(), ports = 2 * (size_t)t.mw;
     const size_t nent = ((nc << t.lg) + 1) * ports;
-    if (nent * sizeof(WormEntry) >= ((size_t)1 << 32))  // the kernel's offsets have 32 bits
+    const size_t ww = worm_wide_words(ns);
+    if (nent * ww * 4 >= ((size_t)1 << 32))  // the kernel's offsets have 32 bits
         return "too many worm table entries";
     for (int i : rep) {
         const sse_vertex_data_desc &vd = m.types[i];
@@ -117,7 +118,11 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
                                               t.thr.begin()) + 1u;
     };
     const uint32_t always = 0xFFFFFFFFu;
-    t.wide.assign(nent, WormEntry{{always, always, always}, {1u << 31, 1u << 31, 1u << 31, 1u << 31}, 0u});
+    t.nent = (int)nent;
+    t.wide.assign(nent * ww, 1u << 31);
+    for (size_t e = 0; e < nent; ++e)
+        for (int j = 0; j < 4; ++j)
+            t.wide[ww * e + (j < 3 ? j : 7)] = always;
     // 16-byte entries: exits of 16 bits (selector, port, code; bit 15: none, with
     // selector and port 0, which the step follows before it sees the bit), ranks in
     // three 10-bit fields (511: always), for four sites per bond a fifth exit
@@ -155,25 +160,26 @@ inline const char *build_worm_tables(const sse_model_desc &m, WormTables &t)
                     };
                     const auto vertex = [&](int j) { return vd.exit_target[off + j] >> 1; };
                     const auto code = [&](int j) { return (uint32_t)(base[i] + vertex(j)); };
-                    // exits and thresholds 0..2; exit 3 stands for every word past
-                    // the third threshold: the fourth exit if it ends the list at
-                    // 1, else none (the exact search decides)
-                    const int ends = cnt == 4 && cum(3) >= kWormTail ? 4 : std::min(cnt, 3);
-                    WormEntry &x = t.wide[ix];
+                    // the last exit stands for every word past the thresholds: it
+                    // has to end the list at 1, else none (the exact search decides)
+                    const auto held = [&](int nt) { return cnt == nt + 1 && cum(nt) >= kWormTail ? cnt : std::min(cnt, nt); };
+                    uint32_t *x = &t.wide[ww * ix];
+                    const int nt = ns == 4 ? 4 : 3;
+                    for (int j = 0; j < held(nt); ++j) {
+                        x[j < 4 ? 3 + j : 8] = worm_entry_word(leg(j), port(j), vertex(j) - v);
+                        if (j < nt)
+                            x[j < 3 ? j : 7] = cum(j) >= kWormTail ? always : (uint32_t)(cum(j) >> 21);
+                        if (j > 0 && j < nt)
+                            x[j < 3 ? j : 7] = std::max(x[j < 3 ? j : 7], x[j - 1]);
+                    }
                     uint32_t r[3] = {511u, 511u, 511u}, o[5] = {0x8000u, 0x8000u, 0x8000u, 0x8000u, 0x8000u};
                     const auto narrow = [&](int j) { return leg(j) | port(j) << lcb | code(j) << 8; };
-                    for (int j = 0; j < ends; ++j) {
-                        x.out[j] = worm_entry_word(leg(j), port(j), vertex(j) - v);
-                        if (small)
-                            o[j] = narrow(j);
-                        if (j < 3) {
-                            x.r[j] = cum(j) >= kWormTail ? always : (uint32_t)(cum(j) >> 21);
+                    for (int j = 0; small && j < held(3); ++j) {
+                        o[j] = narrow(j);
+                        if (j < 3)
                             r[j] = std::min(rank(cum(j)), 511u);
-                        }
-                        if (j > 0 && j < 3) {
-                            x.r[j] = std::max(x.r[j], x.r[j - 1]);
+                        if (j > 0 && j < 3)
                             r[j] = std::max(r[j], r[j - 1]);
-                        }
                     }
                     if (small) {
                         uint32_t r3 = 511u;

@@ -6,6 +6,7 @@ checked on the CPU (test_worm_tables_cpu.py).
 Bit-exact: the tables hold the same lists, so nothing may differ."""
 import pytest
 
+from fixtures import plaquette_ring, trimer_ring
 from test_gpu_parity import _compare, _say
 from test_worm_tables_cpu import honeycomb_dz, random_bonds, trimer_split
 
@@ -38,4 +39,64 @@ def test_exit_tables(sse_pkg, oracle_mod, kind, records):
         for o in oracles:
             o.sweep(1)
         _compare(batch, oracles, f"{kind} sweep {s}")
+    batch.close()
+
+
+@pytest.mark.parametrize("make", [trimer_ring, plaquette_ring])
+@pytest.mark.parametrize("n", [7, 64])
+def test_global_records_of_growing_walkers(sse_pkg, oracle_mod, make, n):
+    """Global records of three- and four-site bonds while a cold walker's cutoff
+    grows from 64 slots: its slab holds all partners of an entry side by side at
+    first (448 slots for 64), not when 394 slots are full of operators, and again
+    in the next slab."""
+    flat = make(sse_pkg, n)[0]
+    walkers = [sse_pkg.walker_desc(T=T, seed=260 + k, init_opstring_cutoff=64, diagonal_warmup_sweeps=0)
+               for k, T in enumerate((0.01, 0.05, 2.0))]
+    _say(f"global records: {make.__name__} {n}")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    batch.set_option(sse_pkg.capi.SSE_OPT_WORM_RECORDS, 2)
+    oracles = [oracle_mod.OracleWalker(sse_pkg.capi, flat, w) for w in walkers]
+    batch.init()
+    for o in oracles:
+        o.init()
+    full = 0.0
+    for s in range(8):
+        batch.sweep(1)
+        for o in oracles:
+            o.sweep(1)
+        _compare(batch, oracles, f"sweep {s}")
+        sc = batch.get_walker(0)[0]
+        full = max(full, sc["num_operators"] if sc["cutoff"] == 394 else 0)
+    # bytes of the records with 8-byte partners against the slab's
+    ns = flat.bond_n_sites
+    assert 10 * (ns * full + 2 * n) > 6 * (ns * 448 + 2 * n)
+    batch.close()
+
+
+@pytest.mark.parametrize("make,n", [(trimer_ring, 64), (plaquette_ring, 20)])
+@pytest.mark.parametrize("k2_lds", [768, 1280, 2048])
+def test_codes_in_lds_without_the_records(sse_pkg, oracle_mod, make, n, k2_lds):
+    """Three- and four-site bonds with LDS for the codes of some walkers and not for
+    their partners, for neither of others; the walkers change sides as they grow."""
+    flat = make(sse_pkg, n)[0]
+    walkers = [sse_pkg.walker_desc(T=T, seed=360 + k, thermalization=4)
+               for k, T in enumerate((0.2, 0.35, 0.6, 1.0, 3.0))]
+    _say(f"codes in LDS: {make.__name__} {k2_lds}")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    batch.set_option(sse_pkg.capi.SSE_OPT_K2_LDS, k2_lds)
+    oracles = [oracle_mod.OracleWalker(sse_pkg.capi, flat, w) for w in walkers]
+    batch.init()
+    for o in oracles:
+        o.init()
+    code = 1 if flat.bond_n_sites == 3 else 2
+    hybrid = 0
+    for s in range(14):
+        batch.sweep(1)
+        for o in oracles:
+            o.sweep(1)
+        _compare(batch, oracles, f"sweep {s}")
+        for k in range(len(walkers)):
+            e = flat.bond_n_sites * batch.get_walker(k)[0]["num_operators"] + 2 * n
+            hybrid += code * e <= k2_lds < (code + 2) * e
+    assert hybrid > 0
     batch.close()

@@ -53,7 +53,7 @@ class Tables:
             self.thr = image(0, np.uint64)
             self.row = image(1, np.uint32)
             self.exit = image(2, np.uint32).reshape(-1, 4)
-            self.wide = image(3, WIDE)
+            self.wide = image(3, np.uint32).reshape(self.nent, -1)
             self.code = image(4, np.uint32).reshape(-1, 2)
             self.bond = image(5, np.uint32).reshape(-1, 4)
         host.wt_free(h)
@@ -83,18 +83,16 @@ class Tables:
         return o & ((1 << lcb) - 1), (o >> lcb) & ((1 << (8 - lcb)) - 1), o >> 8
 
     def wides(self, ix, m):
-        x, w = self.wide[ix], m >> 21
-        r = [int(v) for v in x["r"]]
-        j = next((k for k in range(3) if w < r[k]), 3)
-        o = int(x["out"][j])
+        x, w = [int(v) for v in self.wide[ix]], m >> 21
+        r, out = x[:3], x[3:7]
+        if self.ns == 4:
+            r, out = r + [x[7]], out + [x[8]]
+        o = out[next((k for k in range(len(r)) if w < r[k]), len(r))]
         if w in r or w == 0xFFFFFFFF or o >> 31:
             return None
         step = (o >> 20) & 0x7FF
         code = (ix // self.ports) >> self.lg
         return (o & 127) >> 4, (o >> 7) & 0x1FFF, code + (step - 2048 if step >= 1024 else step)
-
-
-WIDE = np.dtype([("r", np.uint32, 3), ("out", np.uint32, 4), ("pad", np.uint32)])
 
 
 def k_of(c):

@@ -19,7 +19,7 @@ void wt_info(void *h, int64_t *out)
     out[0] = t.nthr;
     out[1] = t.lg;
     out[2] = t.mw;
-    out[3] = (int64_t)t.wide.size();
+    out[3] = t.nent;
 }
 
 // image 0 thresholds, 1 rows, 2 16-byte exits, 3 wide entries, 4 codes, 5 bonds
