@@ -278,9 +278,8 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
         if (do_diag) {
             const uint32_t D = 2u * (uint32_t)popc(identm) + (uint32_t)popc(diam);
             const uint32_t off = 2u * bits_below(identm) + bits_below(diam);
-            if (D > 0u)
-                rs.ensure(D);
-            const uint64_t x0 = rs.peek(D ? off : 0u), x1 = rs.peek(D ? off + 1u : 0u);
+            rs.ensure(D + 2u);  // as in k1_walker_t
+            const uint64_t x0 = rs.peek(off), x1 = rs.peek(off + 1u);
             // rand(1:n_bonds): high half of word * n_bonds, rejected where the low
             // half could be below 2^64 mod n_bonds
             const uint64_t pl = (uint64_t)(uint32_t)x0 * nbonds;
