@@ -561,7 +561,7 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
             }
         }
         const uint32_t op = cur[slot];
-        const uint32_t vc = op_vcode(op);
+        const uint32_t vc = op_vcode(op), vx = vc >> 1;
         const bool ident = valid && op == 0u;
         const bool dia = op != 0u && (vc & 1u);
         const bool offd = op != 0u && !(vc & 1u);
@@ -587,6 +587,9 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
             const uint64_t ph = (uint64_t)(uint32_t)(x0 >> 32) * nbonds + (pl >> 32);
             const bool maybe = ident && (uint32_t)ph == 0u && (uint32_t)pl < nbonds;
             if (__builtin_expect(force_serial || wave_any(maybe), 0)) {
+                bad |= op != 0u && vx >= tab.nv(tab.bond(b).t);
+                if (wave_any(bad))  // its lookups take indexes as they are
+                    break;
                 const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, pm_raw, pr_raw, do_diag,
                                                            do_vl, sp, cnt);
                 n0 = uni((uint32_t)so.n);
@@ -598,6 +601,9 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
             u = word_to_float(ident ? x1 : x0);
             rs.advance(D);
         } else if (force_serial) {
+            bad |= op != 0u && vx >= tab.nv(tab.bond(b).t);
+            if (wave_any(bad))
+                break;
             const K1SerialOut so = k1_serial_chunk_ool(w, &m, rs, base, n0, pm_raw, pr_raw, do_diag,
                                                        do_vl, sp, cnt);
             n0 = uni((uint32_t)so.n);
@@ -608,7 +614,6 @@ __device__ __forceinline__ void k1_walker_t(DevWalker *W, const DevModel *models
 
         const K1Bond br = tab.bond(b);
         const uint32_t s0 = br.s0, s1 = br.s1;
-        const uint32_t vx = vc >> 1;
         uint32_t vi = vx;
         if (Tab::kChecked) {
             const uint32_t nv = tab.nv(br.t);

@@ -286,6 +286,9 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
             const uint64_t ph = (uint64_t)(uint32_t)(x0 >> 32) * nbonds + (pl >> 32);
             const bool maybe = ident && (uint32_t)ph == 0u && (uint32_t)pl < nbonds;
             if (__builtin_expect(force_serial || wave_any(maybe), 0)) {
+                bad |= isop && (int)(vc >> 1) >= tab.nv(tab.type(b));
+                if (wave_any(bad))  // its lookups take indexes as they are
+                    break;
                 k1n_serial_chunk<NS>(w, m, rs, base, n0, pm_raw, pr_raw, do_diag, do_vl, sp, cnt);
                 continue;
             }
@@ -293,6 +296,9 @@ __device__ void k1n_walker(DevWalker *W, const DevModel *models, DevPool *pool, 
             u = word_to_float(ident ? x1 : x0);
             rs.advance(D);
         } else if (force_serial) {
+            bad |= isop && (int)(vc >> 1) >= tab.nv(tab.type(b));
+            if (wave_any(bad))
+                break;
             k1n_serial_chunk<NS>(w, m, rs, base, n0, pm_raw, pr_raw, do_diag, do_vl, sp, cnt);
             continue;
         }
