@@ -85,14 +85,22 @@ def poisson_jobs(n_jobs, rate=200.0, seed=7, L_range=(8, 48), beta_range=(1.0, 3
     return jobs
 
 
-def footprint_bytes(n_sites, n_bonds, T):
-    """Slab bytes a job needs at its steady-state cutoff: n ~ beta * (|E| +
-    sum of bond offsets) bounded by beta * 0.375 * Nb * 2.5, L ~ 2.2 n."""
+def slab_bytes(cap, max_sites):
+    """Bytes of a wave-mode slab of cap slots for a two-site model with worm codes
+    of two bytes, in a batch whose largest lattice has max_sites sites
+    (slab_bytes of csrc/sse_common.h)."""
+    return (24 * cap + 12 * max_sites + 255) & ~255
+
+
+def footprint_bytes(max_sites, n_bonds, T):
+    """Slab bytes a job needs at its steady-state cutoff, in a batch whose largest
+    lattice has max_sites sites: n ~ beta * (|E| + sum of bond offsets) bounded by
+    beta * 0.375 * Nb * 2.5, L ~ 2.2 n."""
     beta = 1.0 / T
     n_est = beta * n_bonds * 0.375 * 2.5 + 64
     L = int(2.2 * n_est) + 128
     cap = L + L // 2 + 100
-    return 24 * cap + 12 * n_sites
+    return slab_bytes(cap, max_sites)
 
 
 def latency_stats(jobs, t_end):
@@ -165,6 +173,7 @@ class ServingLoop:
     def run(self, jobs, time_limit=None, log=None):
         """Serve `jobs` (sorted by arrival); returns the finished jobs and stats."""
         b = self.batch
+        max_sites = max(f.n_sites for f in b.flats)
         pending = list(jobs)
         queue = []           # arrived, not admitted (FIFO)
         free = list(range(self.n_slots))
@@ -186,7 +195,7 @@ class ServingLoop:
                 job = queue[0]
                 mi = self.model_index(job.model_key)
                 flat = b.flats[mi]
-                fp = footprint_bytes(flat.n_sites, flat.n_bonds, job.T)
+                fp = footprint_bytes(max_sites, flat.n_bonds, job.T)
                 if used + fp > self.memory_budget and running:
                     break
                 queue.pop(0)
@@ -346,6 +355,7 @@ class SizeClassServing:
 
     def _serve(self, c, t0, done, done_lock, stop, time_limit):
         b = c.batch
+        max_sites = max(f.n_sites for f in b.flats)
         free = list(range(c.n_slots))
         running = {}
         used = 0
@@ -359,7 +369,7 @@ class SizeClassServing:
                     job = c.queue[0]
                     mi = c.model_index[job.model_key]
                     flat = b.flats[mi]
-                    fp = footprint_bytes(flat.n_sites, flat.n_bonds, job.T)
+                    fp = footprint_bytes(max_sites, flat.n_bonds, job.T)
                     if used + fp > c.memory_budget and running:
                         break
                     c.queue.pop(0)

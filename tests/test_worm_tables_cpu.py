@@ -29,6 +29,8 @@ def host(tmp_path_factory):
     lib.wt_build.argtypes = [C.c_void_p, C.POINTER(C.c_char_p)]
     lib.wt_free.argtypes = [C.c_void_p]
     lib.wt_info.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
+    lib.wt_slab_bytes.restype = C.c_int64
+    lib.wt_slab_bytes.argtypes = [C.c_int64, C.c_int, C.c_int, C.c_int]
     lib.wt_image.restype = C.c_void_p
     lib.wt_image.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_int64)]
     return lib
@@ -297,3 +299,14 @@ def test_word_of_a_missing_exit(sse_pkg, host, name):
     assert len(none)
     assert ((none & ((1 << (lcb - 1)) - 1)) < tab.ns).all()
     assert ((none >> lcb & ((1 << (8 - lcb)) - 1)) < tab.ports).all()
+
+
+@pytest.mark.parametrize("cap", [64, 448, 100032])
+@pytest.mark.parametrize("sites", [16, 64, 2304])
+def test_serving_footprint(host, cap, sites):
+    """Admission by memory counts what the slab pool hands out: the guards of the
+    batch's largest lattice come with every slab."""
+    from importlib import import_module
+    sv = import_module("sse_amd.serving")
+    assert sv.slab_bytes(cap, sites) == host.wt_slab_bytes(cap, 2, 6, sites)
+    assert sv.footprint_bytes(sites, 128, 1.0) == sv.slab_bytes(898, sites)

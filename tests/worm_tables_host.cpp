@@ -22,6 +22,17 @@ void wt_info(void *h, int64_t *out)
     out[3] = t.nent;
 }
 
+// bytes of a slab (csrc/sse_common.h) of cap slots, codes chase codes and sites
+// sites of the batch's largest lattice
+int64_t wt_slab_bytes(int64_t cap, int ns, int codes, int sites)
+{
+    DevModel m;
+    memset(&m, 0, sizeof m);
+    m.nsb = ns;
+    m.w_ncode = codes;
+    return (int64_t)slab_bytes(cap, m, sites, true);
+}
+
 // image 0 thresholds, 1 rows, 2 16-byte exits, 3 wide entries, 4 codes, 5 bonds
 const void *wt_image(void *h, int which, int64_t *bytes)
 {
