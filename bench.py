@@ -246,8 +246,8 @@ def parallelism(choice, walkers, generic=False):
     if generic:
         lds = "worm LDS sized from the largest walker"
     if choice["persistent"]:
-        return (f"autotuned: persistent work-queue launch (one workgroup per walker task, "
-                f"{walkers} tasks per call, HIP-graph replay), {lds}")
+        return (f"autotuned: persistent work-queue launch ({walkers} walkers per call, their sweeps "
+                f"in up to 16 tasks each, HIP-graph replay), {lds}")
     return (f"autotuned: {choice['groups']} stream groups of per-sweep kernels (one stream and "
             f"hardware queue per group, direct launches), one wavefront per walker, {lds}")
 
@@ -393,15 +393,25 @@ def sweep_budgets(cost, factor=4, cap=400):
     return np.minimum(cap, np.maximum(1, np.round(factor * cost.max() / cost))).astype(np.int64)
 
 
-def operator_count_costs(batch, n_walkers, k2_lds, slow=3.0):
+# Time of a worm step with the records in global memory over one with them in LDS
+# (205 against 92 ns, one walker: 32x32 at beta = 10 and 16x16 at beta = 8).
+RECORDS_IN_L2 = 2.2
+
+
+def operator_count_costs(batch, n_walkers, k2_lds, slow=3.0, sites=None):
     """Work per sweep of each walker from its chain: the operator count n,
     times `slow` when the worm update cannot hold the walker's records in
-    LDS (8 bytes per operator cover its 6-byte record, the exit table and
-    the site entries; larger walkers are taken to read records from L2 at
-    about three times the time per step)."""
+    LDS.  With the walkers' site counts the records are those of two-site bonds:
+    6 bytes per operator and 8 per site behind some 2 KB of exit tables, and less
+    than 32768 entries (two per operator and per site) with them.  Without,
+    8 bytes per operator up to 4096 stand for all of it."""
     ns = np.array([batch.get_walker(k, with_ops=False, with_spins=False)[0]["num_operators"]
                    for k in range(n_walkers)], dtype=np.float64)
-    in_lds = ns <= min(4096, k2_lds // 8)
+    if sites is None:
+        in_lds = ns <= min(4096, k2_lds // 8)
+    else:
+        sites = np.asarray(sites, dtype=np.float64)
+        in_lds = (6 * ns + 8 * sites + 2048 <= k2_lds) & (2 * ns + 2 * sites + 3072 < 32768)
     return np.maximum(ns, 1.0) * np.where(in_lds, 1.0, slow), ns, in_lds
 
 
@@ -419,7 +429,8 @@ def extra_heterogeneous(sse, walkers=2048, thermalization=300, steps=6, seed=3):
 
     def refine(batch, choice):
         k2 = int(choice["k2_lds"]) if choice and choice["k2_lds"] else int(batch.lds_bytes()[1])
-        cost, ns, in_lds = operator_count_costs(batch, walkers, k2)
+        cost, ns, in_lds = operator_count_costs(batch, walkers, k2, RECORDS_IN_L2,
+                                                [f.n_sites for f in flats])
         info.update({"worm_lds_bytes": k2, "walkers_records_in_lds": int(in_lds.sum()),
                      "n_quantiles_50_90_99_100": np.percentile(ns, [50, 90, 99, 100]).tolist()})
         log(f"heterogeneous: budgets from operator counts, {int(in_lds.sum())} of {walkers} "
@@ -429,8 +440,8 @@ def extra_heterogeneous(sse, walkers=2048, thermalization=300, steps=6, seed=3):
     r = run_batch(sse, flats, wds, thermalization, steps, "heterogeneous", budgets=budgets,
                   refine=refine)
     r["budgets"] = dict(info, rule="about 4 sweeps of the costliest walker's work per call, "
-                                   "cost = operator count x (3 if the records exceed the worm "
-                                   "LDS), at most 400 sweeps")
+                                   f"cost = operator count x ({RECORDS_IN_L2} if the records exceed "
+                                   "the worm LDS), at most 400 sweeps")
     r["workload"] = ("heterogeneous XXZ batch: 2048 walkers, L in {8,12,16,24,32}, "
                      "beta log-uniform [0.5,16], Jz ~ U[0.5,1.5], h=0.1")
     return r
