@@ -4,6 +4,7 @@ with their exits in LDS and in global memory.  Which table a model gets is
 checked on the CPU (test_worm_tables_cpu.py).
 
 Bit-exact: the tables hold the same lists, so nothing may differ."""
+import numpy as np
 import pytest
 
 from fixtures import plaquette_ring, trimer_ring
@@ -99,4 +100,41 @@ def test_codes_in_lds_without_the_records(sse_pkg, oracle_mod, make, n, k2_lds):
             e = flat.bond_n_sites * batch.get_walker(k)[0]["num_operators"] + 2 * n
             hybrid += code * e <= k2_lds < (code + 2) * e
     assert hybrid > 0
+    batch.close()
+
+
+def test_generic_work_queue_hands_walkers_over(sse_pkg, oracle_mod):
+    """2600 rings of three-site bonds, more than the card holds workgroups: the
+    tuner's work-queue calls cut the sweeps of a walker into tasks that other
+    workgroups take over, and all chains and sums stay those of one stream."""
+    n = 2600
+    flat = trimer_ring(sse_pkg, 6)[0]
+    walkers = [sse_pkg.walker_desc(T=0.7, seed=800 + k, thermalization=2) for k in range(n)]
+    _say(f"generic work queue: {n} walkers")
+    batch = sse_pkg.Batch([flat], walkers, mode=0)
+    batch.init()
+    sweeps = 0
+    while batch.tuning(0) is None and sweeps < 80:
+        batch.run(8, measure=True)
+        sweeps += 8
+    assert batch.tuning(0)["candidates_measured"] >= 3
+    batch.run(6, measure=True)
+    sweeps += 6
+    one = sse_pkg.Batch([flat], walkers, mode=0)
+    one.set_option(sse_pkg.capi.SSE_OPT_STREAMS, 1)
+    one.init()
+    one.run(sweeps, measure=True)
+    for a, b in zip(batch.accumulators_raw(), one.accumulators_raw()):
+        assert np.array_equal(a, b)
+    for k in range(0, n, 13):
+        a, b = batch.get_walker(k), one.get_walker(k)
+        assert a[0]["rng_counter"] == b[0]["rng_counter"]
+        assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+    for k in (0, 1, n // 2, n - 1):
+        o = oracle_mod.OracleWalker(sse_pkg.capi, flat, walkers[k])
+        o.init()
+        o.sweep(sweeps)
+        a, b = batch.get_walker(k), o.state()
+        assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
+    one.close()
     batch.close()
