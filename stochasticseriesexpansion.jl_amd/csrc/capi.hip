@@ -47,7 +47,7 @@ int fail(int code, const std::string &msg)
 // while every field is unchanged.  Compared bytewise (constructed zeroed).
 struct GraphKey {
     int32_t kind;       // 1 one stream, 2 stream groups, 3 persistent launch
-    int32_t sweeps, measure, groups, rec_mode, chase, use_order, n_tasks, segments, fuse, lane_width, generic;
+    int32_t sweeps, measure, groups, rec_mode, use_order, n_tasks, segments, fuse, lane_width, generic;
     size_t lds[9];      // worm-kernel LDS (one stream / per group), persistent LDS
     const void *models, *budgets, *order;
     GraphKey() { memset(this, 0, sizeof *this); }
@@ -175,7 +175,7 @@ struct sse_batch {
     // size, each group's worm kernel sized for its own largest walker)
     int32_t *d_order = nullptr;
     bool use_order = true;
-    int n_big = 0;  // leading walkers of the schedule too large for 8-byte LDS records
+    int n_big = 0;  // leading walkers of the schedule expected to need more than 32 KB of LDS
     int64_t *d_pt_acc = nullptr, *d_pt_prop = nullptr;
     std::vector<uint8_t> pt_member;
 };
@@ -1211,7 +1211,6 @@ static GraphKey graph_key(const sse_batch *b, int kind, int sweeps, int measure)
     k.sweeps = sweeps;
     k.measure = measure;
     k.rec_mode = b->wave.rec_mode;
-    k.chase = b->wave.chase;
     k.fuse = b->wave.fuse_measure;
     k.lane_width = b->lane_width;
     k.generic = b->wave.generic;
@@ -2648,10 +2647,9 @@ int sse_set_option(sse_batch *b, int32_t option, int64_t value)
         return SSE_OK;
     case SSE_OPT_CHASE:
         if (value != 0 && value != 1)
-            return fail(SSE_ERR_INVALID, "SSE_OPT_CHASE takes 0 (plain) or 1 (record lookahead)");
+            return fail(SSE_ERR_INVALID, "SSE_OPT_CHASE takes 0 or 1 (no effect: the traversal has one form)");
         HIPCHECK(hipStreamSynchronize(b->stream));
         b->tune = false;
-        b->wave.chase = (int)value;
         return SSE_OK;
     case SSE_OPT_LANE_WIDTH:
         if (value < 1 || value > 64)

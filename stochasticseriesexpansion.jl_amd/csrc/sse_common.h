@@ -94,10 +94,10 @@ struct DevModel {
 
 // Exit j of a scatter is the first j with r < cum[j], r = (word >> 11) * 2^-53.
 // With m = word >> 11 (an integer < 2^53) and K = ceil(cum * 2^53) this is
-// exactly m < K.  A model has few distinct K (the Heisenberg magnet 2, the
-// tables of this repository's tests at most 157), so a word is reduced once to
-// q = the number of K of the model that are <= m, and m < K becomes q < r with
-// r = 1 + the index of K: exact, and independent of where the worm is.
+// exactly m < K.  A model of few bond types has few distinct K (the Heisenberg
+// magnet 2), so a word is reduced once to q = the number of K of the model that are
+// <= m, and m < K becomes q < r with r = 1 + the index of K: exact, and independent
+// of where the worm is.  The tables in LDS use q, the wide table the words.
 //
 // Exit entry (c, worm-1, side the worm enters by: 0 lower, 1 upper) has index
 // c * 2 * w_mw + 2 * (worm - 1) + side.  Its exit word names the leg relative
@@ -422,7 +422,7 @@ __device__ __host__ __forceinline__ int64_t slab_capacity(int64_t L)
     return (c + 63) & ~(int64_t)63;
 }
 
-// Bytes of a chase code in global records: 2, or 4 when the codes need them.
+// Bytes of a worm code in global records: 2, or 4 when the codes need them.
 __device__ __host__ __forceinline__ int worm_code_bytes(const DevModel &m)
 {
     return ((int64_t)m.w_ncode << m.w_lg) <= 65535 ? 2 : 4;
@@ -430,7 +430,7 @@ __device__ __host__ __forceinline__ int worm_code_bytes(const DevModel &m)
 
 // Slab of a walker: ops[cap], then the record region.  Lane kernels: dense
 // links.  Wave kernels: idx (4 bytes per slot and bond site), then the global
-// worm records (a 4-byte partner and a chase code per entry, one entry per slot
+// worm records (a 4-byte partner and a worm code per entry, one entry per slot
 // and bond site and two more per lattice site of the batch's largest lattice, so
 // that a slot's slab serves every model of its shape); the entry words of the
 // LDS layouts, 4 or 8 bytes per slot, take the same place.

@@ -10,7 +10,7 @@
 //   * spins at identity slots and places along the sites: every lane ORs its
 //     bit into per-site LDS lane masks (one for bond position 0, one for 1);
 //     "latest earlier operator on site s" is the highest lower bit of the mask
-//     filtered by the off-diagonal (spins) or final non-identity (links) set.
+//     filtered by the off-diagonal (spins) or final non-identity (places) set.
 //   * the acceptance tests depend on the running operator count n, but each
 //     is monotone in n and n moves by at most one per slot: a lane's decision
 //     is fixed if it agrees at both ends of its window [n0-lane, n0+lane];
@@ -32,8 +32,7 @@ struct WaveConfig {
     int max_warmup = 0;
     size_t lds_k1 = 0, lds_k2 = 0, lds_k3 = 0;
     size_t lds_limit = 65536;  // device limit on dynamic LDS per workgroup
-    int rec_mode = 0;          // worm-kernel layout (worm_walker): 0 auto, 1 wide codes, 2 global
-    int chase = 0;             // SSE_OPT_CHASE as set (the traversal has one form)
+    int rec_mode = 0;          // SSE_OPT_WORM_RECORDS (worm_walker's mode)
     size_t lds_k2_fixed = 0;   // worm-kernel LDS per walker set by the caller (0 = sized here)
     size_t lds_k2_group[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // per stream group (0 = lds_k2)
     int fuse_measure = 0;      // measuring sweeps: worm update + measurement in one kernel
@@ -75,7 +74,6 @@ __device__ __noinline__ void wave_refill(uint64_t *buf, uint64_t key, uint64_t b
 
 template <int NW>
 struct WaveStreamT {
-    static constexpr uint32_t kNW = NW;
     uint64_t *buf;
     uint64_t key, bbase;
     uint32_t off;  // next word is bbase + off; off > 256 marks an empty buffer
@@ -101,13 +99,6 @@ struct WaveStreamT {
             off = (uint32_t)(c - bbase);
             wave_refill<NW>(buf, key, bbase);
         }
-    }
-    // the buffer is used up (off == NW): load the next NW words
-    __device__ __forceinline__ void refill_next()
-    {
-        bbase += off;
-        off = 0;
-        wave_refill<NW>(buf, key, bbase);
     }
     // word k positions after the next one (after ensure)
     __device__ __forceinline__ uint64_t peek(uint32_t k) const { return buf[off + k]; }
@@ -137,16 +128,14 @@ struct WaveStreamT {
 };
 
 typedef WaveStreamT<256> WaveStream;
-typedef WaveStreamT<128> WaveStream128;
-// The worm kernel's Philox words in registers: lane l holds word bbase + l of
-// the walker's stream (bbase even) and that word's 53-bit mantissa
-// (word >> 11, the integer behind rand()).  A wave-uniform draw is two
-// v_readlane with a scalar index; lanes that draw different words read them
-// with ds_bpermute.  No LDS and no barrier; all members except the four
-// per-lane words are wave-uniform and every call is made by the whole wave.
+// The state refresh's Philox words in registers: lane l holds word bbase + l of
+// the walker's stream (bbase even).  A wave-uniform draw is two v_readlane with a
+// scalar index; lanes that draw different words read them with ds_bpermute.  No
+// LDS and no barrier; all members except the two per-lane words are wave-uniform
+// and every call is made by the whole wave.
 struct K2RegStream {
     static constexpr uint32_t kNW = 64;
-    uint32_t wlo, whi, mlo, mhi;
+    uint32_t wlo, whi;
     uint64_t key, bbase;
     uint32_t off;  // next word is bbase + off; off >= 1024 marks an empty buffer
     __device__ void init(uint64_t k, uint64_t c)
@@ -162,9 +151,6 @@ struct K2RegStream {
         philox_block((bbase >> 1) + (lane >> 1), key, o0, o1, o2, o3);
         wlo = (lane & 1u) ? o2 : o0;
         whi = (lane & 1u) ? o3 : o1;
-        const uint64_t mm = (((uint64_t)whi << 32) | wlo) >> 11;
-        mlo = (uint32_t)mm;
-        mhi = (uint32_t)(mm >> 32);
     }
     __device__ __forceinline__ uint64_t ctr() const { return bbase + off - (off >= 1024 ? 1024 : 0); }
     // make words [ctr, ctr+need) resident (need <= 63)
@@ -182,14 +168,7 @@ struct K2RegStream {
             fill();
         }
     }
-    // the buffer is used up (off == kNW): load the next kNW words
-    __device__ __forceinline__ void refill_next()
-    {
-        bbase += off;
-        off = 0;
-        fill();
-    }
-    // word k (wave-uniform, < kNW) of the buffer and its mantissa
+    // word k (wave-uniform, < kNW) of the buffer
     __device__ __forceinline__ uint64_t word_at(uint32_t k) const
     {
         const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)wlo, (int)k);
@@ -212,7 +191,6 @@ struct K2RegStream {
         ++off;
         return x;
     }
-    __device__ __forceinline__ double next_float() { return word_to_float(next()); }
     __device__ __forceinline__ uint64_t range(uint64_t s)
     {
         uint64_t x = next();
