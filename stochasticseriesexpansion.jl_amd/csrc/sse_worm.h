@@ -787,12 +787,15 @@ __device__ __noinline__ uint64_t worm_exact(const DevModel *mp, uint32_t c, uint
 template <int NS, bool kWide>
 struct WormHop {
     uint64_t all;
-    uint32_t q[NS];
+    // members of their own: of an array the compiler makes a select between its
+    // elements' addresses, and keeps it in scratch memory
+    uint32_t q0, q1, q2, q3;
     __device__ __forceinline__ explicit WormHop(const uint32_t *e)
     {
-#pragma unroll
-        for (int k = 0; k < NS; ++k)
-            q[k] = e[k];
+        q0 = e[0];
+        q1 = NS > 1 ? e[NS > 1 ? 1 : 0] : 0u;
+        q2 = NS > 2 ? e[NS > 2 ? 2 : 0] : 0u;
+        q3 = NS > 3 ? e[NS > 3 ? 3 : 0] : 0u;
         if constexpr (!kWide && NS == 2) {
             const uint32_t pe = e[0] | e[1] << 16;
             all = (uint64_t)(pe - 0x00010001u) | (uint64_t)(pe + 0x00010001u) << 32;
@@ -811,11 +814,13 @@ struct WormHop {
             return (sh & 64u) ? t + 1u : t - 1u;
         } else {
             const bool up = NS <= 2 ? (sh & 32u) != 0u : (sh & 64u) != 0u;
-            const uint32_t rel = NS == 1 ? 0u : NS == 2 ? (sh >> 4) & 1u : (sh >> 4) & 3u;
-            uint32_t t = q[0];
-#pragma unroll
-            for (int k = 1; k < NS; ++k)
-                t = rel == (uint32_t)k ? q[k] : t;
+            uint32_t t = q0;
+            if constexpr (NS >= 2)
+                t = (sh & 16u) ? q1 : t;
+            if constexpr (NS >= 3) {
+                const uint32_t h = NS == 4 && (sh & 16u) ? q3 : q2;
+                t = (sh & 32u) ? h : t;
+            }
             return up ? t + 1u : t - 1u;
         }
     }
