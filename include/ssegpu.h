@@ -200,7 +200,7 @@ int sse_run_budgets(sse_batch *b, const int64_t *sweeps, int32_t measure);
  * reference.  For callers that cannot allocate device memory during the
  * call (serving loops that forbid it, harnesses that do).  The task counter
  * and the budgets live in a static device array of each GPU the library
- * runs on (about 0.75 MiB, held until the process ends), so the batch may
+ * runs on (about 1 MiB, held until the process ends), so the batch may
  * hold at most SSE_NOALLOC_MAX_WALKERS walkers (SSE_ERR_INVALID beyond).
  * Tasks run in the batch's schedule order; results are identical to
  * sse_run_budgets.  No events or graphs are made, so sse_call_time is not
@@ -343,18 +343,21 @@ int sse_pt_get_ladders(sse_batch *b, int32_t *slot_walkers, int64_t *accepted,
  *                a walker's records in LDS where they fit (two entries per
  *                operator of a two-site bond, 3 bytes each with <= 256 worm
  *                codes, else 4), with the model's exit table beside them, else
- *                both in global memory; the kernel's LDS per walker is capped
- *                at 64 KiB, so larger walkers take the global layout.  1 =
- *                4-byte entries and the exit table in global memory; 2 forces
- *                global records; 3 = the exit table in global memory.
+ *                in global memory; with three and four sites to a bond the codes
+ *                stay in LDS where they fit it without the rest.  The kernel's
+ *                LDS per walker is sized for at most 64 KiB and then widened
+ *                within the same residency (two walkers to a compute unit: 79
+ *                KiB).  1 = 4-byte entries and the exit table in global memory;
+ *                2 forces global records; 3 = the exit table in global memory.
  *                Results are identical; this is a tuning/testing knob.
  * SSE_OPT_PERSISTENT (default 0): 1 = sse_run/sse_sweep issue one persistent,
  *                work-queue-driven launch per call (wave mode): each
- *                workgroup takes a walker from an atomic task counter and runs
- *                all of that walker's sweeps of the call (diagonal update,
- *                vertex list, worm update, measurement) before it takes the
- *                next; walkers never wait for each other.  Results are
- *                identical.
+ *                workgroup takes a task from an atomic counter and runs its
+ *                sweeps (diagonal update, vertex list, worm update,
+ *                measurement) before it takes the next; walkers never wait for
+ *                each other.  A task is a walker's whole call, or with more
+ *                walkers than resident workgroups one of up to 16 shares of it.
+ *                Results are identical.
  * SSE_OPT_STREAMS (default 0): wave mode splits the walkers into this many
  *                groups, each swept on its own HIP stream (forked from and
  *                joined into the batch stream), so the slow tail of one
@@ -379,7 +382,8 @@ int sse_pt_get_ladders(sse_batch *b, int32_t *slot_walkers, int64_t *accepted,
  *                groups at 2, 4, 8 (with more hardware queues than 8) and
  *                hardware-queue-count groups; the
  *                persistent work-queue launch with the worm-kernel LDS sized
- *                from the largest walker or capped at 32 KiB.  Each is
+ *                from the largest walker or for five walkers per compute unit (with
+ *                bonds of other than two sites also for eight).  Each is
  *                scored by vertex updates (the chains' own counters) per second; the
  *                fastest is kept.  sse_run_budgets tunes the same way over
  *                its first calls (work-queue forms only).  Setting

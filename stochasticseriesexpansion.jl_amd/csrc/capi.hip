@@ -1559,8 +1559,14 @@ static void tune_apply(sse_batch *b, const sse_batch::TuneCfg &c)
 // Candidates: the stream-group pipeline at 2, 4 and (queue count) groups
 // (not for budgeted calls, which always use the work-queue launch), and the
 // persistent work-queue launch with the worm-kernel LDS sized from the
-// largest walker or capped at 32 KiB (more workgroups per CU; larger walkers
-// then keep their records in global memory).
+// largest walker or for five walkers per CU (larger walkers then keep their
+// records in global memory).  Five is 32000 bytes: at 32768 only four run, and
+// 4096 rings of 256 three-site bonds (beta = 8) take 9.1 ms per sweep against
+// 7.6, dimer ladders of 128 rungs (beta = 16) 9.5 against 7.8.  Walkers of three-
+// and four-site bonds beyond that size step through global memory, whose latency
+// more of them per CU hide, so a batch that fills the chip also tries eight: 4096 rings of 256 four-site bonds (beta = 8) 17.0 ms per sweep, 21.0 with
+// five per CU, 26.4 sized from the largest (two per CU); on two-site bonds it was
+// never the fastest (24x24 at beta = 10: 14.9 against 13.2).
 static void tune_init(sse_batch *b, sse_batch::Tuner &t, bool budgets)
 {
     t.cands.clear();
@@ -1578,7 +1584,9 @@ static void tune_init(sse_batch *b, sse_batch::Tuner &t, bool budgets)
             t.cands.push_back({0, 1, 0});
     }
     t.cands.push_back({1, 0, 0});
-    t.cands.push_back({1, 0, 32768});
+    t.cands.push_back({1, 0, lds_for_walkers(5)});
+    if (b->wave.generic && n > 5 * b->n_cu)
+        t.cands.push_back({1, 0, lds_for_walkers(8)});
     t.rate.assign(t.cands.size(), 0.0);
     t.runs.assign(t.cands.size(), 0);
     t.best = -1;
@@ -2739,7 +2747,8 @@ int sse_lds_bytes(const sse_batch *b, int64_t *k1, int64_t *k2, int32_t *k2_per_
         int nb = 0;
         HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (const void *)wave_worm_kernel, 64,
                                                               b->wave.lds_k2));
-        *k2_per_cu = nb;
+        // (the query counts a fifth walker at 32768 bytes; four run)
+        *k2_per_cu = std::min(nb, (int)lds_walkers(b->wave.lds_k2));
     }
     return SSE_OK;
 }

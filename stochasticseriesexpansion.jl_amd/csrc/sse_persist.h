@@ -204,20 +204,10 @@ static inline size_t persist_lds_bytes(const WaveConfig &c)
     return std::max(c.generic ? c.lds_k1n : c.lds_k1, c.lds_k2);
 }
 
-// Workgroups the device holds at once at lds bytes per workgroup, from the
-// residency measured on MI355X (a workgroup takes round512(bytes + 256) of
-// about 162816 usable LDS bytes per CU; 64-lane workgroups, registers allow
-// at least 8 per CU)
+// Workgroups the device holds at once at lds bytes per workgroup
 static inline int persist_resident(size_t lds, int n_cu)
 {
-    const size_t per_cu_lds = 162816;
-    const size_t alloc = (lds + 256 + 511) & ~(size_t)511;
-    size_t k = per_cu_lds / alloc;
-    if (k < 1)
-        k = 1;
-    if (k > 8)
-        k = 8;
-    return (int)k * n_cu;
+    return (int)lds_walkers(lds) * n_cu;
 }
 
 // Segments of a launch: 1 where every walker has a workgroup of its own for the

@@ -1285,6 +1285,17 @@ static inline int wave_configure(WaveConfig &c, const std::vector<DevModel> &mod
 // its records in global memory instead of lowering every walker's residency
 constexpr size_t K2_LDS_CAP = 65536;
 
+// Residency measured on MI355X: a workgroup takes round512(bytes + 256) of the CU's
+// LDS and 162816 bytes are usable per CU (26880 B run 6 walkers per CU, 32000 B run 5,
+// 32256 B and up only 4, whatever the occupancy query says); registers allow 8.
+constexpr size_t kLdsPerCu = 162816;
+static inline size_t lds_walkers(size_t bytes)
+{
+    return std::min((size_t)8, std::max((size_t)1, kLdsPerCu / ((bytes + 256 + 511) & ~(size_t)511)));
+}
+// the largest size that k walkers per CU can have
+static inline size_t lds_for_walkers(size_t k) { return ((kLdsPerCu / k) & ~(size_t)511) - 256; }
+
 // Worm-kernel LDS per walker for the largest need (worm_lds_need) among the
 // last call's walkers, with a little headroom; walkers that do not fit keep
 // their records in global memory for that sweep.  The allocation is then
@@ -1300,19 +1311,9 @@ static inline size_t wave_k2_lds_for(const WaveConfig &c, unsigned long long max
     need = (need + 255) & ~(size_t)255;
     if (need > c.lds_limit)
         need = c.lds_limit;
-    // Residency measured on MI355X: a workgroup takes round512(bytes + 256) of
-    // the CU's LDS and about 162816 bytes are usable per CU (26880 B runs 6
-    // walkers per CU, 27136-30720 B run 5, 32256 B and up only 4, whatever the
-    // occupancy query says).
-    const size_t per_cu = std::min(c.lds_limit, (size_t)162816);
-    auto alloc = [](size_t b) { return (b + 256 + 511) & ~(size_t)511; };
     // walkers per CU: as many as fit, at most the 8 that the registers allow.  So
     // batches of small walkers keep one size, and a captured launch stays valid.
-    const size_t k = std::min((size_t)8, std::max((size_t)1, per_cu / alloc(need)));
-    size_t wide = ((per_cu / k) & ~(size_t)511) - 256;
-    if (wide < need)
-        wide = need;
-    return wide;
+    return std::max(need, std::min(c.lds_limit, lds_for_walkers(lds_walkers(need))));
 }
 
 static inline void wave_resize_lds(WaveConfig &c, unsigned long long max_need)

@@ -138,3 +138,31 @@ def test_generic_work_queue_hands_walkers_over(sse_pkg, oracle_mod):
         assert np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
     one.close()
     batch.close()
+
+
+@pytest.mark.parametrize("k2_lds,walkers", [(19712, 8), (26880, 6), (32000, 5), (32256, 4), (32768, 4), (40192, 4), (81152, 2)])
+def test_residency_report(sse_pkg, k2_lds, walkers):
+    """Walkers per CU as they run: a workgroup takes its LDS + 256 in steps of 512
+    bytes, out of 162816."""
+    flat = trimer_ring(sse_pkg, 6)[0]
+    batch = sse_pkg.Batch([flat], [sse_pkg.walker_desc(T=0.7, seed=1)], mode=0)
+    batch.set_option(sse_pkg.capi.SSE_OPT_K2_LDS, k2_lds)
+    assert batch.lds_bytes()[1:] == (k2_lds, walkers)
+    assert walkers == min(8, 162816 // (-(-(k2_lds + 256) // 512) * 512))
+    batch.close()
+
+
+def test_tuner_tries_more_walkers_per_cu(sse_pkg):
+    """A batch of other than two-site bonds that fills the chip has one candidate
+    more than a small one: eight walkers per CU."""
+    flat = trimer_ring(sse_pkg, 6)[0]
+    measured = []
+    for n in (200, 1400):
+        batch = sse_pkg.Batch([flat], [sse_pkg.walker_desc(T=0.7, seed=k, thermalization=2) for k in range(n)], mode=0)
+        batch.init()
+        for _ in range(20):
+            if batch.tuning(0) is None:
+                batch.run(8, measure=True)
+        measured.append(batch.tuning(0)["candidates_measured"])
+        batch.close()
+    assert measured[1] == measured[0] + 1
